@@ -170,13 +170,13 @@ class Pool {
 };
 
 // Device copy of the tables that depend only on the low-word size and the
-// bond topology (low-word ranks and states, class offsets, flip tables).
+// cross-bond topology (low-word ranks, states and page positions, class
+// offsets, flip tables).
 struct SharedTables {
   DevBuf buf;
   std::shared_ptr<const FlipTables> keep;  // keeps the key alive
-  const uint32_t *lo_rank = nullptr, *lo_state = nullptr, *lo_class_off = nullptr, *nbp_off = nullptr,
-                 *xn_off = nullptr;
-  const uint16_t *nbp16 = nullptr, *xn16 = nullptr;
+  const uint32_t *lo_rank = nullptr, *lo_state = nullptr, *lo_class_off = nullptr, *xn_off = nullptr;
+  const uint16_t *lo_page = nullptr, *lo_word = nullptr, *xn16 = nullptr;
 };
 
 enum State { kPending, kRunning, kRefining, kDone };
@@ -223,6 +223,8 @@ struct Problem {
   double t_submit = 0, t_admit = 0, t_done = 0;
   bool sized = false;  // layout built
   alps_ed_solve_result result{};
+  // Which of the H.v launches its items belong to (launch_batch_hv).
+  bool staged() const { return !trans && layout.stage; }
 };
 
 }  // namespace
@@ -290,11 +292,14 @@ size_t table_bytes(const SectorLayout& L) {
   add(L.proc_hi.size(), 4);
   add(L.diag_lo_cls.size(), 8);
   add(L.diag_hi.size(), 8);
-  add(L.ll_t.size(), 8);
+  add(L.ll_c.size(), sizeof(PageBond));
   add(L.hh_off.size(), 4);
   add(L.hh_ent.size(), sizeof(HHEntry));
   add(L.xb_c.size(), sizeof(XBondConst));
   add(L.xb_nb.size(), 4);
+  add(L.xb_p.size(), sizeof(PageBond));
+  add(L.xs.size(), sizeof(XStage));
+  add(L.xw.size(), 8);
   add(L.site_dn.size(), 8);
   add(L.site_up.size(), 8);
   add(L.bond_p1.size(), 4);
@@ -327,18 +332,16 @@ DevLayout place_tables(const SectorLayout& L, char* base, char* stage, const Sha
   d.D = (uint32_t)L.D;
   d.n_seg = (uint32_t)L.seg_hi.size();
   d.max_seg = L.max_seg;
-  d.n_ll_p = L.n_ll_p;
-  d.n_hh_p = L.n_hh_p;
-  d.n_xb_p = L.n_xb_p;
   d.n_ll = (int)L.ll.size();
-  d.n_hh = (int)L.hh.size();
   d.n_xb = (int)L.xb.size();
+  d.n_xb_p = L.n_xb_p;
+  d.n_xs = L.stage ? (int)L.xb_grp.size() : 0;
   d.n_bonds = (int)L.bond_p1.size();
   d.lo_rank = sh.lo_rank;
   d.lo_state = sh.lo_state;
   d.lo_class_off = sh.lo_class_off;
-  d.nbp16 = sh.nbp16;
-  d.nbp_off = sh.nbp_off;
+  d.lo_page = sh.lo_page;
+  d.lo_word = sh.lo_word;
   d.xn16 = sh.xn16;
   d.xn_off = sh.xn_off;
   size_t o = 0;
@@ -355,11 +358,14 @@ DevLayout place_tables(const SectorLayout& L, char* base, char* stage, const Sha
   d.proc_hi = put(L.proc_hi);
   d.diag_lo_cls = put(L.diag_lo_cls);
   d.diag_hi = put(L.diag_hi);
-  d.ll_t = put(L.ll_t);
+  d.ll_c = put(L.ll_c);
   d.hh_off = put(L.hh_off);
   d.hh_ent = put(L.hh_ent);
   d.xb_c = put(L.xb_c);
   d.xb_nb = put(L.xb_nb);
+  d.xb_p = put(L.xb_p);
+  d.xs = put(L.xs);
+  d.xw = put(L.xw);
   d.site_dn = put(L.site_dn);
   d.site_up = put(L.site_up);
   d.bond_p1 = put(L.bond_p1);
@@ -612,16 +618,17 @@ void ensure_stage(alps_ed_batch b, size_t bytes) {
 // Copies jobs, work items and the job list of a launch group to the device.
 struct Group {
   BatchJob* jobs = nullptr;
-  BatchItem* hv32 = nullptr;
-  BatchItem* hv64 = nullptr;
+  BatchItem* hv32[2] = {nullptr, nullptr};  // gathered, staged (Problem::staged)
+  BatchItem* hv64[2] = {nullptr, nullptr};
   BatchItem* up32 = nullptr;
   BatchItem* up64 = nullptr;
   BatchItem* st32 = nullptr;  // start-vector items of the problems new this round
   BatchItem* st64 = nullptr;
   uint32_t* list = nullptr;
   uint32_t* st_list = nullptr;
-  uint32_t n_hv32 = 0, n_hv64 = 0, n_up32 = 0, n_up64 = 0, n_list = 0, n_st32 = 0, n_st64 = 0, n_st_list = 0;
-  uint32_t seg32 = 0, seg64 = 0;
+  uint32_t n_hv32[2] = {0, 0}, n_hv64[2] = {0, 0};
+  uint32_t n_up32 = 0, n_up64 = 0, n_list = 0, n_st32 = 0, n_st64 = 0, n_st_list = 0;
+  uint32_t lds32 = kHvMinLds, lds64 = kHvMinLds;  // the largest LDS need of an H.v item
 };
 
 Group upload_group(alps_ed_batch b, const std::vector<Problem*>& run) {
@@ -632,21 +639,25 @@ Group upload_group(alps_ed_batch b, const std::vector<Problem*>& run) {
   // new this round, then the job list and the new jobs' list.
   Group g;
   const size_t nj = run.size();
-  size_t n_hv[2] = {0, 0}, n_up[2] = {0, 0}, n_st[2] = {0, 0}, n_new = 0;
+  size_t n_hv[2][2] = {{0, 0}, {0, 0}}, n_up[2] = {0, 0}, n_st[2] = {0, 0}, n_new = 0;
   for (const Problem* p : run) {
     const int f = p->fp32 ? 1 : 0;
-    n_hv[f] += p->n_hv;
+    n_hv[f][p->staged()] += p->n_hv;
     n_up[f] += p->n_chunks;
     if (p->j == 0) {
       n_st[f] += p->n_chunks;
       ++n_new;
     }
-    if (!p->trans) (p->fp32 ? g.seg32 : g.seg64) = std::max(p->fp32 ? g.seg32 : g.seg64, p->layout.max_seg);
+    if (!p->trans) {
+      uint32_t& lds = p->fp32 ? g.lds32 : g.lds64;
+      lds = std::max(lds, hv_lds_bytes(p->layout.B));
+    }
   }
   auto ib = [](size_t n) { return align_up((n + 1) * sizeof(BatchItem)); };
   const size_t bj = align_up(nj * sizeof(BatchJob));
   const size_t bl = align_up((nj + 1) * sizeof(uint32_t));
-  const size_t total = bj + ib(n_hv[1]) + ib(n_hv[0]) + ib(n_up[1]) + ib(n_up[0]) + ib(n_st[1]) + ib(n_st[0]) + 2 * bl;
+  const size_t total = bj + ib(n_hv[1][0]) + ib(n_hv[1][1]) + ib(n_hv[0][0]) + ib(n_hv[0][1]) + ib(n_up[1]) +
+                       ib(n_up[0]) + ib(n_st[1]) + ib(n_st[0]) + 2 * bl;
   ensure_buf(b->jobs_d, b->jobs_cap, total);
   ensure_stage(b, total);
   char* s = static_cast<char*>(b->stage);
@@ -661,8 +672,10 @@ Group upload_group(alps_ed_batch b, const std::vector<Problem*>& run) {
     o += ib(n);
     return h;
   };
-  BatchItem* hv32 = region(n_hv[1], g.hv32, g.n_hv32);
-  BatchItem* hv64 = region(n_hv[0], g.hv64, g.n_hv64);
+  BatchItem* hv32[2];
+  BatchItem* hv64[2];
+  for (int s = 0; s < 2; ++s) hv32[s] = region(n_hv[1][s], g.hv32[s], g.n_hv32[s]);
+  for (int s = 0; s < 2; ++s) hv64[s] = region(n_hv[0][s], g.hv64[s], g.n_hv64[s]);
   BatchItem* up32 = region(n_up[1], g.up32, g.n_up32);
   BatchItem* up64 = region(n_up[0], g.up64, g.n_up64);
   BatchItem* st32 = region(n_st[1], g.st32, g.n_st32);
@@ -677,7 +690,7 @@ Group upload_group(alps_ed_batch b, const std::vector<Problem*>& run) {
   uint32_t k_new = 0;
   for (uint32_t i = 0; i < nj; ++i) {
     const Problem& p = *run[i];
-    BatchItem*& hv = p.fp32 ? hv32 : hv64;
+    BatchItem*& hv = (p.fp32 ? hv32 : hv64)[p.staged()];
     BatchItem*& up = p.fp32 ? up32 : up64;
     for (uint32_t sg = 0; sg < p.n_hv; ++sg) *hv++ = {i, sg};
     for (uint32_t c = 0; c < p.n_chunks; ++c) *up++ = {i, c};
@@ -734,7 +747,7 @@ const SharedTables& shared_tables(alps_ed_batch b, const SectorLayout& L) {
   const LowTables& low = *L.low;
   const FlipTables& flip = *L.flip;
   const size_t o1 = sz(low.lo_rank.size(), 4), o2 = sz(low.lo_state.size(), 4), o3 = sz(low.lo_class_off.size(), 4),
-               o4 = sz(flip.nbp16.size(), 2), o5 = sz(flip.nbp_off.size(), 4), o6 = sz(flip.xn16.size(), 2),
+               o4 = sz(low.lo_page.size(), 2), o5 = sz(low.lo_word.size(), 2), o6 = sz(flip.xn16.size(), 2),
                o7 = sz(flip.xn_off.size(), 4);
   t.buf.alloc(total);
   char* d = t.buf.as<char>();
@@ -748,8 +761,8 @@ const SharedTables& shared_tables(alps_ed_batch b, const SectorLayout& L) {
   t.lo_rank = up(o1, low.lo_rank);
   t.lo_state = up(o2, low.lo_state);
   t.lo_class_off = up(o3, low.lo_class_off);
-  t.nbp16 = up(o4, flip.nbp16);
-  t.nbp_off = up(o5, flip.nbp_off);
+  t.lo_page = up(o4, low.lo_page);
+  t.lo_word = up(o5, low.lo_word);
   t.xn16 = up(o6, flip.xn16);
   t.xn_off = up(o7, flip.xn_off);
   return t;
@@ -891,7 +904,7 @@ void refine(alps_ed_batch b) {
   std::vector<std::vector<PlainHvJob>> hj(max_nv);
   std::vector<std::vector<BatchItem>> hi(max_nv);
   std::vector<std::vector<size_t>> who(max_nv);  // positions in work
-  std::vector<uint32_t> max_seg(max_nv, 0);
+  std::vector<uint32_t> lds(max_nv, kHvMinLds);
   for (size_t v = 0; v < max_nv; ++v)
     for (size_t wi = 0; wi < work.size(); ++wi) {
       Problem* p = work[wi];
@@ -906,7 +919,7 @@ void refine(alps_ed_batch b) {
       hj[v].push_back(j);
       who[v].push_back(wi);
       for (uint32_t sg = 0; sg < p->n_hv; ++sg) hi[v].push_back({ji, sg});
-      if (!p->trans) max_seg[v] = std::max(max_seg[v], p->layout.max_seg);
+      if (!p->trans) lds[v] = std::max(lds[v], hv_lds_bytes(p->layout.B));
     }
   // One pinned stage holds every upload of the pass: the Ritz coefficients
   // (scattered to each problem's coefficient buffer), the Ritz jobs and
@@ -962,7 +975,7 @@ void refine(alps_ed_batch b) {
   std::vector<std::vector<double>> yhy(work.size());
   for (size_t v = 0; v < max_nv; ++v) {
     hip_check(launch_batch_plain_hv(reinterpret_cast<PlainHvJob*>(dv + hj_at[v]), reinterpret_cast<BatchItem*>(dv + hi_at[v]),
-                                    (uint32_t)hi[v].size(), max_seg[v], b->stream),
+                                    (uint32_t)hi[v].size(), lds[v], b->stream),
               "plain hv");
     hip_check(hipStreamSynchronize(b->stream), "sync");
     for (size_t wi : who[v]) {
@@ -1049,8 +1062,11 @@ void round(alps_ed_batch b) {
     }
     auto steps = [&] {
       for (int t = 0; t < S; ++t) {
-        hip_check(launch_batch_hv<float>(g.jobs, g.hv32, g.n_hv32, t, g.seg32, b->stream), "batch hv");
-        hip_check(launch_batch_hv<double>(g.jobs, g.hv64, g.n_hv64, t, g.seg64, b->stream), "batch hv");
+        for (int s = 0; s < 2; ++s) {
+          hip_check(launch_batch_hv<float>(g.jobs, g.hv32[s], g.n_hv32[s], t, s == 1, g.lds32, b->stream), "batch hv");
+          hip_check(launch_batch_hv<double>(g.jobs, g.hv64[s], g.n_hv64[s], t, s == 1, g.lds64, b->stream),
+                    "batch hv");
+        }
         hip_check(launch_batch_finish(g.jobs, g.list, g.n_list, t, kBatchAlpha, b->stream), "batch finish");
         hip_check(launch_batch_update<float>(g.jobs, g.up32, g.n_up32, t, b->stream), "batch update");
         hip_check(launch_batch_update<double>(g.jobs, g.up64, g.n_up64, t, b->stream), "batch update");
@@ -1062,9 +1078,10 @@ void round(alps_ed_batch b) {
     // a round that repeats the previous one replays them from a graph.
     bool replayed = false;
     if (b->cfg.graphs && g.n_st_list == 0) {
-      const std::vector<uint64_t> key{(uint64_t)g.jobs, (uint64_t)g.hv32, (uint64_t)g.hv64, (uint64_t)g.up32,
-                                      (uint64_t)g.up64, (uint64_t)g.list, g.n_hv32, g.n_hv64, g.n_up32, g.n_up64,
-                                      g.n_list, g.seg32, g.seg64, (uint64_t)S};
+      const std::vector<uint64_t> key{(uint64_t)g.jobs, (uint64_t)g.hv32[0], (uint64_t)g.hv32[1], (uint64_t)g.hv64[0],
+                                      (uint64_t)g.hv64[1], (uint64_t)g.up32, (uint64_t)g.up64, (uint64_t)g.list,
+                                      g.n_hv32[0], g.n_hv32[1], g.n_hv64[0], g.n_hv64[1], g.n_up32, g.n_up64,
+                                      g.n_list, g.lds32, g.lds64, (uint64_t)S};
       if (key == b->last_key) {
         if (!b->graph_exec || key != b->graph_key) {
           if (b->graph_exec) hip_check(hipGraphExecDestroy(b->graph_exec), "graph destroy");

@@ -89,8 +89,8 @@ template <class V>
 hipError_t launch_batch_start(const BatchJob* jobs, const BatchItem* items, uint32_t n_items, hipStream_t st);
 // Step t of a launch group: w = H u_j into slot j+1, alpha partials.
 template <class V>
-hipError_t launch_batch_hv(const BatchJob* jobs, const BatchItem* items, uint32_t n_items, int t,
-                           uint32_t max_seg, hipStream_t st);
+hipError_t launch_batch_hv(const BatchJob* jobs, const BatchItem* items, uint32_t n_items, int t, bool stage,
+                           uint32_t lds, hipStream_t st);
 // r = s_j w - alpha_j s_j u_j - beta_{j-1} s_{j-1} u_{j-1} in place of w.
 template <class V>
 hipError_t launch_batch_update(const BatchJob* jobs, const BatchItem* items, uint32_t n_items, int t,
@@ -102,6 +102,6 @@ hipError_t launch_batch_finish(const BatchJob* jobs, const uint32_t* job_list, u
 template <class V>
 hipError_t launch_batch_ritz(const RitzJob* jobs, const BatchItem* items, uint32_t n_items, hipStream_t st);
 hipError_t launch_batch_plain_hv(const PlainHvJob* jobs, const BatchItem* items, uint32_t n_items,
-                                 uint32_t max_seg, hipStream_t st);
+                                 uint32_t lds, hipStream_t st);
 
 }  // namespace alps_ed

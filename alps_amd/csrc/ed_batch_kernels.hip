@@ -39,7 +39,10 @@ __global__ __launch_bounds__(kBlock) void batch_start_kernel(const BatchJob* __r
   if (threadIdx.x == 0) part[it.idx] = s;
 }
 
-template <class V>
+// STAGE: the items' problems stage their cross bonds (n_xs > 0); the others,
+// and momentum sectors, have a launch of their own, so that neither variant's
+// code costs the other registers.
+template <class V, bool STAGE>
 __global__ __launch_bounds__(kBlock, HvWaves<V>::value) void batch_hv_kernel(const BatchJob* __restrict__ jobs,
                                                           const BatchItem* __restrict__ items, int t) {
   const BatchItem it = ldc_struct(items + blockIdx.x);
@@ -53,15 +56,14 @@ __global__ __launch_bounds__(kBlock, HvWaves<V>::value) void batch_hv_kernel(con
   const V* x = slot_ptr<V>(vec, stride, cap, j);
   V* y = slot_ptr<V>(vec, stride, cap, j + 1);
   double* part = ldc(&J->part_hv);
-  if (ldc(&J->Bl.dk) != 0u) {  // momentum sector: uniform over the workgroup
+  if (!STAGE && ldc(&J->Bl.dk) != 0u) {  // momentum sector: uniform over the workgroup
     const DevBloch Bl = ldc_struct(&J->Bl);
     const double p = bloch_row<V, true>(L, Bl, x, y, it.idx * kBlock + threadIdx.x);
-    const double s = block_sum_all(p);
-    if (threadIdx.x == 0) part[it.idx] = s;
+    store_block_sum_lds<kBlock>(part + it.idx, p);
     return;
   }
   const uint32_t h = ldc(L.proc_hi + it.idx);
-  hv_segment<V, true>(L, h, x, y, part + it.idx);
+  hv_segment_at<V, true, STAGE>(L, seg_record(L, h), x, y, part + it.idx);
 }
 
 template <class V>
@@ -200,12 +202,14 @@ __global__ __launch_bounds__(kBlock) void batch_plain_hv_kernel(const PlainHvJob
   if (ldc(&J->Bl.dk) != 0u) {  // momentum sector: uniform over the workgroup
     const DevBloch Bl = ldc_struct(&J->Bl);
     const double p = bloch_row<double, true>(L, Bl, ldc(&J->x), ldc(&J->y), it.idx * kBlock + threadIdx.x);
-    const double s = block_sum_all(p);
-    if (threadIdx.x == 0) ldc(&J->part)[it.idx] = s;
+    store_block_sum_lds<kBlock>(ldc(&J->part) + it.idx, p);
     return;
   }
   const uint32_t h = ldc(L.proc_hi + it.idx);
-  hv_segment<double, true>(L, h, ldc(&J->x), ldc(&J->y), ldc(&J->part) + it.idx);
+  if (L.n_xs > 0)
+    hv_segment_at<double, true, true>(L, seg_record(L, h), ldc(&J->x), ldc(&J->y), ldc(&J->part) + it.idx);
+  else
+    hv_segment_at<double, true, false>(L, seg_record(L, h), ldc(&J->x), ldc(&J->y), ldc(&J->part) + it.idx);
 }
 
 }  // namespace
@@ -218,11 +222,13 @@ hipError_t launch_batch_start(const BatchJob* jobs, const BatchItem* items, uint
 }
 
 template <class V>
-hipError_t launch_batch_hv(const BatchJob* jobs, const BatchItem* items, uint32_t n_items, int t,
-                           uint32_t max_seg, hipStream_t st) {
+hipError_t launch_batch_hv(const BatchJob* jobs, const BatchItem* items, uint32_t n_items, int t, bool stage,
+                           uint32_t lds, hipStream_t st) {
   if (n_items == 0) return hipSuccess;
-  const size_t lds = (size_t)(max_seg + 1) * sizeof(double);  // the FP64 slice of hv_segment
-  hipLaunchKernelGGL((batch_hv_kernel<V>), dim3(n_items), dim3(kBlock), lds, st, jobs, items, t);
+  if (stage)
+    hipLaunchKernelGGL((batch_hv_kernel<V, true>), dim3(n_items), dim3(kBlock), lds, st, jobs, items, t);
+  else
+    hipLaunchKernelGGL((batch_hv_kernel<V, false>), dim3(n_items), dim3(kBlock), lds, st, jobs, items, t);
   return hipGetLastError();
 }
 
@@ -249,16 +255,15 @@ hipError_t launch_batch_ritz(const RitzJob* jobs, const BatchItem* items, uint32
 }
 
 hipError_t launch_batch_plain_hv(const PlainHvJob* jobs, const BatchItem* items, uint32_t n_items,
-                                 uint32_t max_seg, hipStream_t st) {
+                                 uint32_t lds, hipStream_t st) {
   if (n_items == 0) return hipSuccess;
-  const size_t lds = (size_t)(max_seg + 1) * sizeof(double);
   hipLaunchKernelGGL(batch_plain_hv_kernel, dim3(n_items), dim3(kBlock), lds, st, jobs, items);
   return hipGetLastError();
 }
 
 #define ALPS_ED_BATCH_INSTANTIATE(V)                                                                           \
   template hipError_t launch_batch_start<V>(const BatchJob*, const BatchItem*, uint32_t, hipStream_t);       \
-  template hipError_t launch_batch_hv<V>(const BatchJob*, const BatchItem*, uint32_t, int, uint32_t,         \
+  template hipError_t launch_batch_hv<V>(const BatchJob*, const BatchItem*, uint32_t, int, bool, uint32_t,   \
                                          hipStream_t);                                                       \
   template hipError_t launch_batch_update<V>(const BatchJob*, const BatchItem*, uint32_t, int, hipStream_t); \
   template hipError_t launch_batch_ritz<V>(const RitzJob*, const BatchItem*, uint32_t, hipStream_t);

@@ -76,7 +76,8 @@ struct alps_ed_operator_s {
   SectorLayout layout;
   DevLayout dev{};
   DevBuf tables;  // every layout table, packed (operator_upload)
-  DevBuf lists;   // per-high-word lists built on the device: hh_off and xb_nb,
+  DevBuf lists;   // per-high-word lists built on the device: hh_off, xb_nb or
+                  // xs and xw,
   DevBuf hh_ent;  // and the listed high-high flips
   DevBuf seg_rec; // per processing index: the segment's record (SegRec)
   uint64_t bytes = 0;
@@ -265,6 +266,10 @@ class PackedUpload {
   size_t off_ = 0;
 };
 
+// The layout of an operator (the shared low-word and flip tables are read
+// where they are, the per-high-word lists are built on the device).
+SectorLayout operator_layout(const alps_ed_model* model) { return build_layout(model_spec(model), -1, false); }
+
 void operator_upload(alps_ed_operator op) {
   SectorLayout& L = op->layout;
   DevLayout& d = op->dev;
@@ -276,17 +281,17 @@ void operator_upload(alps_ed_operator op) {
   d.D = (uint32_t)L.D;
   d.n_seg = (uint32_t)L.seg_hi.size();
   d.max_seg = L.max_seg;
-  d.n_ll_p = L.n_ll_p;
-  d.n_hh_p = L.n_hh_p;
-  d.n_xb_p = L.n_xb_p;
   d.n_ll = (int)L.ll.size();
-  d.n_hh = (int)L.hh.size();
   d.n_xb = (int)L.xb.size();
+  d.n_xb_p = L.n_xb_p;
+  d.n_xs = L.stage ? (int)L.xb_grp.size() : 0;
   d.n_bonds = (int)L.bond_p1.size();
   PackedUpload pk;
 #define ALPS_ED_UP(field) pk.add(L.field, &d.field);
-  ALPS_ED_UP(lo_rank)
-  ALPS_ED_UP(lo_state)
+  pk.add(L.low->lo_rank, &d.lo_rank);
+  pk.add(L.low->lo_state, &d.lo_state);
+  pk.add(L.low->lo_page, &d.lo_page);
+  pk.add(L.low->lo_word, &d.lo_word);
   ALPS_ED_UP(lo_class_off)
   ALPS_ED_UP(hi_base)
   ALPS_ED_UP(seg_hi)
@@ -294,23 +299,27 @@ void operator_upload(alps_ed_operator op) {
   ALPS_ED_UP(proc_hi)
   ALPS_ED_UP(diag_lo_cls)
   ALPS_ED_UP(diag_hi)
-  ALPS_ED_UP(nbp16)
-  ALPS_ED_UP(nbp_off)
-  ALPS_ED_UP(xn16)
+  ALPS_ED_UP(ll_c)
+  pk.add(L.flip->xn16, &d.xn16);
   ALPS_ED_UP(xn_off)
-  ALPS_ED_UP(ll_t)
   ALPS_ED_UP(xb_c)
+  ALPS_ED_UP(xb_p)
   const bool dev_lists = L.hh_off.empty();  // host_lists = false: built below
   const uint32_t *hh_mask = nullptr, *xb_hbit = nullptr;
   const double* hh_t = nullptr;
+  XSource X{nullptr, nullptr, d.n_xs, L.B};
   if (dev_lists) {
     pk.add(L.hh_mask, &hh_mask);
     pk.add(L.hh_t, &hh_t);
     pk.add(L.xb_hbit, &xb_hbit);
+    pk.add(L.xb_grp, &X.grp);
+    pk.add(L.xb_w, &X.w);
   } else {
     ALPS_ED_UP(hh_off)
     ALPS_ED_UP(hh_ent)
     ALPS_ED_UP(xb_nb)
+    ALPS_ED_UP(xs)
+    ALPS_ED_UP(xw)
   }
   ALPS_ED_UP(site_dn)
   ALPS_ED_UP(site_up)
@@ -324,15 +333,22 @@ void operator_upload(alps_ed_operator op) {
   op->bytes = pk.bytes();
   op->n = L.D;
   if (dev_lists && L.D > 0) {
-    // count, prefix sums and cross-bond neighbours, then (once the entry
-    // count is known) the entries; on the null stream, finished before return
+    // count, prefix sums and cross-bond neighbours or stages, then (once the
+    // entry count is known) the entries; on the null stream, finished before
+    // return
     const uint32_t nhi = 1u << L.NH;
-    const size_t off_bytes = ((size_t)(nhi + 1) * 4 + 255) & ~size_t(255);
-    const size_t xb_bytes = std::max<size_t>((size_t)nhi * L.n_xb_p * 4, 4);
-    op->lists.alloc(off_bytes + xb_bytes);
-    uint32_t* off = op->lists.as<uint32_t>();
-    uint32_t* xnb = reinterpret_cast<uint32_t*>(op->lists.as<char>() + off_bytes);
-    hip_check(launch_hh_count(nhi, d.hi_base, hh_mask, (int)L.hh_mask.size(), off, xb_hbit, L.n_xb_p, xnb, nullptr),
+    auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
+    const size_t nb_at = up((size_t)(nhi + 1) * 4), xs_at = nb_at + (L.stage ? 0 : up((size_t)nhi * L.n_xb_p * 4)),
+                 xw_at = xs_at + up((size_t)nhi * d.n_xs * sizeof(XStage)),
+                 end = xw_at + (L.stage ? (size_t)nhi * kXwStride * sizeof(double) : 0);
+    op->lists.alloc(end);
+    char* lists = op->lists.as<char>();
+    uint32_t* off = reinterpret_cast<uint32_t*>(lists);
+    uint32_t* xnb = reinterpret_cast<uint32_t*>(lists + nb_at);
+    XStage* xs = reinterpret_cast<XStage*>(lists + xs_at);
+    double* xw = reinterpret_cast<double*>(lists + xw_at);
+    hip_check(launch_hh_count(nhi, d.hi_base, hh_mask, (int)L.hh_mask.size(), off, xb_hbit, L.n_xb_p, xnb, X, xs, xw,
+                              nullptr),
               "high-high lists");
     uint32_t total = 0;
     hip_check(hipMemcpy(&total, off + nhi, sizeof(uint32_t), hipMemcpyDeviceToHost), "high-high lists");
@@ -345,6 +361,8 @@ void operator_upload(alps_ed_operator op) {
     d.hh_off = off;
     d.hh_ent = op->hh_ent.as<HHEntry>();
     d.xb_nb = xnb;
+    d.xs = xs;
+    d.xw = xw;
     op->bytes += op->lists.bytes + op->hh_ent.bytes;
   }
   if (d.n_seg > 0) {
@@ -488,9 +506,8 @@ int alps_ed_synchronize(void) {
 int alps_ed_operator_create(const alps_ed_model* model, alps_ed_operator* out) {
   return guarded([&] {
     require(out != nullptr, "output handle is null");
-    ModelSpec spec = model_spec(model);
     std::unique_ptr<alps_ed_operator_s> op(new alps_ed_operator_s);
-    op->layout = build_layout(spec);
+    op->layout = operator_layout(model);
     operator_upload(op.get());
     tune_schedule(op.get());
     *out = op.release();
@@ -504,7 +521,7 @@ int alps_ed_operator_create_momentum(const alps_ed_model* model, int n_translati
     require(out != nullptr && model != nullptr, "null argument");
     const Translations t = read_translations(model->n_sites, n_translations, perm, phase_re, phase_im);
     std::unique_ptr<alps_ed_operator_s> op(new alps_ed_operator_s);
-    op->layout = build_layout(model_spec(model));
+    op->layout = operator_layout(model);
     require(op->layout.D >= 1, "empty sector");
     operator_upload(op.get());
     bloch_upload(op.get(), bloch_sector(bloch_orbits(op->layout, t), t, op->layout.N));
@@ -1478,7 +1495,7 @@ SectorSolve solve_sector(const alps_ed_model* model, const alps_ed_solve_params*
   std::memset(result, 0, sizeof(*result));
   out.op.reset(new alps_ed_operator_s);
   alps_ed_operator_s* op = out.op.get();
-  op->layout = mom ? *mom->layout : build_layout(model_spec(model));
+  op->layout = mom ? *mom->layout : operator_layout(model);
   if (op->layout.D > 0) operator_upload(op);
   if (mom && op->layout.D > 0) bloch_upload(op, bloch_sector(*mom->orbits, *mom->trans, op->layout.N));
   const uint64_t D = mom ? op->n / 2 : op->layout.D;  // the sector's dimension
@@ -1700,7 +1717,7 @@ extern "C" int alps_ed_sparsediag_momentum(const alps_ed_model* model, int n_tra
   return guarded([&] {
     require(model && params && result, "null argument");
     const Translations t = read_translations(model->n_sites, n_translations, perm, phase_re, phase_im);
-    const SectorLayout L = build_layout(model_spec(model));
+    const SectorLayout L = operator_layout(model);
     const BlochOrbits o = bloch_orbits(L, t);
     const MomentumInput mi{&L, &o, &t};
     SectorSolve s = solve_sector(model, params, false, &mi);
@@ -1938,7 +1955,7 @@ extern "C" int alps_ed_run_parameter_file(const char* text, char* out, size_t ou
         for (const auto& k : ks) trans.push_back(lattice_translations(m.graph, k));
         const MeasurePlan plan = measure_plan(ms, m.graph);
         for (size_t i = 0; i < models.size(); ++i) {
-          const SectorLayout L = build_layout(model_spec(&models[i]));
+          const SectorLayout L = operator_layout(&models[i]);
           const BlochOrbits orb = bloch_orbits(L, trans[0]);
           std::unique_ptr<alps_ed_operator_s> plain;  // the fixed-Sz sector, for the spin sums
           for (size_t q = 0; q < nk; ++q) {
@@ -2037,7 +2054,7 @@ extern "C" int alps_ed_run_parameter_file(const char* text, char* out, size_t ou
           }
         } else {
           for (size_t i = 0; i < models.size(); ++i) {
-            const SectorLayout L = build_layout(model_spec(&models[i]));
+            const SectorLayout L = operator_layout(&models[i]);
             const BlochOrbits orb = bloch_orbits(L, trans[0]);
             for (size_t q = 0; q < nk; ++q) {
               const MomentumInput mi{&L, &orb, &trans[q]};

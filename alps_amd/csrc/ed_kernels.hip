@@ -5,13 +5,15 @@
 // src/ietl/interface/ublas.h:57-63).  The rows of one sector split into
 // segments that share the high word h of the state (see ed_layout.hpp); one
 // workgroup owns one segment:
-//   - the segment's slice of x is staged in LDS, so every low-low spin flip
-//     is an LDS gather; its target row comes from a per-class table read
-//     with coalesced 16-bit loads;
+//   - the segment's slice of x is staged in an LDS page indexed by the low
+//     word, so every low-low spin flip is an LDS read at the row's position
+//     xor a constant of the bond;
 //   - h is uniform, so the high-high flips are scalar decisions whose x
 //     reads are contiguous runs of a neighbouring segment (coalesced);
-//   - a cross flip (one bit in h, one in the low word) reads one element of
-//     a neighbouring segment, its rank coming from a per-class table;
+//   - for the cross flips (one bit in h, one in the low word) the segment
+//     across each high bit is staged in a second page where several bonds
+//     share it, else each flip reads one element of it, its rank coming from
+//     a per-class table;
 //   - the diagonal is two table values plus the cross bonds.
 // Every global load is a wave-uniform base plus a per-lane offset, so the
 // address costs no vector ALU work.  Bond lists are padded with null bonds to
@@ -33,11 +35,11 @@ using namespace dev;
 // ---------------------------------------------------------------------------
 // H.v: one workgroup per segment, longest segments first
 // ---------------------------------------------------------------------------
-template <class V, bool DOT, int W, int CLL, int CHH, int CX>
-__global__ __launch_bounds__(kBlock, W) void hv_kernel(DevLayout L, const V* __restrict__ x, V* __restrict__ y,
-                                                       double* __restrict__ dot_out) {
-  hv_segment_at<V, DOT, CLL, CHH, CX>(L, ldc_struct(L.seg_rec + blockIdx.x), x, y,
-                                      DOT ? dot_out + blockIdx.x : nullptr);
+template <class V, bool DOT, bool STAGE, int NT, int W, int CLL, int CHH>
+__global__ __launch_bounds__(NT, W) void hv_kernel(DevLayout L, const V* __restrict__ x, V* __restrict__ y,
+                                                   double* __restrict__ dot_out) {
+  hv_segment_at<V, DOT, STAGE, NT, CLL, CHH>(L, ldc_struct(L.seg_rec + blockIdx.x), x, y,
+                                             DOT ? dot_out + blockIdx.x : nullptr);
 }
 
 // seg_rec[i] for processing index i (the record hv_segment would look up).
@@ -47,29 +49,38 @@ __global__ __launch_bounds__(kBlock) void seg_rec_kernel(DevLayout L, SegRec* __
   out[i] = seg_record(L, L.proc_hi[i]);
 }
 
-template <class V, bool DOT, int W, int CLL, int CHH, int CX>
-void launch_hv_with(const DevLayout& L, const V* x, V* y, double* dot_out, hipStream_t st, size_t lds) {
-  hipLaunchKernelGGL((hv_kernel<V, DOT, W, CLL, CHH, CX>), dim3(hv_blocks(L)), dim3(kBlock), lds, st, L, x, y,
-                     dot_out);
+template <class V, bool DOT, bool STAGE, int NT, int W, int CLL, int CHH>
+void launch_hv_with(const DevLayout& L, const V* x, V* y, double* dot_out, hipStream_t st) {
+  hipLaunchKernelGGL((hv_kernel<V, DOT, STAGE, NT, W, CLL, CHH>), dim3(hv_blocks(L)), dim3(NT), hv_lds_bytes(L.B), st, L,
+                     x, y, dot_out);
 }
 
 // The schedule table of ed_kernels.hpp as template arguments.
-template <class V, bool DOT>
-void launch_hv_schedule(const DevLayout& L, const V* x, V* y, double* dot_out, hipStream_t st, size_t lds,
-                        int schedule) {
-  constexpr int W = HvWaves<V>::value;
+template <class V, bool DOT, bool STAGE>
+void launch_hv_schedule(const DevLayout& L, const V* x, V* y, double* dot_out, hipStream_t st, int schedule) {
+  if (L.n_seg <= kFewSegments) {
+    launch_hv_with<V, DOT, STAGE, 512, sizeof(V) == 4 ? 8 : 6, 4, 4>(L, x, y, dot_out, st);
+    return;
+  }
   if constexpr (sizeof(V) == 4) {
     static_assert(kHvSchedules == 6, "one case per schedule");
     switch (schedule) {
-      case 1: launch_hv_with<V, DOT, 8, 4, 8, 2>(L, x, y, dot_out, st, lds); return;
-      case 2: launch_hv_with<V, DOT, 6, 4, 8, 2>(L, x, y, dot_out, st, lds); return;
-      case 3: launch_hv_with<V, DOT, 6, 4, 4, 2>(L, x, y, dot_out, st, lds); return;
-      case 4: launch_hv_with<V, DOT, 8, 8, 4, 2>(L, x, y, dot_out, st, lds); return;
-      case 5: launch_hv_with<V, DOT, 6, 8, 8, 4>(L, x, y, dot_out, st, lds); return;
-      default: break;
+      case 1: launch_hv_with<V, DOT, STAGE, kBlock, 8, 1, 4>(L, x, y, dot_out, st); return;
+      case 2: launch_hv_with<V, DOT, STAGE, kBlock, 8, 4, 4>(L, x, y, dot_out, st); return;
+      case 3: launch_hv_with<V, DOT, STAGE, kBlock, 7, 2, 4>(L, x, y, dot_out, st); return;
+      case 4: launch_hv_with<V, DOT, STAGE, kBlock, 6, 2, 4>(L, x, y, dot_out, st); return;
+      case 5: launch_hv_with<V, DOT, STAGE, kBlock, 6, 4, 4>(L, x, y, dot_out, st); return;
+      default: launch_hv_with<V, DOT, STAGE, kBlock, 8, 2, 4>(L, x, y, dot_out, st); return;
     }
+  } else {
+    launch_hv_with<V, DOT, STAGE, kBlock, 6, 2, 2>(L, x, y, dot_out, st);
   }
-  launch_hv_with<V, DOT, W, 4, 4, 2>(L, x, y, dot_out, st, lds);
+}
+
+template <class V, bool DOT>
+void launch_hv_stage(const DevLayout& L, const V* x, V* y, double* dot_out, hipStream_t st, int schedule) {
+  if (L.n_xs > 0) launch_hv_schedule<V, DOT, true>(L, x, y, dot_out, st, schedule);
+  else launch_hv_schedule<V, DOT, false>(L, x, y, dot_out, st, schedule);
 }
 
 // ---------------------------------------------------------------------------
@@ -152,6 +163,16 @@ __global__ __launch_bounds__(kBlock) void xb_nb_kernel(uint32_t nhi, int n_xb_p,
     v = nb == 0xffffffffu ? own : nb;
   }
   out[i] = v;
+}
+
+// kXwStride threads per high word: its entries of xw, the last one its stages.
+__global__ __launch_bounds__(kBlock) void cross_stages_kernel(uint32_t nhi, const uint32_t* __restrict__ hi_base,
+                                                              XSource X, XStage* __restrict__ xs,
+                                                              double* __restrict__ xw) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x, h = i / kXwStride, p = i % kXwStride;
+  if (h >= nhi || hi_base[h] == 0xffffffffu) return;
+  if (p <= (uint32_t)X.B) xw[i] = cross_weight(h, (int)p, X);
+  if (p == kXwStride - 1) cross_stages(h, hi_base, X, xs + (size_t)h * X.ng);
 }
 
 // One workgroup per item; 16-byte moves where source and destination allow.
@@ -672,11 +693,8 @@ template <class V>
 hipError_t launch_hv(const DevLayout& L, const V* x, V* y, double* dot_out, hipStream_t st, int schedule) {
   if (L.n_seg == 0) return hipSuccess;
   if (schedule < 0 || schedule >= kHvSchedules || L.seg_rec == nullptr) return hipErrorInvalidValue;
-  const size_t lds = (size_t)(L.max_seg + 1) * sizeof(double);  // the FP64 slice of hv_segment
-  if (dot_out)
-    launch_hv_schedule<V, true>(L, x, y, dot_out, st, lds, schedule);
-  else
-    launch_hv_schedule<V, false>(L, x, y, dot_out, st, lds, schedule);
+  if (dot_out) launch_hv_stage<V, true>(L, x, y, dot_out, st, schedule);
+  else launch_hv_stage<V, false>(L, x, y, dot_out, st, schedule);
   return hipGetLastError();
 }
 
@@ -732,12 +750,16 @@ hipError_t launch_normalize(uint64_t n, V* v, Partials norm_in, double* b_out, h
 }
 
 hipError_t launch_hh_count(uint32_t nhi, const uint32_t* hi_base, const uint32_t* mask, int nb, uint32_t* off,
-                           const uint32_t* hbit, int n_xb_p, uint32_t* xb_nb, hipStream_t st) {
+                           const uint32_t* hbit, int n_xb_p, uint32_t* xb_nb, const XSource& X, XStage* xs,
+                           double* xw, hipStream_t st) {
   const unsigned g = (unsigned)((nhi + kBlock - 1) / kBlock);
   hipLaunchKernelGGL(hh_count_kernel, dim3(g), dim3(kBlock), 0, st, nhi, hi_base, mask, nb, off);
   hipLaunchKernelGGL(scan_inclusive_kernel, dim3(1), dim3(kScanBlock), 0, st, off + 1, nhi);
   const uint64_t nx = (uint64_t)nhi * n_xb_p;
-  if (nx > 0)
+  if (X.ng > 0)
+    hipLaunchKernelGGL(cross_stages_kernel, dim3((nhi * kXwStride + kBlock - 1) / kBlock), dim3(kBlock), 0, st, nhi,
+                       hi_base, X, xs, xw);
+  else if (nx > 0)
     hipLaunchKernelGGL(xb_nb_kernel, dim3((unsigned)((nx + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, nhi, n_xb_p,
                        hi_base, hbit, xb_nb);
   return hipGetLastError();

@@ -14,8 +14,9 @@ struct DevLayout {
   int N, k, B, NH;
   uint32_t D;
   uint32_t n_seg, max_seg;
-  int n_ll_p, n_hh_p, n_xb_p, n_bonds;  // padded flip-bond counts (table strides)
-  int n_ll, n_hh, n_xb;                 // flip bonds per class
+  int n_bonds;
+  int n_ll, n_xb, n_xb_p;     // low-low and cross flip bonds; the cross tables' stride
+  int n_xs;                   // high bits with staged cross bonds; 0: gathered
   const uint32_t* lo_rank;
   const uint32_t* lo_state;
   const uint32_t* lo_class_off;
@@ -25,15 +26,20 @@ struct DevLayout {
   const uint32_t* proc_hi;    // H.v processing order
   const double* diag_lo_cls;  // low-word diagonal in lo_state order
   const double* diag_hi;
-  const uint16_t* nbp16;
-  const uint32_t* nbp_off;
-  const uint16_t* xn16;
-  const uint32_t* xn_off;
-  const double* ll_t;
+  const uint16_t* lo_page;    // 8 * each low word's page position, in lo_state order
+  const uint16_t* lo_word;    // and the words
+  const PageBond* ll_c;       // [n_ll] low-low bonds
   const uint32_t* hh_off;     // [2^NH + 1] per high word: its flipping high-high bonds
   const HHEntry* hh_ent;      //   (neighbour segment, coefficient), padded with 0-coefficient entries
-  const XBondConst* xb_c;     // [n_xb_p] cross-bond constants
-  const uint32_t* xb_nb;      // [2^NH * n_xb_p] first row of the cross-bond neighbour segment
+  // gathered cross bonds
+  const uint16_t* xn16;
+  const uint32_t* xn_off;
+  const XBondConst* xb_c;     // [n_xb_p] constants
+  const uint32_t* xb_nb;      // [2^NH * n_xb_p] first row of the neighbour segment
+  // staged cross bonds
+  const PageBond* xb_p;
+  const XStage* xs;           // [2^NH * n_xs] per high word: the segments staged for them
+  const double* xw;           // [2^NH * kXwStride] and their share of the diagonal
   const SegRec* seg_rec;      // [n_seg] per processing index (single operators; the batch looks them up)
   // reference-order description for the element enumeration
   const double* site_dn;
@@ -88,6 +94,12 @@ template <class V>
 struct HvWaves {
   static constexpr int value = sizeof(V) == 4 ? 8 : 1;
 };
+// Bytes of an LDS page: FP64 elements (converted once per row, not once per
+// flip that reads it) for the words of one parity; and the LDS of an H.v
+// workgroup, which also holds its reduction.
+inline __host__ __device__ uint32_t page_bytes(int low_bits) { return low_bits < 2 ? 16u : 4u << low_bits; }
+constexpr uint32_t kHvMinLds = 256;
+inline uint32_t hv_lds_bytes(int low_bits) { return page_bytes(low_bits) < kHvMinLds ? kHvMinLds : page_bytes(low_bits); }
 // FP32 storage of the Lanczos vectors is used, when asked for, only where it
 // pays: sectors of at least kFp32MinDim states (in small sectors the Krylov
 // space is a large part of the sector).  Without reorthogonalization (the
@@ -104,8 +116,7 @@ constexpr int kFp32MaxNev = 2;
 inline bool use_fp32(bool asked, uint64_t dim, int nev) { return asked && dim >= kFp32MinDim && nev <= kFp32MaxNev; }
 inline bool use_fp32_reorth(bool asked, uint64_t dim) { return asked && dim >= kFp32MinDim; }
 constexpr int kMaxRitz = 8;     // Ritz vectors per pass of launch_ritz
-// H.v rows per thread: a segment of up to kRows*kBlock rows is one workgroup
-constexpr int kRows = 4;
+constexpr int kMaxSegRows = 1024;  // a segment (of at most 924 rows) is one H.v workgroup
 
 // Number of blocks of the streaming kernels for a vector of length n.
 inline unsigned stream_blocks(uint64_t n) {
@@ -125,17 +136,18 @@ inline unsigned fused_blocks(uint64_t n) { return stream_blocks(n); }
 inline unsigned hv_blocks(const DevLayout& L) { return L.n_seg ? L.n_seg : 1; }
 
 // H.v schedules for FP32 vectors: the waves per SIMD the kernel is compiled
-// for and the chunk sizes of its low-low, high-high and cross flip loops.
-// Schedule 0 is the default (FP64 vectors always use it); an operator of a
-// large FP32 sector picks its schedule by timing them all (the autotuner in
-// ed_capi.hip).  Every schedule adds the bonds in the same order and forms
-// the dot partials the same way, so all give identical results.
+// for and the chunk sizes of its low-low and high-high flip loops.  Schedule
+// 0 is the default; an operator of a large FP32 sector picks its schedule by
+// timing them all (the autotuner in ed_capi.hip).  Every schedule adds the
+// bonds in the same order and forms the dot partials the same way, so all
+// give identical results.
 struct HvSchedule {
-  int waves, cll, chh, cx;
+  int waves, cll, chh;
 };
 constexpr int kHvSchedules = 6;
-constexpr HvSchedule kHvSchedule[kHvSchedules] = {{8, 4, 4, 2}, {8, 4, 8, 2}, {6, 4, 8, 2},
-                                                  {6, 4, 4, 2}, {8, 8, 4, 2}, {6, 8, 8, 4}};
+constexpr HvSchedule kHvSchedule[kHvSchedules] = {{8, 2, 4}, {8, 1, 4}, {8, 4, 4}, {7, 2, 4}, {6, 2, 4}, {6, 4, 4}};
+// Layouts of at most kFewSegments segments take 512 threads a workgroup
+// instead of kBlock, whatever the schedule.
 
 // y = H x; with dot_out set, per-block partials of sum_i x_i (H x)_i (FP64,
 // before y is rounded to the storage type).
@@ -194,11 +206,13 @@ hipError_t launch_reorth(uint64_t n, int j, V* r, const double* scale, const Reo
 
 // The per-high-word lists of a layout on the device: launch_hh_count writes
 // off[0..nhi] (the prefix sums of each high word's flipping high-high bond
-// count, rounded up to kHHList; 0xffffffff once they reach 2^32 - 1) and
-// xb_nb[nhi * n_xb_p]; launch_hh_fill then writes the off[nhi] entries.  The
+// count, rounded up to kHHList; 0xffffffff once they reach 2^32 - 1) and, for
+// gathered cross bonds, xb_nb[nhi * n_xb_p], for staged ones (X.ng > 0)
+// xs[nhi * ng] and xw; launch_hh_fill then writes the off[nhi] entries.  The
 // same lists build_layout makes on the host with host_lists.
 hipError_t launch_hh_count(uint32_t nhi, const uint32_t* hi_base, const uint32_t* mask, int nb, uint32_t* off,
-                           const uint32_t* hbit, int n_xb_p, uint32_t* xb_nb, hipStream_t st);
+                           const uint32_t* hbit, int n_xb_p, uint32_t* xb_nb, const XSource& X, XStage* xs,
+                           double* xw, hipStream_t st);
 hipError_t launch_hh_fill(uint32_t nhi, const uint32_t* hi_base, const uint32_t* mask, const double* t, int nb,
                           const uint32_t* off, HHEntry* ent, hipStream_t st);
 

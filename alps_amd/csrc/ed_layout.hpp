@@ -120,7 +120,7 @@ struct HHEntry {
   double t;      // coefficient
 };
 
-// The per-bond constants of a cross bond as the H.v kernel reads them.
+// The per-bond constants of a gathered cross bond as the H.v kernel reads them.
 struct XBondConst {
   double de;      // e_anti - e_par
   double t;       // flip coefficient
@@ -128,22 +128,48 @@ struct XBondConst {
   uint32_t pad;
 };
 
+// The cross bonds of one high bit: xb_p[info & 0xffff, + info >> 16).
+struct XGroup {
+  uint32_t hbit, info;
+};
+
+// A segment staged for the cross bonds of one high bit: its first row, and
+// the bonds xb_p[first, first + n).
+struct XStage {
+  uint32_t nb;
+  uint32_t info;  // first | n << 16 | (the bit is set in h) << 31; 0: none
+};
+
+// A flip bond as the H.v kernel reads it from an LDS page: the coefficient
+// and 8 * the page position of its low bits (page_pos), the distance (by xor)
+// from a row's element to the flipped row's.
+struct PageBond {
+  double t;
+  uint32_t m;
+  uint32_t pad;
+};
+
 // What the H.v kernel needs of the segment it processes, one record per
 // processing index (built on the device for a single operator): its high
-// word, first row, class offset and length, flip-table offsets, the range
-// of its listed high-high flips and the high word's diagonal.  Read with
-// one pair of scalar loads instead of two dependent rounds of table reads.
+// word, first row, class offset and length, the flip-table offset, those of the
+// classes with one low bit more and one fewer (the segments across a cross
+// bond), the range of its listed high-high flips and the high word's
+// diagonal.  Read with one scalar load instead of two dependent rounds of
+// table reads.
 struct SegRec {
-  uint32_t h, base, cls0, len, nbp, xnp, e0, e1;
-  double dh, pad;
+  uint32_t h, base, cls0, len;
+  uint32_t e0, e1, xnp, pad;
+  uint32_t cls_up, len_up, cls_dn, len_dn;
+  double dh, pad2;
 };
+static_assert(sizeof(SegRec) == 64, "one 64-byte scalar load");
 
 struct SectorLayout {
   int N = 0, k = 0, B = 0, NH = 0;
   uint64_t D = 0;
   // the shared tables the low-word and flip-table vectors below copy: the
-  // same objects for every sector with the same low-word size and low-low /
-  // cross-bond topology (lets a batch upload them once)
+  // same objects for every sector with the same low-word size and cross-bond
+  // topology (lets a batch upload them once)
   const LowTables* low = nullptr;
   std::shared_ptr<const FlipTables> flip;
   std::vector<uint32_t> lo_rank;       // [2^B]
@@ -155,21 +181,32 @@ struct SectorLayout {
   std::vector<double> diag_lo_cls;     // diag_lo in lo_state order (coalesced)
   std::vector<uint32_t> proc_hi;       // hi words in H.v processing order (by class)
   uint32_t max_seg = 0;                // longest segment
-  // H.v tables.  Bond lists are padded with null bonds (coefficient 0,
-  // never active) to multiples of the kernel's chunk sizes.
-  //   nbp16[nbp_off[c] + flip_index(r, b, n_ll_p, kLLChunk)]: 8 * the row
-  //     reached from row r of a class-c segment by low-low bond b, or
-  //     8 * C(B,c) (the zero slot) if not allowed: the byte offset of the
-  //     row's FP64 element in the segment's LDS slice;
+  // H.v tables.
+  //   ll_c[ll.size()]: the low-low bonds as the kernel reads them.
+  // Cross bonds, where few share a high bit (stage false): gathered,
+  //   xb_c[n_xb_p]: their constants, padded with null bonds;
   //   xn16[xn_off[c] + flip_index(r, b, n_xb_p, kXChunk)]: 4 * the rank of
   //     lo ^ lbit_b in its class, with bit 15 = the low bit of cross bond b
-  //     in row r: the byte offset of an FP32 element of x (twice it for FP64).
-  // Both are used as byte offsets without a shift (C(12,6) * 8 < 2^16,
-  // C(12,6) * 4 < 2^15).
+  //     in row r: the byte offset of an FP32 element of x (twice it for FP64),
+  //     used without a shift (C(12,6) * 4 < 2^15);
+  //   xb_nb[h * n_xb_p + b]: the first row of the neighbour segment.
+  // Where several share one (stage true): staged in an LDS page,
+  //   xb_p[xb.size()]: the bonds, those of one high bit adjacent;
+  //   xb_grp[n_xs]: per high bit that has any, its bit and their range;
+  //   xs[h * n_xs + i]: the segments that high word h stages for them, the
+  //     bits set in h first (their segments' words have one low bit more);
+  //     bits across which there is no segment have none (info 0, at the end);
+  //   xw[h * kXwStride + p]: what low bit p set adds to the diagonal of the
+  //     rows of h through the cross bonds, and [B]: what every row gets.
+  // A host-side description of the low-low flips (only with copy_shared):
+  //   nbp16[nbp_off[c] + flip_index(r, b, n_ll_p, kLLChunk)]: 8 * the row
+  //     reached from row r of a class-c segment by low-low bond b, or
+  //     8 * C(B,c) if the bond does not flip it.
   int n_ll_p = 0, n_hh_p = 0, n_xb_p = 0;
   std::vector<uint16_t> nbp16, xn16;
   std::vector<uint32_t> nbp_off, xn_off;  // [B+2]
-  std::vector<double> ll_t;               // [n_ll_p]
+  std::vector<PageBond> ll_c;
+  bool stage = false;                     // cross bonds staged, not gathered
   // The high-high bonds that flip the rows of high word h (the two bits of
   // h & mask differ), in bond order: entries [hh_off[h], hh_off[h+1]) of
   // hh_ent, each the first row of the segment of h ^ mask and the bond's
@@ -184,10 +221,15 @@ struct SectorLayout {
   // xb_nb[h * n_xb_p + c]: the first row of the segment of h ^ hbit_c, or of
   // h's own segment when that high word has none (no row of h flips then)
   std::vector<uint32_t> xb_nb;
+  std::vector<PageBond> xb_p;
+  std::vector<XGroup> xb_grp;
+  std::vector<double> xb_w;               // XSource::w
+  std::vector<XStage> xs;                 // [2^NH * n_xs] (empty when built on the device)
+  std::vector<double> xw;                 // [2^NH * kXwStride] (empty when built on the device)
   std::vector<double> diag_lo;         // [2^B] site + low-low bond diagonal
   std::vector<double> diag_hi;         // [2^NH] site + high-high bond diagonal + every cross bond's par value
   std::vector<FlipBond> ll, hh;        // low-low and high-high flip bonds
-  std::vector<CrossBond> xb;           // cross bonds (all, for the diagonal)
+  std::vector<CrossBond> xb;           // cross bonds (all, for the diagonal), by high bit
   // reference-order description for the element enumeration
   std::vector<double> site_dn, site_up;          // per site
   std::vector<uint32_t> bond_p1, bond_p2;        // bit positions per bond
@@ -208,7 +250,7 @@ inline int round_up(int n, int m) { return (n + m - 1) / m * m; }
 // contiguous, row after row: one load brings a row's ch entries, and the
 // loads of a wave's 64 consecutive rows cover one contiguous run.  A class
 // of len rows takes round_up(len, 64) * n_pad entries.
-constexpr int kLLChunk = 4, kXChunk = 2;  // u16 entries per load (8 and 4 bytes)
+constexpr int kLLChunk = 4, kXChunk = 2;  // u16 entries per record
 static_assert(kPadLL % kLLChunk == 0 && kPadX % kXChunk == 0, "chunks divide the padding");
 
 inline size_t flip_index(uint32_t r, int b, int n_pad, int ch) {
@@ -222,11 +264,25 @@ inline int choose_low_bits(int N) {
   return N < 12 ? N : 12;
 }
 
+// Position of low word lo in an LDS page of 2^(B-1) elements (page_entries):
+// its Gray code without the lowest bit.  The map is linear over xor, so the
+// flip of the bits m moves every row by the same xor, page_pos(lo ^ m) =
+// page_pos(lo) ^ page_pos(m), and needs no table.  Two words share a position
+// only if they differ in bit 0 alone, so words of one parity (a class and
+// those two bits away, or the two classes one bit away) do not.  The Gray
+// code spreads a wave's rows over the LDS: 2.2 of 32 consecutive rows share
+// the busiest of 32 places on average over the classes of 12 bits, against
+// 2.7 with the word itself; the best linear map that a random search found
+// gives 2.0.
+inline uint32_t page_pos(uint32_t lo) { return (lo ^ (lo >> 1)) >> 1; }
+
 // Tables of the B-bit low word, the same for every sector with that B:
 // colex rank of each word within its popcount class, the words of each class
-// in ascending order, and the class offsets.  Built once per B.
+// in ascending order (as 16 bits too, with 8 * their page positions), and
+// the class offsets.  Built once per B.
 struct LowTables {
   std::vector<uint32_t> lo_rank, lo_state, lo_class_off;
+  std::vector<uint16_t> lo_word, lo_page;
 };
 
 inline const LowTables& low_tables(int B) {
@@ -251,22 +307,31 @@ inline const LowTables& low_tables(int B) {
     for (int c = 0; c <= B; ++c) T.lo_class_off[c + 1] += T.lo_class_off[c];
     T.lo_state.assign(nlo, 0);
     for (uint32_t v = 0; v < nlo; ++v) T.lo_state[T.lo_class_off[__builtin_popcount(v)] + T.lo_rank[v]] = v;
+    for (uint32_t v : T.lo_state) {
+      T.lo_word.push_back((uint16_t)v);
+      T.lo_page.push_back((uint16_t)(8u * page_pos(v)));
+    }
   }
   return *slot;
 }
 
-// Per-class flip tables of a set of low-word masks (low-low bonds, padded
-// to n_pad with null bonds) and of cross-bond low bits, cached by their key:
-// many sectors of one batch share the lattice and so these tables.
+// Offsets of the classes' tables of n_pad entries a row (flip_index), [B+2].
+inline std::vector<uint32_t> flip_offsets(int B, int n_pad) {
+  std::vector<uint32_t> off(B + 2, 0);
+  for (int c = 0; c <= B; ++c) off[c + 1] = off[c] + (uint32_t)(round_up((int)binom(B, c), 64) * n_pad);
+  return off;
+}
+
+// Per-class flip table of a set of cross-bond low bits (padded to n_pad with
+// null bonds), cached by its key: many sectors of one batch share the lattice
+// and so the table.
 struct FlipTables {
-  std::vector<uint32_t> nbp_off, xn_off;
-  std::vector<uint16_t> nbp16, xn16;
+  std::vector<uint32_t> xn_off;
+  std::vector<uint16_t> xn16;
 };
 
-inline std::shared_ptr<const FlipTables> flip_tables(int B, const std::vector<uint32_t>& ll_masks, int n_ll_p,
-                                                     const std::vector<uint32_t>& x_lbits, int n_xb_p) {
-  std::vector<uint32_t> key{(uint32_t)B, (uint32_t)n_ll_p, (uint32_t)n_xb_p, (uint32_t)ll_masks.size()};
-  key.insert(key.end(), ll_masks.begin(), ll_masks.end());
+inline std::shared_ptr<const FlipTables> flip_tables(int B, const std::vector<uint32_t>& x_lbits, int n_xb_p) {
+  std::vector<uint32_t> key{(uint32_t)B, (uint32_t)n_xb_p};
   key.insert(key.end(), x_lbits.begin(), x_lbits.end());
   static std::mutex mu;
   static std::map<std::vector<uint32_t>, std::shared_ptr<const FlipTables>> cache;
@@ -278,26 +343,11 @@ inline std::shared_ptr<const FlipTables> flip_tables(int B, const std::vector<ui
   if (4 * binom(B, B / 2) >= 32768) throw std::invalid_argument("low word too wide for the flip tables");
   const LowTables& T = low_tables(B);
   std::shared_ptr<FlipTables> F(new FlipTables);
-  F->nbp_off.assign(B + 2, 0);
-  F->xn_off.assign(B + 2, 0);
-  for (int c = 0; c <= B; ++c) {
-    const uint64_t len64 = (uint64_t)round_up((int)binom(B, c), 64);
-    F->nbp_off[c + 1] = F->nbp_off[c] + (uint32_t)(len64 * n_ll_p);
-    F->xn_off[c + 1] = F->xn_off[c] + (uint32_t)(len64 * n_xb_p);
-  }
-  F->nbp16.assign(F->nbp_off[B + 1], 0);
+  F->xn_off = flip_offsets(B, n_xb_p);
   F->xn16.assign(F->xn_off[B + 1], 0);
   for (int c = 0; c <= B; ++c) {
     const uint32_t len = (uint32_t)binom(B, c);
     const uint32_t* ls = T.lo_state.data() + T.lo_class_off[c];
-    uint16_t* nb = F->nbp16.data() + F->nbp_off[c];
-    for (int b = 0; b < n_ll_p; ++b) {
-      const uint32_t m = b < (int)ll_masks.size() ? ll_masks[b] : 0u;
-      for (uint32_t r = 0; r < len; ++r) {
-        const uint32_t lo = ls[r], bits = lo & m;
-        nb[flip_index(r, b, n_ll_p, kLLChunk)] = (uint16_t)(8u * ((bits != 0u && bits != m) ? T.lo_rank[lo ^ m] : len));
-      }
-    }
     uint16_t* xn = F->xn16.data() + F->xn_off[c];
     for (int b = 0; b < (int)x_lbits.size(); ++b) {
       const uint32_t lb = x_lbits[b];
@@ -314,10 +364,71 @@ inline std::shared_ptr<const FlipTables> flip_tables(int B, const std::vector<ui
   return F;
 }
 
+// Layouts of at most this many segments are launched with a workgroup of 512
+// threads per segment instead of 256: with two segments or fewer per compute
+// unit the launch lasts as long as one segment's chain of memory rounds, and
+// fewer rows per thread shorten it (FP64, 256 and 512 threads: 20 sites 4.67
+// and 4.38 us, 21 sites 5.82 and 5.36, 20-site J1-J2 13.4 and 10.4; above the
+// line 22 sites 8.23 and 8.28, 23 sites 13.4 and 15.3).
+constexpr size_t kFewSegments = 512;
+
+// Whether the cross bonds are staged in LDS (hv_rows, ed_device.hpp): where a
+// high bit has two or more of them on average, so that a staged segment
+// serves several bonds, and there are enough for the fixed part (clearing
+// the page, the diagonal's tables) to pay.  Gathered and staged: J1-J2 on 30
+// sites (FP32) 3931 and 3367 us, on 24 sites 48.5 and 45.1 us, in FP64 78.5
+// and 69.1 us, on 20 sites (FP64) 12.0 and 10.8 us; with one bond per high
+// bit (the 24-site ring) 14.6 and 20.4 us, with two bonds in all (13 and 14
+// sites, ring) 3.1 and 3.6, 3.5 and 4.6 us.  (B = 12: the diagonal's split of
+// the low word into halves.)
+inline bool stage_cross(int B, size_t n_bonds, size_t n_groups) {
+  return B == 12 && n_bonds >= 8 && n_bonds >= 2 * n_groups;
+}
+
+// What the cross stages of high word h are built from, on the host and on
+// the device.
+constexpr int kXwStride = 16;
+struct XSource {
+  const XGroup* grp;  // [ng]
+  const double* w;    // [ng * kXwStride]: e_anti - e_par summed per low bit, and in all at [B]
+  int ng, B;
+};
+
+// The cross stages of high word h (SectorLayout::xs).
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+inline void cross_stages(uint32_t h, const uint32_t* hi_base, const XSource& X, XStage* out) {
+  int n = 0;
+  for (int set = 1; set >= 0; --set)
+    for (int g = 0; g < X.ng; ++g) {
+      const XGroup G = X.grp[g];
+      if (((h & G.hbit) != 0u) != (set == 1)) continue;
+      const uint32_t nb = hi_base[h ^ G.hbit];
+      if (nb != 0xffffffffu) out[n++] = XStage{nb, G.info | (set ? 0x80000000u : 0u)};
+    }
+  for (; n < X.ng; ++n) out[n] = XStage{0u, 0u};
+}
+
+// Entry p of xw[h]: a cross bond is antiparallel where the low bit differs
+// from the high one.
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+inline double cross_weight(uint32_t h, int p, const XSource& X) {
+  double w = 0.0;
+  for (int g = 0; g < X.ng; ++g) {
+    const bool set = (h & X.grp[g].hbit) != 0u;
+    const double v = X.w[g * kXwStride + p];
+    w += p == X.B ? (set ? v : 0.0) : (set ? -v : v);
+  }
+  return w;
+}
+
 // copy_shared = false leaves lo_rank, lo_state, nbp16 and xn16 empty: the
-// batch engine reads them from the shared tables (L.low, L.flip), which it
-// uploads once per shape.  host_lists = false leaves the per-high-word lists
-// (hh_off, hh_ent, xb_nb) empty: a single operator builds them on the device
+// engine reads the shared tables (L.low, L.flip; the batch uploads them once
+// per shape) and needs no nbp16.  host_lists = false leaves the per-high-word lists
+// (hh_off, hh_ent, xb_nb or xs and xw) empty: a single operator builds them on the device
 // from hi_base and the bond masks (build_hv_lists), which avoids building
 // and uploading up to 2^NH * (high-high + cross bonds) entries on the host.
 inline SectorLayout build_layout(const ModelSpec& m, int B_override = -1, bool copy_shared = true,
@@ -503,6 +614,9 @@ inline SectorLayout build_layout(const ModelSpec& m, int B_override = -1, bool c
       L.xb.push_back({1u << (ph - B), 1u << pl, b.e_par, b.e_anti, b.t});
     }
   }
+  // the cross bonds of one high bit are adjacent (the kernel stages the
+  // segment across that bit once for all of them)
+  std::stable_sort(L.xb.begin(), L.xb.end(), [](const CrossBond& a, const CrossBond& b) { return a.hbit < b.hbit; });
   auto fill = [](std::vector<double>& d, uint32_t n, double base, const std::vector<double>& su,
                  const std::vector<std::vector<std::pair<uint32_t, std::pair<double, double>>>>& bl) {
     d.assign(n, 0.0);
@@ -530,20 +644,27 @@ inline SectorLayout build_layout(const ModelSpec& m, int B_override = -1, bool c
   L.n_hh_p = round_up((int)L.hh.size(), kPadHH);
   L.n_xb_p = round_up((int)L.xb.size(), kPadX);
   {
-    std::vector<uint32_t> llm, xlb;
-    for (const FlipBond& f : L.ll) llm.push_back(f.mask);
+    std::vector<uint32_t> xlb;
     for (const CrossBond& x : L.xb) xlb.push_back(x.lbit);
-    std::shared_ptr<const FlipTables> F = flip_tables(B, llm, L.n_ll_p, xlb, L.n_xb_p);
-    L.flip = F;
-    L.nbp_off = F->nbp_off;
-    L.xn_off = F->xn_off;
-    if (copy_shared) {
-      L.nbp16 = F->nbp16;
-      L.xn16 = F->xn16;
+    L.flip = flip_tables(B, xlb, L.n_xb_p);
+    L.xn_off = L.flip->xn_off;
+    if (copy_shared) L.xn16 = L.flip->xn16;
+  }
+  if (copy_shared) {
+    L.nbp_off = flip_offsets(B, L.n_ll_p);
+    L.nbp16.assign(L.nbp_off[B + 1], 0);
+    for (int c = 0; c <= B; ++c) {
+      const uint32_t len = (uint32_t)binom(B, c);
+      for (int b = 0; b < L.n_ll_p; ++b)
+        for (uint32_t r = 0; r < len; ++r) {
+          const uint32_t lo = L.lo_state[L.lo_class_off[c] + r];
+          const uint32_t m = b < (int)L.ll.size() ? L.ll[b].mask : 0u, bits = lo & m;
+          L.nbp16[L.nbp_off[c] + flip_index(r, b, L.n_ll_p, kLLChunk)] =
+              (uint16_t)(8u * ((bits != 0u && bits != m) ? L.lo_rank[lo ^ m] : len));
+        }
     }
   }
-  L.ll_t.assign(L.n_ll_p, 0.0);
-  for (size_t b = 0; b < L.ll.size(); ++b) L.ll_t[b] = L.ll[b].t;
+  for (const FlipBond& f : L.ll) L.ll_c.push_back(PageBond{f.t, 8u * page_pos(f.mask), 0u});
   L.hh_mask.assign(L.hh.size(), 0u);
   L.hh_t.assign(L.hh.size(), 0.0);
   for (size_t q = 0; q < L.hh.size(); ++q) {
@@ -596,10 +717,35 @@ inline SectorLayout build_layout(const ModelSpec& m, int B_override = -1, bool c
   }
   L.xb_hbit.assign(L.n_xb_p, 0u);
   for (size_t b = 0; b < L.xb.size(); ++b) L.xb_hbit[b] = L.xb[b].hbit;
+  if (L.xb.size() >= 0x7fffu) throw std::invalid_argument("too many cross bonds");
   L.xb_c.assign(L.n_xb_p, XBondConst{0.0, 0.0, 0u, 0u});
-  for (size_t b = 0; b < L.xb.size(); ++b) L.xb_c[b] = {L.xb[b].e_anti - L.xb[b].e_par, L.xb[b].t, L.xb[b].hbit, 0u};
-  if (host_lists) L.xb_nb.assign((size_t)nhi * L.n_xb_p, 0u);
-  for (uint32_t h = 0; h < (host_lists ? nhi : 0u); ++h) {
+  for (size_t b = 0; b < L.xb.size(); ++b) {
+    const CrossBond& x = L.xb[b];
+    L.xb_c[b] = {x.e_anti - x.e_par, x.t, x.hbit, 0u};
+    L.xb_p.push_back(PageBond{x.t, 8u * page_pos(x.lbit), 0u});
+    if (L.xb_grp.empty() || L.xb_grp.back().hbit != x.hbit) {
+      L.xb_grp.push_back(XGroup{x.hbit, (uint32_t)b});
+      L.xb_w.resize(L.xb_w.size() + kXwStride, 0.0);
+    }
+    L.xb_grp.back().info += 1u << 16;
+    double* w = L.xb_w.data() + L.xb_w.size() - kXwStride;
+    w[__builtin_ctz(x.lbit)] += x.e_anti - x.e_par;
+    w[B] += x.e_anti - x.e_par;
+  }
+  L.stage = stage_cross(B, L.xb.size(), L.xb_grp.size());
+  if (host_lists && L.stage) {
+    const XSource X{L.xb_grp.data(), L.xb_w.data(), (int)L.xb_grp.size(), B};
+    L.xs.assign((size_t)nhi * L.xb_grp.size(), XStage{0u, 0u});
+    L.xw.assign((size_t)nhi * kXwStride, 0.0);
+    for (uint32_t h = 0; h < nhi; ++h)
+      if (L.hi_base[h] != 0xffffffffu) {
+        cross_stages(h, L.hi_base.data(), X, L.xs.data() + (size_t)h * X.ng);
+        for (int p = 0; p <= B; ++p) L.xw[(size_t)h * kXwStride + p] = cross_weight(h, p, X);
+      }
+  }
+  const bool host_nb = host_lists && (copy_shared || !L.stage);
+  if (host_nb) L.xb_nb.assign((size_t)nhi * L.n_xb_p, 0u);
+  for (uint32_t h = 0; h < (host_nb ? nhi : 0u); ++h) {
     const uint32_t own = L.hi_base[h];
     if (own == 0xffffffffu) continue;
     for (int c = 0; c < L.n_xb_p; ++c) {

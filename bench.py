@@ -34,7 +34,7 @@ HBM_PEAK_GBS = 8000.0
 # schedule (the order of SCHEDULES below), from rocprofv3 --pmc FETCH_SIZE and
 # WRITE_SIZE scaled by a copy kernel of known size
 # (profiles/hv_kernel_heisenberg_L24.md); valid for that kernel version and L
-# only.  The schedules that spill write their scratch too.
+# only.
 PMC_TRAFFIC_BYTES = {24: [53.38e6, 53.47e6, 53.35e6, 53.30e6, 58.25e6, 54.01e6]}
 # SHA-256 of the row kernel's source (alps_amd/csrc/ed_device.hpp) when those
 # counters were taken: if the source differs, the table no longer describes
@@ -43,9 +43,9 @@ PMC_TRAFFIC_KERNEL_SHA256 = "8dd16111070282a21ca2d360f4733c5027e3ac0292ebee8e726
 PMC_TRAFFIC_SOURCE = ("profiles/hv_kernel_heisenberg_L24.md, section 'HBM byte counters', column "
                       "'traffic per launch' (FETCH_SIZE + WRITE_SIZE, scaled by the copy kernel), "
                       "row of the chosen schedule")
-# H.v schedules (waves per SIMD, low-low / high-high / cross chunk sizes), in
-# the order of the engine's schedule table
-SCHEDULES = [(8, 4, 4, 2), (8, 4, 8, 2), (6, 4, 8, 2), (6, 4, 4, 2), (8, 8, 4, 2), (6, 8, 8, 4)]
+# H.v schedules (waves per SIMD, low-low / high-high chunk sizes), in the
+# order of the engine's schedule table
+SCHEDULES = [(8, 2, 4), (8, 1, 4), (8, 4, 4), (7, 2, 4), (6, 2, 4), (6, 4, 4)]
 
 
 class HipEvents:
@@ -409,7 +409,7 @@ def j1j2_leg(ev, iterations=300):
         "dim": D, "bonds": len(t["bond_s"]),
         "hv_ms": round(ms, 4), "hv_gbs_8D": round(8.0 * D / (ms * 1e-3) / 1e9, 1),
         "hv_frac_of_hbm_peak": round(8.0 * D / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-        "hv_schedule": {"chosen": sched, "waves_cll_chh_cx": SCHEDULES[sched],
+        "hv_schedule": {"chosen": sched, "waves_cll_chh": SCHEDULES[sched],
                         "ms_per_schedule": None if sched_s is None else [round(t * 1e3, 3) for t in sched_s]},
         "iterations": iterations,
         "f32_eigenvalues": r32["ev"].tolist(), "f64_eigenvalues": r64["ev"].tolist(), "rel_err_f32": rel,
@@ -628,10 +628,10 @@ def main():
                      "frac": round(gbs / HBM_PEAK_GBS, 4),
                      "traffic": PMC_TRAFFIC_BYTES[L][sched] if traffic_ok else None,
                      "traffic_source": PMC_TRAFFIC_SOURCE if traffic_ok else traffic_note,
-                     "kernel": "hv_kernel<float,false,%d,%d,%d,%d>" % SCHEDULES[sched],
+                     "kernel": "hv_kernel<float,false,false,256,%d,%d,%d>" % SCHEDULES[sched],
                      "bytes_per_launch": bytes_per_hv},
         "timed_wall_s": round(wall, 4),
-        "hv_schedule": {"chosen": sched, "waves_cll_chh_cx": SCHEDULES[sched],
+        "hv_schedule": {"chosen": sched, "waves_cll_chh": SCHEDULES[sched],
                         "us_per_schedule": None if sched_s is None else [round(t * 1e6, 2) for t in sched_s]},
         "device": info["name"],
     }
