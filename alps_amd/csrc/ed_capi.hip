@@ -775,6 +775,24 @@ int alps_ed_vector_nrm2(alps_ed_vector x, double* result) {
   });
 }
 
+namespace {
+
+// Scratch of a measurement: partial sums and results, one size so that the
+// pool hands the same buffer to the next call.
+constexpr size_t kMeasureBytes = size_t(24) << 20;
+constexpr int kFlipPairs = 512;  // site pairs per launch of the pair kernel
+static_assert((kMomentBlocks + 64) * moment_values(kMaxHigh) * sizeof(double) <= kMeasureBytes, "moments");
+static_assert((kGramBlocks + 1) * 256 * gram_tiles(2) * sizeof(double) <= kMeasureBytes, "flip matrix");
+static_assert(kFlipPairs * (2 + 2048) * sizeof(double) <= kMeasureBytes, "flip pairs");
+// From this many pairs on, the flip amplitudes of all pairs are formed at
+// once, whose time does not depend on their number.  A call with 24 and 64
+// pairs and with all of them: 24 sites (FP64) pair kernel 97, 198 and 810 us,
+// all at once 123 us; 28 sites (FP32) 837, 1982 and 13333 us against 1094 us;
+// 20 sites 43, 52 and 79 us against 44 us.
+constexpr int kGramPairs = 36;
+
+}  // namespace
+
 int alps_ed_vector_spin_moments(alps_ed_operator op, alps_ed_vector v, double* norm2, double* sz, double* szsz) {
   return guarded([&] {
     require(op != nullptr, "operator is null");
@@ -783,20 +801,19 @@ int alps_ed_vector_spin_moments(alps_ed_operator op, alps_ed_vector v, double* n
     require(v->n == op->layout.D, "vector size != operator dimension");
     require(op->layout.D >= 1, "empty sector");
     const DevLayout& L = op->dev;
-    const int N = L.N;
-    DevBuf stats((size_t)hv_blocks(L) * moment_stat_count(L) * sizeof(double));
-    DevBuf out((size_t)(1 + N + N * N) * sizeof(double));
+    const MomentPlan plan = moment_plan(L);
+    const int nv = moment_values(moment_high_bits(L.NH));
+    PooledBuf work(kMeasureBytes);
+    double* const out = static_cast<double*>(work.p);
     hipStream_t st = current_stream();
     with_dtype(v->dtype, [&](auto z) {
       using V = decltype(z);
-      hip_check(launch_spin_moments<V>(L, v->buf.as<V>(), stats.as<double>(), out.as<double>(), st), "moments");
+      hip_check(launch_spin_moments<V>(L, plan, v->buf.as<V>(), out + nv, out, st), "moments");
     });
-    std::vector<double> h(1 + N + N * N);
-    hip_check(hipMemcpyAsync(h.data(), out.p, h.size() * sizeof(double), hipMemcpyDeviceToHost, st), "copy");
+    std::vector<double> h(nv);
+    hip_check(hipMemcpyAsync(h.data(), out, h.size() * sizeof(double), hipMemcpyDeviceToHost, st), "copy");
     hip_check(hipStreamSynchronize(st), "sync");
-    if (norm2) *norm2 = h[0];
-    if (sz) std::copy(h.begin() + 1, h.begin() + 1 + N, sz);
-    if (szsz) std::copy(h.begin() + 1 + N, h.end(), szsz);
+    read_moments(L, h.data(), norm2, sz, szsz);
   });
 }
 
@@ -832,27 +849,42 @@ int alps_ed_vector_flip_pairs(alps_ed_operator op, alps_ed_vector v, int n_pairs
     require(n_pairs <= (1 << 19), "at most 2^19 pairs per call");
     require(op->layout.D >= 1, "empty sector");
     const DevLayout& L = op->dev;
-    std::vector<uint32_t> masks(2 * (size_t)n_pairs);
     for (int p = 0; p < n_pairs; ++p) {
       require(site_i[p] >= 0 && site_i[p] < L.N && site_j[p] >= 0 && site_j[p] < L.N, "site out of range");
       require(site_i[p] != site_j[p], "a flip pair needs two different sites");
-      masks[2 * p] = 1u << (L.N - 1 - site_j[p]);
-      masks[2 * p + 1] = 1u << (L.N - 1 - site_i[p]);
     }
     hipStream_t st = current_stream();
-    DevBuf dm(masks.size() * sizeof(uint32_t));
-    DevBuf part((size_t)n_pairs * flip_pair_blocks(L) * sizeof(double));
-    DevBuf dout((size_t)n_pairs * sizeof(double));
-    hip_check(hipMemcpyAsync(dm.p, masks.data(), masks.size() * sizeof(uint32_t), hipMemcpyHostToDevice, st),
-              "copy");
+    PooledBuf work(kMeasureBytes);
     with_dtype(v->dtype, [&](auto z) {
       using V = decltype(z);
-      hip_check(launch_flip_pairs<V>(L, v->buf.as<V>(), dm.as<uint32_t>(), n_pairs, part.as<double>(),
-                                     dout.as<double>(), st),
-                "flip pairs");
+      if (n_pairs >= kGramPairs) {
+        const int nv = flip_gram_values(L);
+        double* const sums = static_cast<double*>(work.p);
+        hip_check(launch_flip_gram<V>(L, v->buf.as<V>(), sums + nv, sums, st), "flip pairs");
+        std::vector<double> h(nv);
+        hip_check(hipMemcpyAsync(h.data(), sums, h.size() * sizeof(double), hipMemcpyDeviceToHost, st), "copy");
+        hip_check(hipStreamSynchronize(st), "sync");
+        // an element that is not finite reaches the sums of all pairs there
+        if (std::all_of(h.begin(), h.end(), [](double e) { return std::isfinite(e); })) {
+          for (int p = 0; p < n_pairs; ++p) out[p] = read_flip(L, h.data(), site_i[p], site_j[p]);
+          return;
+        }
+      }
+      std::vector<uint32_t> masks(2 * kFlipPairs);
+      for (int p0 = 0; p0 < n_pairs; p0 += kFlipPairs) {
+        const int np = std::min(kFlipPairs, n_pairs - p0);
+        for (int p = 0; p < np; ++p) {
+          masks[2 * p] = 1u << (L.N - 1 - site_j[p0 + p]);
+          masks[2 * p + 1] = 1u << (L.N - 1 - site_i[p0 + p]);
+        }
+        uint32_t* const dm = static_cast<uint32_t*>(work.p);
+        double* const dout = reinterpret_cast<double*>(dm + 2 * kFlipPairs);
+        hip_check(hipMemcpyAsync(dm, masks.data(), 2 * np * sizeof(uint32_t), hipMemcpyHostToDevice, st), "copy");
+        hip_check(launch_flip_pairs<V>(L, v->buf.as<V>(), dm, np, dout + kFlipPairs, dout, st), "flip pairs");
+        hip_check(hipMemcpyAsync(out + p0, dout, np * sizeof(double), hipMemcpyDeviceToHost, st), "copy");
+        hip_check(hipStreamSynchronize(st), "sync");
+      }
     });
-    hip_check(hipMemcpyAsync(out, dout.p, (size_t)n_pairs * sizeof(double), hipMemcpyDeviceToHost, st), "copy");
-    hip_check(hipStreamSynchronize(st), "sync");
   });
 }
 

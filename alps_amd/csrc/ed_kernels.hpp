@@ -264,12 +264,26 @@ template <class V>
 hipError_t launch_ritz(uint64_t n, const V* const* slots, const double* scale, int m, int nvec,
                        const double* coef, double* const* outs, hipStream_t st);
 
-// Diagonal spin moments of v (ed_measure.hip): out[0] = sum v_r^2,
-// out[1 + i] = sum v_r^2 Sz_i(r), out[1 + N + i*N + j] = sum v_r^2 Sz_i Sz_j;
-// `stats` holds n_seg * moment_stat_count(L) doubles of scratch.
-int moment_stat_count(const DevLayout& L);
+// Diagonal spin moments of v (ed_measure.hip).  The launch leaves
+// moment_values(moment_high_bits(NH)) sums in out, from which read_moments
+// takes sum v_r^2, sum v_r^2 Sz_i(r) and sum v_r^2 Sz_i Sz_j (any may be
+// null); `part` holds as many doubles for each of plan.blocks workgroups.
+constexpr int kMaxHigh = kMaxSites - 12;
+constexpr uint32_t kMomentBlocks = 1024;
+// The kernel is compiled for two numbers of high bits.
+constexpr int moment_high_bits(int nh) { return nh <= 12 ? 12 : kMaxHigh; }
+constexpr int moment_values(int nhx) { return (1 + nhx > 16 ? 768 : 512) + (nhx * (nhx / 2) + 15) / 16 * 16; }
+struct MomentPlan {
+  uint32_t chunk;      // segments per workgroup
+  uint32_t blocks;
+  uint32_t count[13];  // segments per popcount of the low word
+  uint32_t first[14];  // and the first workgroup of each
+};
+MomentPlan moment_plan(const DevLayout& L);
 template <class V>
-hipError_t launch_spin_moments(const DevLayout& L, const V* v, double* stats, double* out, hipStream_t st);
+hipError_t launch_spin_moments(const DevLayout& L, const MomentPlan& plan, const V* v, double* part, double* out,
+                               hipStream_t st);
+void read_moments(const DevLayout& L, const double* sums, double* norm2, double* sz, double* szsz);
 // Flip amplitudes out[p] = <v| S+_i S-_j |v> for masks[2p] = bit of site j,
 // masks[2p+1] = bit of site i (i != j); `part` holds
 // n_pairs * flip_pair_blocks(L) doubles of scratch.
@@ -277,6 +291,15 @@ uint32_t flip_pair_blocks(const DevLayout& L);
 template <class V>
 hipError_t launch_flip_pairs(const DevLayout& L, const V* v, const uint32_t* masks, int n_pairs, double* part,
                              double* out, hipStream_t st);
+// Those of all pairs at once: flip_gram_values(L) sums in out, read with
+// read_flip; `part` holds as many for each of flip_gram_blocks(L) workgroups.
+constexpr uint32_t kGramBlocks = 1536;  // as many as are resident (1024: 5 % slower)
+constexpr int gram_tiles(int ht) { return (ht + 1) * (ht + 2) / 2; }  // pairs of 1 + ht tiles of 16 bits
+uint32_t flip_gram_blocks(const DevLayout& L);
+inline int flip_gram_values(const DevLayout& L) { return 256 * gram_tiles(L.NH <= 16 ? 1 : 2); }
+template <class V>
+hipError_t launch_flip_gram(const DevLayout& L, const V* v, double* part, double* out, hipStream_t st);
+double read_flip(const DevLayout& L, const double* sums, int site_i, int site_j);
 
 // Lanes per row of the listed-flips Bloch kernel (4 measured fastest on the
 // L=24 ring's k = 0 sector: 6.05 us against 6.19 us with 2 and 7.52 us with
