@@ -38,6 +38,7 @@ namespace {
 // slots.  Partial counts follow the producing kernel's grid.
 struct Reducer {
   DevBuf pa, pb, pc, results;
+  MappedBuf mapped;  // results that the kernels write for the host (thread_reducer)
   size_t cap = 0;
   void ensure(size_t nblocks) {
     if (nblocks <= cap) return;
@@ -51,6 +52,8 @@ struct Reducer {
   double* b() { return pb.as<double>(); }
   double* c() { return pc.as<double>(); }
   double* result(int i) { return results.as<double>() + i; }
+  double* mapped_d(int i) { return static_cast<double*>(mapped.d) + i; }
+  double mapped_h(int i) const { return static_cast<const volatile double*>(mapped.h)[i]; }
 };
 
 Reducer& thread_reducer() {
@@ -59,6 +62,7 @@ Reducer& thread_reducer() {
   // teardown may already be under way
   thread_local Reducer* r = new Reducer;
   r->ensure(2048);
+  if (!r->mapped.h) r->mapped.alloc(16 * sizeof(double));
   return *r;
 }
 
@@ -418,11 +422,11 @@ template <class V>
 double dot_sync(uint64_t n, const V* x, const V* y) {
   Reducer& r = thread_reducer();
   hip_check(launch_dot<V>(n, x, y, r.a(), current_stream()), "dot");
-  hip_check(launch_finish(Partials{r.a(), stream_blocks(n)}, nullptr, r.result(0), nullptr, kSum, current_stream()), "finish");
-  double h = 0.0;
-  hip_check(hipMemcpyAsync(&h, r.result(0), sizeof(double), hipMemcpyDeviceToHost, current_stream()), "copy");
+  hip_check(launch_finish(Partials{r.a(), stream_blocks(n)}, nullptr, r.result(0), nullptr, kSum, current_stream(),
+                          r.mapped_d(0)),
+            "finish");
   hip_check(hipStreamSynchronize(current_stream()), "sync");
-  return h;
+  return r.mapped_h(0);
 }
 
 // One Lanczos step of the device-resident recurrence (see alps_ed_lanczos_*),
@@ -446,9 +450,11 @@ void lanczos_step_dev(alps_ed_lanczos lz, int j) {
   double* scale = lz->scale.as<double>();
   hip_check(op_hv<V>(lz->op, cur, w, lz->red.a(), lz->stream), "hv");
   hip_check(launch_update_fused<V>(lz->op->n, w, cur, prev, next, Partials{lz->red.a(), op_hv_blocks(lz->op)},
-                                   Partials{norm_buf(lz, j), lz->norm_count[j & 1]}, alpha + j,
-                                   j > 0 ? beta + j - 1 : nullptr, scale + j, j > 0 ? scale + j - 1 : nullptr,
-                                   norm_buf(lz, j + 1), lz->stream, lz->alpha_h(j), j > 0 ? lz->beta_h(j - 1) : nullptr),
+                                   Partials{norm_buf(lz, j), lz->norm_count[j & 1]},
+                                   UpdateScalars{alpha + j, j > 0 ? beta + j - 1 : nullptr, scale + j,
+                                                 j > 0 ? scale + j - 1 : nullptr, lz->alpha_h(j),
+                                                 j > 0 ? lz->beta_h(j - 1) : nullptr},
+                                   norm_buf(lz, j + 1), lz->stream),
             "update");
   lz->norm_count[(j + 1) & 1] = fused_blocks(lz->op->n);
   // partial reorthogonalization: the omega step of step j and, when it calls
@@ -918,23 +924,22 @@ int alps_ed_lanczos_step_vectors(alps_ed_operator op, alps_ed_vector v_prev, alp
     require(v_prev->dtype == v_cur->dtype && v_cur->dtype == w->dtype, "dtype mismatch");
     Reducer& r = thread_reducer();
     r.ensure(std::max<size_t>(op_hv_blocks(op), stream_blocks(n)));
-    double* res = r.result(0);
-    hip_check(hipMemcpyAsync(res + 2, &beta_prev, sizeof(double), hipMemcpyHostToDevice, current_stream()), "copy");
     with_dtype(w->dtype, [&](auto z) {
       using V = decltype(z);
       V* wv = w->buf.as<V>();
       hip_check(op_hv<V>(op, v_cur->buf.as<V>(), wv, r.a(), current_stream()), "hv");
-      hip_check(launch_finish(Partials{r.a(), op_hv_blocks(op)}, nullptr, res, nullptr, kAlpha, current_stream()), "finish");
-      hip_check(launch_update<V>(n, wv, v_cur->buf.as<V>(), v_prev->buf.as<V>(), wv, res, nullptr, res + 2, nullptr,
-                                 r.b(), current_stream()),
+      UpdateScalars s{};
+      s.alpha_h = r.mapped_d(0);
+      hip_check(launch_update_step<V>(n, wv, v_cur->buf.as<V>(), v_prev->buf.as<V>(),
+                                      Partials{r.a(), op_hv_blocks(op)}, beta_prev, s, r.b(), current_stream()),
                 "update");
-      hip_check(launch_normalize<V>(n, wv, Partials{r.b(), stream_blocks(n)}, res + 1, current_stream()), "normalize");
+      hip_check(launch_normalize<V>(n, wv, Partials{r.b(), fused_blocks(n)}, nullptr, r.mapped_d(1),
+                                    current_stream()),
+                "normalize");
     });
-    double h[2];
-    hip_check(hipMemcpyAsync(h, res, 2 * sizeof(double), hipMemcpyDeviceToHost, current_stream()), "copy");
     hip_check(hipStreamSynchronize(current_stream()), "sync");
-    *alpha = h[0];
-    *beta = h[1];
+    *alpha = r.mapped_h(0);
+    *beta = r.mapped_h(1);
   });
 }
 
@@ -993,17 +998,16 @@ int alps_ed_lanczos_step_vectors_noalloc(alps_ed_operator op, alps_ed_vector v_p
     double* norm_part = hv_part + kStaticHvPartials;
     double* res = norm_part + kStaticNormPartials;
     hipStream_t st = current_stream();
-    // beta_prev enters through a one-element fill kernel, not a host copy
-    hip_check(launch_fill<double>(1, res + 2, beta_prev, st), "fill");
     with_dtype(w->dtype, [&](auto z) {
       using V = decltype(z);
       V* wv = w->buf.as<V>();
       hip_check(op_hv<V>(op, v_cur->buf.as<V>(), wv, hv_part, st), "hv");
-      hip_check(launch_finish(Partials{hv_part, op_hv_blocks(op)}, nullptr, res, nullptr, kAlpha, st), "finish");
-      hip_check(launch_update<V>(n, wv, v_cur->buf.as<V>(), v_prev->buf.as<V>(), wv, res, nullptr, res + 2, nullptr,
-                                 norm_part, st),
+      UpdateScalars s{};
+      s.alpha_j = res;
+      hip_check(launch_update_step<V>(n, wv, v_cur->buf.as<V>(), v_prev->buf.as<V>(),
+                                      Partials{hv_part, op_hv_blocks(op)}, beta_prev, s, norm_part, st),
                 "update");
-      hip_check(launch_normalize<V>(n, wv, Partials{norm_part, stream_blocks(n)}, res + 1, st), "normalize");
+      hip_check(launch_normalize<V>(n, wv, Partials{norm_part, fused_blocks(n)}, res + 1, nullptr, st), "normalize");
     });
     double h[2];
     hip_check(hipMemcpyAsync(h, res, 2 * sizeof(double), hipMemcpyDeviceToHost, st), "copy");

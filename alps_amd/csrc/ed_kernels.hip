@@ -191,31 +191,6 @@ __global__ __launch_bounds__(kBlock) void scatter_copy_kernel(const unsigned cha
 // ---------------------------------------------------------------------------
 // Lanczos update, reductions, vector kernels
 // ---------------------------------------------------------------------------
-// `out` may alias w or u_prev: every element is read before the same thread
-// writes it.
-template <class V>
-__global__ __launch_bounds__(kBlock) void update_kernel(uint64_t n, const V* w, const V* __restrict__ u_cur,
-                                                        const V* u_prev, V* out, const double* __restrict__ alpha,
-                                                        const double* __restrict__ s_cur,
-                                                        const double* __restrict__ beta_prev,
-                                                        const double* __restrict__ s_prev,
-                                                        double* __restrict__ norm_out) {
-  const double sc = s_cur ? *s_cur : 1.0;
-  const double ca = (*alpha) * sc;
-  const double cb = beta_prev ? (*beta_prev) * (s_prev ? *s_prev : 1.0) : 0.0;
-  double acc = 0.0;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    double r = sc * (double)w[i] - ca * (double)u_cur[i];
-    if (beta_prev) r -= cb * (double)u_prev[i];
-    const V rs = (V)r;
-    out[i] = rs;
-    const double rd = (double)rs;
-    acc += rd * rd;
-  }
-  store_partial(norm_out, acc);
-}
-
 // ---------------------------------------------------------------------------
 // Partial reorthogonalization (ReorthDev, ed_kernels.hpp)
 // ---------------------------------------------------------------------------
@@ -410,58 +385,132 @@ __global__ __launch_bounds__(kBlock) void reorth_update_kernel(uint64_t n, int j
   store_partial(norm_out, acc);
 }
 
+// Two sums over a workgroup of kUpdBlock threads, to every thread, through
+// LDS barriers only: the vector elements read before stay in flight.  Once
+// per kernel.
+__device__ __forceinline__ void update_sums(double& a, double& b) {
+  __shared__ double red[2][kUpdBlock / 64];
+  a = wave_sum(a);
+  b = wave_sum(b);
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = a;
+    red[1][threadIdx.x >> 6] = b;
+  }
+  lds_barrier();
+  a = 0.0;
+  b = 0.0;
+#pragma unroll
+  for (int w = 0; w < kUpdBlock / 64; ++w) {
+    a += red[0][w];
+    b += red[1][w];
+  }
+}
+
+// A thread's share of two sums of partials in index order: the first ones are
+// read by the constructor, used by add().
+struct PartialPair {
+  static constexpr int kAhead = 8;
+  double t[kAhead], u;
+  __device__ __forceinline__ PartialPair(const Partials& P, const Partials& Q) {
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      const uint32_t i = threadIdx.x + k * kUpdBlock;
+      t[k] = i < P.n ? P.p[i] : 0.0;
+    }
+    u = threadIdx.x < Q.n ? Q.p[threadIdx.x] : 0.0;
+  }
+  __device__ __forceinline__ void add(const Partials& P, const Partials& Q, double& a, double& b) const {
+    a = 0.0;
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) a += t[k];
+    for (uint32_t i = threadIdx.x + kAhead * kUpdBlock; i < P.n; i += 4u * kUpdBlock) {
+      double x[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) x[k] = i + k * kUpdBlock < P.n ? P.p[i + k * kUpdBlock] : 0.0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) a += x[k];
+    }
+    b = u;
+    for (uint32_t i = threadIdx.x + kUpdBlock; i < Q.n; i += kUpdBlock) b += Q.p[i];
+  }
+};
+
 // One Lanczos update with its scalars: every block first forms, in the same
 // order, scale_j = 1/sqrt(sum(norm_prev)) (the norm of u_j), beta_{j-1} =
-// sqrt(sum(norm_prev)) when j > 0, and alpha_j = scale_j^2 * sum(hv_part)
-// (both sums through one block reduction); block 0 stores them.  Then as
-// update_kernel.  This replaces the two one-block reduction launches of a
-// step.
-template <class V>
-__global__ __launch_bounds__(kBlock) void update_fused_kernel(uint64_t n, const V* w, const V* __restrict__ u_cur,
-                                                              const V* u_prev, V* out, Partials hv_part,
-                                                              Partials norm_prev, double* __restrict__ alpha_j,
-                                                              double* __restrict__ beta_jm1,
-                                                              double* __restrict__ scale_j,
-                                                              const double* __restrict__ scale_jm1,
-                                                              double* __restrict__ norm_out, double* alpha_h,
-                                                              double* beta_h) {
-  const bool has_prev = beta_jm1 != nullptr;
-  const double s_prev = has_prev ? *scale_jm1 : 0.0;
-  double nsum = thread_partials(norm_prev), hsum = thread_partials(hv_part);
-  block_sum_all2(nsum, hsum);
-  const double nrm = sqrt(nsum);
-  const double sc = 1.0 / nrm;
+// sqrt(sum(norm_prev)) when j > 0, and alpha_j = scale_j^2 * sum(hv_part);
+// block 0 stores them.  Then r = scale_j w - alpha_j scale_j u_cur -
+// beta_{j-1} scale_{j-1} u_prev.  STEP: vectors of norm 1 (scale 1, no
+// norm_prev), beta_{j-1} given by value.  `out` may alias w or u_prev: every
+// element is read before the same thread writes it.
+//
+// Bound by its 4 passes over vectors: at 2.7 M rows FP32 43 MB, 6 us at the
+// 7.1 TB/s of a copy that stays in the caches, next to the partials that every
+// block reads (40 KB).  The first kUpdAhead groups of four elements are read
+// before the partials are added up, so that both waits overlap, and two
+// blocks of 512 threads per compute unit read the partials half as often as
+// four of 256: 10.9 -> 9.1 us at that size.  A Lanczos run of 32 steps there
+// takes 886 us with two groups ahead, 904 with four, 930 with blocks of 256
+// threads, 941 with one block of 1024 per compute unit.
+template <class V, bool STEP>
+__global__ __launch_bounds__(kUpdBlock) void update_fused_kernel(uint64_t n, const V* w,
+                                                                 const V* __restrict__ u_cur, const V* u_prev, V* out,
+                                                                 Partials hv_part, Partials norm_prev, double beta,
+                                                                 UpdateScalars S, double* __restrict__ norm_out) {
+  typedef V v4 __attribute__((ext_vector_type(4), aligned(sizeof(V))));
+  constexpr int Q = sizeof(V) == 4 ? kUpdAhead : kUpdAhead / 2;
+  const bool has_prev = STEP || S.beta_jm1 != nullptr;
+  const PartialPair pp(hv_part, norm_prev);
+  const uint64_t stride = (uint64_t)gridDim.x * kUpdBlock;
+  const uint64_t gid = (uint64_t)blockIdx.x * kUpdBlock + threadIdx.x;
+  const uint64_t n4 = n / 4;
+  v4 wv[Q], uv[Q], pv[Q];
+  auto read = [&](uint64_t q0) {
+#pragma unroll
+    for (int c = 0; c < Q; ++c) {
+      const uint64_t q = q0 + c * stride;
+      if (q >= n4) break;
+      wv[c] = *reinterpret_cast<const v4*>(w + 4 * q);
+      uv[c] = *reinterpret_cast<const v4*>(u_cur + 4 * q);
+      if (has_prev) pv[c] = *reinterpret_cast<const v4*>(u_prev + 4 * q);
+    }
+  };
+  read(gid);
+  issue_barrier();
+  const double s_prev = !STEP && has_prev ? *S.scale_jm1 : 0.0;
+  double nsum, hsum;
+  pp.add(hv_part, norm_prev, hsum, nsum);
+  update_sums(nsum, hsum);
+  const double nrm = STEP ? 1.0 : sqrt(nsum);
+  const double sc = STEP ? 1.0 : 1.0 / nrm;
   const double a = sc * sc * hsum;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    *alpha_j = a;
-    *scale_j = sc;
-    if (beta_jm1) *beta_jm1 = nrm;
-    // host-mapped copies for the stopping test (no copy launch needed)
-    if (alpha_h) *alpha_h = a;
-    if (beta_h && beta_jm1) *beta_h = nrm;
+    if (S.alpha_j) *S.alpha_j = a;
+    if (S.scale_j) *S.scale_j = sc;
+    if (S.beta_jm1) *S.beta_jm1 = nrm;
+    // host-mapped copies (no copy launch needed)
+    if (S.alpha_h) *S.alpha_h = a;
+    if (S.beta_h && S.beta_jm1) *S.beta_h = nrm;
   }
   const double ca = a * sc;
-  const double cb = has_prev ? nrm * s_prev : 0.0;
+  const double cb = STEP ? beta : has_prev ? nrm * s_prev : 0.0;
   double acc = 0.0;
-  // four consecutive elements per thread and iteration (vector loads)
-  typedef V v4 __attribute__((ext_vector_type(4), aligned(sizeof(V))));
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t n4 = n / 4;
-  for (uint64_t q = gid; q < n4; q += stride) {
-    const v4 wv = *reinterpret_cast<const v4*>(w + 4 * q);
-    const v4 uv = *reinterpret_cast<const v4*>(u_cur + 4 * q);
-    const v4 pv = has_prev ? *reinterpret_cast<const v4*>(u_prev + 4 * q) : uv;
-    v4 o;
+  for (uint64_t q0 = gid; q0 < n4; q0 += Q * stride) {
+    if (q0 != gid) read(q0);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      double r = sc * (double)wv[c] - ca * (double)uv[c];
-      if (has_prev) r -= cb * (double)pv[c];
-      o[c] = (V)r;
-      const double rd = (double)o[c];
-      acc += rd * rd;
+    for (int c = 0; c < Q; ++c) {
+      const uint64_t q = q0 + c * stride;
+      if (q >= n4) break;
+      v4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        double r = sc * (double)wv[c][e] - ca * (double)uv[c][e];
+        if (has_prev) r -= cb * (double)pv[c][e];
+        o[e] = (V)r;
+        const double rd = (double)o[e];
+        acc += rd * rd;
+      }
+      *reinterpret_cast<v4*>(out + 4 * q) = o;
     }
-    *reinterpret_cast<v4*>(out + 4 * q) = o;
   }
   for (uint64_t i = 4 * n4 + gid; i < n; i += stride) {
     double r = sc * (double)w[i] - ca * (double)u_cur[i];
@@ -471,7 +520,16 @@ __global__ __launch_bounds__(kBlock) void update_fused_kernel(uint64_t n, const 
     const double rd = (double)rs;
     acc += rd * rd;
   }
-  store_partial(norm_out, acc);
+  acc = wave_sum(acc);
+  __shared__ double red_out[kUpdBlock / 64];
+  if ((threadIdx.x & 63) == 0) red_out[threadIdx.x >> 6] = acc;
+  lds_barrier();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+#pragma unroll
+    for (int q = 0; q < kUpdBlock / 64; ++q) s += red_out[q];
+    norm_out[blockIdx.x] = s;
+  }
 }
 
 template <class V>
@@ -503,14 +561,46 @@ __global__ __launch_bounds__(kBlock) void finish_kernel(Partials in, const doubl
   }
 }
 
+// v *= 1/sqrt(sum(norm_in)), the first elements read before the sum is formed
+// (as update_fused_kernel, whose block and group sizes it takes).
 template <class V>
-__global__ __launch_bounds__(kBlock) void normalize_kernel(uint64_t n, V* v, Partials norm_in, double* b_out) {
-  const double ss = sum_partials(norm_in);
+__global__ __launch_bounds__(kUpdBlock) void normalize_kernel(uint64_t n, V* v, Partials norm_in, double* b_out,
+                                                              double* b_h) {
+  typedef V v4 __attribute__((ext_vector_type(4), aligned(sizeof(V))));
+  constexpr int Q = sizeof(V) == 4 ? kUpdAhead : kUpdAhead / 2;
+  const PartialPair pp(norm_in, Partials{nullptr, 0});
+  const uint64_t stride = (uint64_t)gridDim.x * kUpdBlock;
+  const uint64_t gid = (uint64_t)blockIdx.x * kUpdBlock + threadIdx.x;
+  const uint64_t n4 = n / 4;
+  v4 x[Q];
+  auto read = [&](uint64_t q0) {
+#pragma unroll
+    for (int c = 0; c < Q; ++c)
+      if (q0 + c * stride < n4) x[c] = *reinterpret_cast<const v4*>(v + 4 * (q0 + c * stride));
+  };
+  read(gid);
+  issue_barrier();
+  double ss, none;
+  pp.add(norm_in, Partials{nullptr, 0}, ss, none);
+  update_sums(ss, none);
   const double inv = 1.0 / sqrt(ss);
-  if (blockIdx.x == 0 && threadIdx.x == 0 && b_out) *b_out = sqrt(ss);
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
-    v[i] = (V)(inv * (double)v[i]);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (b_out) *b_out = sqrt(ss);
+    if (b_h) *b_h = sqrt(ss);
+  }
+  for (uint64_t q0 = gid; q0 < n4; q0 += Q * stride) {
+    if (q0 != gid) read(q0);
+#pragma unroll
+    for (int c = 0; c < Q; ++c) {
+      const uint64_t q = q0 + c * stride;
+      if (q >= n4) break;
+      v4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (V)(inv * (double)x[c][e]);
+      *reinterpret_cast<v4*>(v + 4 * q) = o;
+    }
+  }
+  for (uint64_t i = 4 * n4 + gid; i < n; i += stride) v[i] = (V)(inv * (double)v[i]);
 }
 
 template <class V>
@@ -699,21 +789,18 @@ hipError_t launch_hv(const DevLayout& L, const V* x, V* y, double* dot_out, hipS
 }
 
 template <class V>
-hipError_t launch_update(uint64_t n, const V* w, const V* u_cur, const V* u_prev, V* out, const double* alpha,
-                         const double* s_cur, const double* beta_prev, const double* s_prev, double* norm_out,
-                         hipStream_t st) {
-  hipLaunchKernelGGL((update_kernel<V>), dim3(stream_blocks(n)), dim3(kBlock), 0, st, n, w, u_cur, u_prev, out,
-                     alpha, s_cur, beta_prev, s_prev, norm_out);
+hipError_t launch_update_fused(uint64_t n, const V* w, const V* u_cur, const V* u_prev, V* out, Partials hv_part,
+                               Partials norm_prev, const UpdateScalars& S, double* norm_out, hipStream_t st) {
+  hipLaunchKernelGGL((update_fused_kernel<V, false>), dim3(fused_blocks(n)), dim3(kUpdBlock), 0, st, n, w, u_cur,
+                     u_prev, out, hv_part, norm_prev, 0.0, S, norm_out);
   return hipGetLastError();
 }
 
 template <class V>
-hipError_t launch_update_fused(uint64_t n, const V* w, const V* u_cur, const V* u_prev, V* out, Partials hv_part,
-                               Partials norm_prev, double* alpha_j, double* beta_jm1, double* scale_j,
-                               const double* scale_jm1, double* norm_out, hipStream_t st, double* alpha_h,
-                               double* beta_h) {
-  hipLaunchKernelGGL((update_fused_kernel<V>), dim3(fused_blocks(n)), dim3(kBlock), 0, st, n, w, u_cur, u_prev, out,
-                     hv_part, norm_prev, alpha_j, beta_jm1, scale_j, scale_jm1, norm_out, alpha_h, beta_h);
+hipError_t launch_update_step(uint64_t n, V* w, const V* v_cur, const V* v_prev, Partials hv_part, double beta_prev,
+                              const UpdateScalars& S, double* norm_out, hipStream_t st) {
+  hipLaunchKernelGGL((update_fused_kernel<V, true>), dim3(fused_blocks(n)), dim3(kUpdBlock), 0, st, n, w, v_cur,
+                     v_prev, w, hv_part, Partials{nullptr, 0}, beta_prev, S, norm_out);
   return hipGetLastError();
 }
 
@@ -744,8 +831,8 @@ hipError_t launch_finish(Partials in, const double* scale, double* out, double* 
 }
 
 template <class V>
-hipError_t launch_normalize(uint64_t n, V* v, Partials norm_in, double* b_out, hipStream_t st) {
-  hipLaunchKernelGGL((normalize_kernel<V>), dim3(stream_blocks(n)), dim3(kBlock), 0, st, n, v, norm_in, b_out);
+hipError_t launch_normalize(uint64_t n, V* v, Partials norm_in, double* b_out, double* b_h, hipStream_t st) {
+  hipLaunchKernelGGL((normalize_kernel<V>), dim3(fused_blocks(n)), dim3(kUpdBlock), 0, st, n, v, norm_in, b_out, b_h);
   return hipGetLastError();
 }
 
@@ -855,13 +942,12 @@ hipError_t launch_elements(const DevLayout& L, uint64_t row0, uint64_t nrows, in
 
 #define ALPS_ED_INSTANTIATE(V)                                                                              \
   template hipError_t launch_hv<V>(const DevLayout&, const V*, V*, double*, hipStream_t, int);              \
-  template hipError_t launch_update<V>(uint64_t, const V*, const V*, const V*, V*, const double*,           \
-                                       const double*, const double*, const double*, double*, hipStream_t); \
   template hipError_t launch_dot<V>(uint64_t, const V*, const V*, double*, hipStream_t);                    \
   template hipError_t launch_update_fused<V>(uint64_t, const V*, const V*, const V*, V*, Partials, Partials,   \
-                                             double*, double*, double*, const double*, double*, hipStream_t,   \
-                                             double*, double*);                                                \
-  template hipError_t launch_normalize<V>(uint64_t, V*, Partials, double*, hipStream_t);                    \
+                                             const UpdateScalars&, double*, hipStream_t);                      \
+  template hipError_t launch_update_step<V>(uint64_t, V*, const V*, const V*, Partials, double,             \
+                                            const UpdateScalars&, double*, hipStream_t);                    \
+  template hipError_t launch_normalize<V>(uint64_t, V*, Partials, double*, double*, hipStream_t);           \
   template hipError_t launch_fill_random<V>(uint64_t, V*, uint64_t, double, double, hipStream_t);           \
   template hipError_t launch_fill<V>(uint64_t, V*, double, hipStream_t);                                    \
   template hipError_t launch_axpby<V>(uint64_t, V*, double, const V*, double, hipStream_t);                 \

@@ -126,11 +126,14 @@ inline unsigned stream_blocks(uint64_t n) {
   return (unsigned)b;
 }
 
-// Blocks of the fused update: as the streaming kernels (at most 1024).  Every
-// block also re-reads all partials of the step; on the L=24 ring 1024 blocks
-// were 4 % faster per Lanczos step than 256 blocks, and than a separate
-// one-block scalar kernel before a full-width update.
-inline unsigned fused_blocks(uint64_t n) { return stream_blocks(n); }
+// The update and normalization kernels: threads per block, groups of four
+// elements that a thread reads ahead (half as many in FP64) and blocks.
+constexpr int kUpdBlock = 512;
+constexpr int kUpdAhead = 2;
+inline unsigned fused_blocks(uint64_t n) {
+  const uint64_t b = (n + (uint64_t)kUpdBlock * 4 - 1) / ((uint64_t)kUpdBlock * 4);
+  return (unsigned)(b < 1 ? 1 : b > 512 ? 512 : b);
+}
 
 // Blocks of the H.v kernel: one per segment.
 inline unsigned hv_blocks(const DevLayout& L) { return L.n_seg ? L.n_seg : 1; }
@@ -161,15 +164,6 @@ enum { kSum = 0, kNorm = 1, kAlpha = 2 };
 // out_h, when set (host-mapped memory), receives a copy of out[0].
 hipError_t launch_finish(Partials in, const double* scale, double* out, double* out2, int mode, hipStream_t st,
                          double* out_h = nullptr);
-
-// Lanczos update: r = s_cur*w - alpha*s_cur*u_cur - beta_prev*s_prev*u_prev
-// stored into `out` (may alias w or u_prev); per-block partials of |r|^2
-// into norm_out.  Scalars are read from device memory; beta_prev == nullptr
-// drops the last term; null s_cur / s_prev mean 1.
-template <class V>
-hipError_t launch_update(uint64_t n, const V* w, const V* u_cur, const V* u_prev, V* out, const double* alpha,
-                         const double* s_cur, const double* beta_prev, const double* s_prev, double* norm_out,
-                         hipStream_t st);
 
 // Partial reorthogonalization (Simon, "The Lanczos algorithm with partial
 // reorthogonalization", Math. Comp. 42 (1984) 115-142) of a recurrence whose
@@ -220,26 +214,38 @@ hipError_t launch_hh_fill(uint32_t nhi, const uint32_t* hi_base, const uint32_t*
 // and lists are on the device.
 hipError_t launch_seg_rec(const DevLayout& L, SegRec* out, hipStream_t st);
 
+// Where the update leaves its scalars (any may be null; scale_jm1 is read).
+// alpha_h / beta_h are host-mapped memory and receive copies of alpha_j and
+// beta_{j-1}.
+struct UpdateScalars {
+  double* alpha_j;
+  double* beta_jm1;  // null at j = 0: no u_prev
+  double* scale_j;
+  const double* scale_jm1;
+  double* alpha_h;
+  double* beta_h;
+};
 // The update with its scalars (one launch instead of three): scale_j =
 // 1/sqrt(sum(norm_prev)), beta_{j-1} = sqrt(sum(norm_prev)) (when beta_jm1 is
-// set; it is null at j = 0), alpha_j = scale_j^2 * sum(hv_part); then
+// set), alpha_j = scale_j^2 * sum(hv_part); then
 // r = scale_j w - alpha_j scale_j u_cur - beta_{j-1} scale_{j-1} u_prev into
-// `out` with per-block partials of |r|^2 into norm_out (fused_blocks(n) of
-// them).  The scalars are bit-identical to launch_finish + launch_update.
-// alpha_h / beta_h, when set (host-mapped memory), receive copies of alpha_j
-// and beta_{j-1}.
+// `out` (may alias w or u_prev) with per-block partials of |r|^2 into
+// norm_out (fused_blocks(n) of them).
 template <class V>
 hipError_t launch_update_fused(uint64_t n, const V* w, const V* u_cur, const V* u_prev, V* out, Partials hv_part,
-                               Partials norm_prev, double* alpha_j, double* beta_jm1, double* scale_j,
-                               const double* scale_jm1, double* norm_out, hipStream_t st, double* alpha_h = nullptr,
-                               double* beta_h = nullptr);
+                               Partials norm_prev, const UpdateScalars& S, double* norm_out, hipStream_t st);
+// The same on vectors of norm 1: w -= alpha v_cur + beta_prev v_prev,
+// alpha = sum(hv_part).
+template <class V>
+hipError_t launch_update_step(uint64_t n, V* w, const V* v_cur, const V* v_prev, Partials hv_part, double beta_prev,
+                              const UpdateScalars& S, double* norm_out, hipStream_t st);
 
 // per-block partials of sum x_i y_i
 template <class V>
 hipError_t launch_dot(uint64_t n, const V* x, const V* y, double* partials, hipStream_t st);
-// v *= 1/sqrt(sum(norm_in)); block 0 stores sqrt(sum) to b_out
+// v *= 1/sqrt(sum(norm_in)); block 0 stores sqrt(sum) to b_out and b_h
 template <class V>
-hipError_t launch_normalize(uint64_t n, V* v, Partials norm_in, double* b_out, hipStream_t st);
+hipError_t launch_normalize(uint64_t n, V* v, Partials norm_in, double* b_out, double* b_h, hipStream_t st);
 
 template <class V>
 hipError_t launch_fill_random(uint64_t n, V* v, uint64_t seed, double lo, double hi, hipStream_t st);
