@@ -225,6 +225,8 @@ struct Problem {
   alps_ed_solve_result result{};
   // Which of the H.v launches its items belong to (launch_batch_hv).
   bool staged() const { return !trans && layout.stage; }
+  // Whether its updates form the scalars of a step.
+  bool fused() const { return n_hv + n_chunks <= kBatchFuse; }
 };
 
 }  // namespace
@@ -232,6 +234,8 @@ struct Problem {
 struct alps_ed_batch_s {
   alps_ed_batch_config cfg{};
   hipStream_t stream = nullptr;
+  hipStream_t stream64 = nullptr;  // the FP64 problems' steps, between fork and join
+  std::unique_ptr<Event> fork, join;
   void* dev_base = nullptr;
   char* host_base = nullptr;   // mapped, pinned
   char* host_dev = nullptr;    // device view of host_base
@@ -268,6 +272,7 @@ struct alps_ed_batch_s {
   std::map<std::pair<const void*, const void*>, std::unique_ptr<SharedTables>> shared;
 
   ~alps_ed_batch_s() {
+    if (stream64) (void)hipStreamSynchronize(stream64);
     if (stream) (void)hipStreamSynchronize(stream);
     if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
     if (dev_base) (void)hipFree(dev_base);
@@ -275,6 +280,7 @@ struct alps_ed_batch_s {
     if (stage) (void)hipHostFree(stage);
     if (tstage) (void)hipHostFree(tstage);
     if (rstage) (void)hipHostFree(rstage);
+    if (stream64) (void)hipStreamDestroy(stream64);
     if (stream) (void)hipStreamDestroy(stream);
   }
 };
@@ -399,7 +405,7 @@ Footprint footprint(const Problem& p) {
   f.dev += align_up((size_t)p.cap * stride * es);
   f.dev += 3 * align_up((size_t)(p.max_iter + 2) * 8);  // alpha, beta, scale
   f.dev += align_up((size_t)std::max<uint32_t>(p.n_hv, 1) * 8);
-  f.dev += align_up((size_t)p.n_chunks * 8);
+  f.dev += align_up((size_t)p.n_chunks * 2 * 8);
   if (p.fp32) {
     f.dev += align_up((size_t)p.nvr * (p.max_iter + 1) * 8);  // coef
     f.dev += align_up((size_t)p.nvr * p.n * 8);              // Ritz vectors
@@ -450,6 +456,7 @@ void place(alps_ed_batch b, Problem& p, char* stage, const SharedTables& sh) {
   J.stride = stride;
   J.cap = p.cap;
   J.n_chunks = p.n_chunks;
+  J.fuse = p.fused() ? 1u : 0u;
   J.j0 = 0;
   J.jmax = p.max_iter;
   J.seed = p.seed;
@@ -462,7 +469,7 @@ void place(alps_ed_batch b, Problem& p, char* stage, const SharedTables& sh) {
   J.part_hv = reinterpret_cast<double*>(q);
   q += align_up((size_t)std::max<uint32_t>(p.n_hv, 1) * 8);
   J.part_up = reinterpret_cast<double*>(q);
-  q += align_up((size_t)p.n_chunks * 8);
+  q += align_up((size_t)p.n_chunks * 2 * 8);
   char* h = b->host_base + p.host_off;
   const size_t hoff = (size_t)(h - b->host_base);
   p.host_alpha = reinterpret_cast<double*>(h);
@@ -624,10 +631,12 @@ struct Group {
   BatchItem* up64 = nullptr;
   BatchItem* st32 = nullptr;  // start-vector items of the problems new this round
   BatchItem* st64 = nullptr;
-  uint32_t* list = nullptr;
-  uint32_t* st_list = nullptr;
+  uint32_t* list = nullptr;     // fused jobs
+  uint32_t* big_list = nullptr; // the others
+  uint32_t* st_list = nullptr;  // and those of them new this round
   uint32_t n_hv32[2] = {0, 0}, n_hv64[2] = {0, 0};
-  uint32_t n_up32 = 0, n_up64 = 0, n_list = 0, n_st32 = 0, n_st64 = 0, n_st_list = 0;
+  uint32_t n_up32 = 0, n_up64 = 0, n_list = 0, n_big_list = 0, n_st32 = 0, n_st64 = 0,
+           n_st_list = 0;
   uint32_t lds32 = kHvMinLds, lds64 = kHvMinLds;  // the largest LDS need of an H.v item
 };
 
@@ -639,14 +648,13 @@ Group upload_group(alps_ed_batch b, const std::vector<Problem*>& run) {
   // new this round, then the job list and the new jobs' list.
   Group g;
   const size_t nj = run.size();
-  size_t n_hv[2][2] = {{0, 0}, {0, 0}}, n_up[2] = {0, 0}, n_st[2] = {0, 0}, n_new = 0;
+  size_t n_hv[2][2] = {{0, 0}, {0, 0}}, n_up[2] = {0, 0}, n_st[2] = {0, 0};
   for (const Problem* p : run) {
     const int f = p->fp32 ? 1 : 0;
     n_hv[f][p->staged()] += p->n_hv;
     n_up[f] += p->n_chunks;
     if (p->j == 0) {
       n_st[f] += p->n_chunks;
-      ++n_new;
     }
     if (!p->trans) {
       uint32_t& lds = p->fp32 ? g.lds32 : g.lds64;
@@ -682,12 +690,10 @@ Group upload_group(alps_ed_batch b, const std::vector<Problem*>& run) {
   BatchItem* st64 = region(n_st[0], g.st64, g.n_st64);
   uint32_t* lst = reinterpret_cast<uint32_t*>(s + o);
   g.list = reinterpret_cast<uint32_t*>(d + o);
-  g.n_list = (uint32_t)nj;
+  // (fused jobs from the front, the others from the back)
   o += bl;
   uint32_t* new_list = reinterpret_cast<uint32_t*>(s + o);
   g.st_list = reinterpret_cast<uint32_t*>(d + o);
-  g.n_st_list = (uint32_t)n_new;
-  uint32_t k_new = 0;
   for (uint32_t i = 0; i < nj; ++i) {
     const Problem& p = *run[i];
     BatchItem*& hv = (p.fp32 ? hv32 : hv64)[p.staged()];
@@ -697,10 +703,12 @@ Group upload_group(alps_ed_batch b, const std::vector<Problem*>& run) {
     if (p.j == 0) {
       BatchItem*& st = p.fp32 ? st32 : st64;
       for (uint32_t c = 0; c < p.n_chunks; ++c) *st++ = {i, c};
-      new_list[k_new++] = i;
+      if (!p.fused()) new_list[g.n_st_list++] = i;
     }
-    lst[i] = i;
+    if (p.fused()) lst[g.n_list++] = i;
+    else lst[nj - ++g.n_big_list] = i;
   }
+  g.big_list = g.list + g.n_list;
   hip_check(hipMemcpyAsync(d, s, total, hipMemcpyHostToDevice, b->stream), "upload work lists");
   return g;
 }
@@ -1055,33 +1063,46 @@ void round(alps_ed_batch b) {
   if (!run.empty()) {
     for (Problem* p : run) p->job.j0 = p->j;
     Group g = upload_group(b, run);
-    if (g.n_st_list) {
+    if (g.n_st32 + g.n_st64) {
       hip_check(launch_batch_start<float>(g.jobs, g.st32, g.n_st32, b->stream), "batch start");
       hip_check(launch_batch_start<double>(g.jobs, g.st64, g.n_st64, b->stream), "batch start");
       hip_check(launch_batch_finish(g.jobs, g.st_list, g.n_st_list, 0, kBatchStart, b->stream), "batch finish");
     }
     auto steps = [&] {
+      // Without reduction launches the two precisions meet only at the end
+      // of the group, so the FP64 problems (small ones, a few wavefronts)
+      // run beside the FP32 ones on a stream of their own.
+      const bool two = g.n_big_list == 0 && g.n_up32 != 0 && g.n_up64 != 0;
+      hipStream_t st64 = two ? b->stream64 : b->stream;
+      if (two) {
+        hip_check(hipEventRecord(b->fork->e, b->stream), "event");
+        hip_check(hipStreamWaitEvent(st64, b->fork->e, 0), "event");
+      }
       for (int t = 0; t < S; ++t) {
         for (int s = 0; s < 2; ++s) {
           hip_check(launch_batch_hv<float>(g.jobs, g.hv32[s], g.n_hv32[s], t, s == 1, g.lds32, b->stream), "batch hv");
-          hip_check(launch_batch_hv<double>(g.jobs, g.hv64[s], g.n_hv64[s], t, s == 1, g.lds64, b->stream),
-                    "batch hv");
+          hip_check(launch_batch_hv<double>(g.jobs, g.hv64[s], g.n_hv64[s], t, s == 1, g.lds64, st64), "batch hv");
         }
-        hip_check(launch_batch_finish(g.jobs, g.list, g.n_list, t, kBatchAlpha, b->stream), "batch finish");
+        hip_check(launch_batch_finish(g.jobs, g.big_list, g.n_big_list, t, kBatchAlpha, b->stream), "batch finish");
         hip_check(launch_batch_update<float>(g.jobs, g.up32, g.n_up32, t, b->stream), "batch update");
-        hip_check(launch_batch_update<double>(g.jobs, g.up64, g.n_up64, t, b->stream), "batch update");
-        hip_check(launch_batch_finish(g.jobs, g.list, g.n_list, t, kBatchBeta, b->stream), "batch finish");
+        hip_check(launch_batch_update<double>(g.jobs, g.up64, g.n_up64, t, st64), "batch update");
+        hip_check(launch_batch_finish(g.jobs, g.big_list, g.n_big_list, t, kBatchBeta, b->stream), "batch finish");
       }
+      if (two) {
+        hip_check(hipEventRecord(b->join->e, st64), "event");
+        hip_check(hipStreamWaitEvent(b->stream, b->join->e, 0), "event");
+      }
+      hip_check(launch_batch_finish(g.jobs, g.list, g.n_list, S, kBatchLast, b->stream), "batch finish");
     };
     // The launches of a round are fixed by the work-list addresses and
     // counts and S (each job's step base j0 is read from device memory), so
     // a round that repeats the previous one replays them from a graph.
     bool replayed = false;
-    if (b->cfg.graphs && g.n_st_list == 0) {
+    if (b->cfg.graphs && g.n_st32 + g.n_st64 == 0) {
       const std::vector<uint64_t> key{(uint64_t)g.jobs, (uint64_t)g.hv32[0], (uint64_t)g.hv32[1], (uint64_t)g.hv64[0],
                                       (uint64_t)g.hv64[1], (uint64_t)g.up32, (uint64_t)g.up64, (uint64_t)g.list,
                                       g.n_hv32[0], g.n_hv32[1], g.n_hv64[0], g.n_hv64[1], g.n_up32, g.n_up64,
-                                      g.n_list, g.lds32, g.lds64, (uint64_t)S};
+                                      g.n_list, g.n_big_list, g.lds32, g.lds64, (uint64_t)S};
       if (key == b->last_key) {
         if (!b->graph_exec || key != b->graph_key) {
           if (b->graph_exec) hip_check(hipGraphExecDestroy(b->graph_exec), "graph destroy");
@@ -1197,6 +1218,9 @@ int alps_ed_batch_create(const alps_ed_batch_config* cfg, alps_ed_batch* out) {
     }
     budget = align_up(budget);
     hip_check(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking), "hipStreamCreate");
+    hip_check(hipStreamCreateWithFlags(&b->stream64, hipStreamNonBlocking), "hipStreamCreate");
+    b->fork.reset(new Event);
+    b->join.reset(new Event);
     hip_check(hipMalloc(&b->dev_base, budget), "hipMalloc arena");
     b->arena.init(budget);
     const size_t hbytes = align_up(cfg->host_bytes ? cfg->host_bytes : ((size_t)256 << 20));

@@ -7,9 +7,10 @@
 // representatives) in a momentum sector -- and (problem, row chunk) for the
 // vector kernels, so a batch of small
 // sectors fills the whole chip in one launch instead of leaving it idle
-// between many tiny ones.  A Lanczos step of the batch is four launches
-// (H.v with the alpha partials, alpha, update with the beta partials,
-// beta), with no host round trip; the host only reads alpha and beta (from
+// between many tiny ones.  A Lanczos step of the batch is two launches per
+// precision (H.v with the alpha partials; the update, which forms the step's
+// scalars from the partials), the two precisions side by side on two
+// streams, with no host round trip; the host only reads alpha and beta (from
 // mapped host memory) when it tests convergence.
 //
 // The per-problem arithmetic (segments, chunks, partial sums and their
@@ -47,8 +48,18 @@ struct BatchJob {
   double* host_alpha;   // device view of mapped host mirrors
   double* host_beta;
   double* part_hv;      // [n_hv]      partials of the H.v dot
-  double* part_up;      // [n_chunks]  partials of |r|^2
+  double* part_up;      // [2 * n_chunks]  partials of |u_j|^2, even and odd j
+  uint32_t fuse;        // the update forms the step's scalars (kBatchFuse)
+  uint32_t pad;
 };
+
+// Up to this many partials of a problem (of its H.v and of a norm), every
+// block of its update adds them up itself; beyond, a reduction launch per
+// scalar is cheaper than blocks x partials reads.  Whole solves with and
+// without: 32 of 16 sites 1.7 and 2.1 ms, 16 of 20 sites 3.7 and 4.1 ms, 4 of
+// 23 sites (3369 partials, 36 MB read per step) 5.7 and 6.0 ms, 4 of 24 sites
+// (6737 partials, 142 MB) 11.0 and 10.1 ms.
+constexpr uint32_t kBatchFuse = 4096;
 
 // Ritz vectors and their Rayleigh quotients for FP32 lanes:
 //   out_i = sum_{j<m} coef[i*m + j] * scale[j] * u_j   (FP64, i < nv)
@@ -81,7 +92,7 @@ struct BatchItem {
 
 constexpr uint32_t kBatchChunk = (uint32_t)kBlock * 4;  // rows per vector work item
 
-enum { kBatchStart = 0, kBatchAlpha = 1, kBatchBeta = 2 };
+enum { kBatchStart = 0, kBatchAlpha = 1, kBatchBeta = 2, kBatchLast = 3 };
 
 // Start vectors u_0 (uniform [-1,1) from the job's seed, the same values as
 // launch_fill_random) with partials of |u_0|^2.
@@ -91,12 +102,14 @@ hipError_t launch_batch_start(const BatchJob* jobs, const BatchItem* items, uint
 template <class V>
 hipError_t launch_batch_hv(const BatchJob* jobs, const BatchItem* items, uint32_t n_items, int t, bool stage,
                            uint32_t lds, hipStream_t st);
-// r = s_j w - alpha_j s_j u_j - beta_{j-1} s_{j-1} u_{j-1} in place of w.
+// r = s_j w - alpha_j s_j u_j - beta_{j-1} s_{j-1} u_{j-1} in place of w; for
+// fused jobs with alpha_j, s_j and beta_{j-1} from the partials.
 template <class V>
 hipError_t launch_batch_update(const BatchJob* jobs, const BatchItem* items, uint32_t n_items, int t,
                                hipStream_t st);
 // One block per listed job: scale[0] (kBatchStart), alpha_j (kBatchAlpha)
-// or beta_j and scale[j+1] (kBatchBeta), from the partials in index order.
+// or beta_j and scale[j+1] (kBatchBeta), from the partials in index order;
+// kBatchLast: beta and scale after the last step of a group of t.
 hipError_t launch_batch_finish(const BatchJob* jobs, const uint32_t* job_list, uint32_t n_jobs, int t, int mode,
                                hipStream_t st);
 template <class V>

@@ -66,9 +66,23 @@ __global__ __launch_bounds__(kBlock, HvWaves<V>::value) void batch_hv_kernel(con
   hv_segment_at<V, true, STAGE>(L, seg_record(L, h), x, y, part + it.idx);
 }
 
+// Where stage j (the start for j = 0, the update of step j - 1 otherwise)
+// leaves its partials of |u_j|^2: two buffers in turn, as the blocks of an
+// update read one while others fill the next.
+__device__ __forceinline__ double* norm_part(const BatchJob* J, int j) {
+  return ldc(&J->part_up) + ((j & 1) != 0 ? ldc(&J->n_chunks) : 0u);
+}
+
+// One row chunk of an update.  A fused job's blocks each form alpha_j, scale_j
+// and beta_{j-1} from the partials (in the same order as batch_finish_kernel,
+// so the values are the same) while their vector elements, read before, are
+// on the way; the first block stores them.  Bound by latency at the sizes of a
+// batch: 64 chains of 12 to 20 sites 12.6 us, against 9.8 us and two
+// reduction launches of 3.6 us each.
 template <class V>
 __global__ __launch_bounds__(kBlock) void batch_update_kernel(const BatchJob* __restrict__ jobs,
                                                               const BatchItem* __restrict__ items, int t) {
+  typedef V v4 __attribute__((ext_vector_type(4), aligned(sizeof(V))));
   const BatchItem it = ldc_struct(items + blockIdx.x);
   const BatchJob* J = jobs + it.job;
   const int j = ldc(&J->j0) + t;
@@ -79,24 +93,52 @@ __global__ __launch_bounds__(kBlock) void batch_update_kernel(const BatchJob* __
   const uint32_t cap = ldc(&J->cap);
   const V* u = slot_ptr<V>(vec, stride, cap, j);
   V* w = slot_ptr<V>(vec, stride, cap, j + 1);
-  const double* alpha = ldc(&J->alpha);
-  const double* beta = ldc(&J->beta);
-  const double* scale = ldc(&J->scale);
-  const double sc = ldc(scale + j);
-  const double ca = ldc(alpha + j) * sc;
+  double* alpha = ldc(&J->alpha);
+  double* beta = ldc(&J->beta);
+  double* scale = ldc(&J->scale);
   const bool has_prev = j > 0;
   const V* up = has_prev ? slot_ptr<V>(vec, stride, cap, j - 1) : u;
-  const double cb = has_prev ? ldc(beta + j - 1) * ldc(scale + j - 1) : 0.0;
-  double* part = ldc(&J->part_up);
   // four consecutive rows per thread (slots are 256-byte aligned, chunks
   // start at multiples of kBatchChunk rows)
   const uint32_t i0 = it.idx * kBatchChunk + 4u * threadIdx.x;
+  const bool full = i0 + 4u <= D;
+  v4 wv, uv, pv;
+  if (full) {
+    wv = *reinterpret_cast<const v4*>(w + i0);
+    uv = *reinterpret_cast<const v4*>(u + i0);
+    pv = *reinterpret_cast<const v4*>(up + i0);
+  }
+  double sc, a, b = 0.0;
+  if (ldc(&J->fuse) != 0u) {  // uniform over the workgroup
+    double nsum = thread_partials(Partials{norm_part(J, j), ldc(&J->n_chunks)});
+    double hsum = thread_partials(Partials{ldc(&J->part_hv), ldc(&J->n_hv)});
+    update_sums<kBlock>(nsum, hsum);
+    const double nrm = sqrt(nsum);
+    sc = 1.0 / nrm;
+    a = sc * sc * hsum;
+    if (it.idx == 0u && threadIdx.x == 0u) {
+      alpha[j] = a;
+      ldc(&J->host_alpha)[j] = a;
+      if (t > 0 || j == 0) scale[j] = sc;  // the last launch of a group before stored it
+      if (t > 0 && has_prev) {
+        beta[j - 1] = nrm;
+        ldc(&J->host_beta)[j - 1] = nrm;
+      }
+    }
+    if (has_prev) b = nrm;
+  } else {
+    sc = ldc(scale + j);
+    a = ldc(alpha + j);
+    if (has_prev) b = ldc(beta + j - 1);
+  }
+  const double ca = a * sc;
+  double cb = 0.0;
+  if (has_prev) {
+    // scale_{j-1}: of the step before, which may be of this launch group
+    cb = b * scale[j - 1];
+  }
   double acc = 0.0;
-  if (i0 + 4u <= D) {
-    typedef V v4 __attribute__((ext_vector_type(4), aligned(sizeof(V))));
-    const v4 wv = *reinterpret_cast<const v4*>(w + i0);
-    const v4 uv = *reinterpret_cast<const v4*>(u + i0);
-    const v4 pv = has_prev ? *reinterpret_cast<const v4*>(up + i0) : uv;
+  if (full) {
     v4 o;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -118,17 +160,23 @@ __global__ __launch_bounds__(kBlock) void batch_update_kernel(const BatchJob* __
     }
   }
   const double s = block_sum_all(acc);
-  if (threadIdx.x == 0) part[it.idx] = s;
+  if (threadIdx.x == 0) norm_part(J, j + 1)[it.idx] = s;
 }
 
 __global__ __launch_bounds__(kBlock) void batch_finish_kernel(const BatchJob* __restrict__ jobs,
                                                               const uint32_t* __restrict__ job_list, int t,
                                                               int mode) {
   const BatchJob* J = jobs + ldc(job_list + blockIdx.x);
-  const int j = ldc(&J->j0) + t;
-  if (mode != kBatchStart && j >= ldc(&J->jmax)) return;
+  const int jmax = ldc(&J->jmax), j0 = ldc(&J->j0);
+  int j = j0 + t;
+  if (mode == kBatchLast) {  // t: the steps of the group
+    j = min(j, jmax) - 1;
+    if (j < j0) return;
+  } else if (mode != kBatchStart && j >= jmax) {
+    return;
+  }
   const bool hv = mode == kBatchAlpha;
-  const double* part = hv ? ldc(&J->part_hv) : ldc(&J->part_up);
+  const double* part = hv ? ldc(&J->part_hv) : norm_part(J, mode == kBatchStart ? 0 : j + 1);
   const uint32_t n = hv ? ldc(&J->n_hv) : ldc(&J->n_chunks);
   const double s = sum_partials(Partials{part, n});
   if (threadIdx.x != 0) return;
@@ -148,40 +196,90 @@ __global__ __launch_bounds__(kBlock) void batch_finish_kernel(const BatchJob* __
   }
 }
 
+// Rows r0 + 4 tid .. + 3 of NV Ritz vectors of a chunk, kRitzAhead basis
+// vectors in flight; their squares into acc2.
+template <class V, int NV>
+__device__ __forceinline__ void ritz_rows(const RitzJob* J, uint32_t r0, int nv, double (&acc2)[NV]) {
+  typedef V v4 __attribute__((ext_vector_type(4), aligned(sizeof(V))));
+  typedef double o4 __attribute__((ext_vector_type(4), aligned(8)));
+  constexpr int kRitzAhead = 8;
+  const V* vec = static_cast<const V*>(ldc(&J->vec));
+  const uint64_t stride = ldc(&J->stride);
+  const uint32_t D = ldc(&J->D);
+  const int m = ldc(&J->m);
+  const double* scale = ldc(&J->scale);
+  const double* coef = ldc(&J->coef);
+  double* out = ldc(&J->out);
+  const uint32_t r = r0 + 4u * threadIdx.x;
+  double acc[NV][4];
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[i][e] = 0.0;
+  auto add = [&](int j, const v4& u) {
+    const double sj = ldc(scale + j);
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      if (i < nv) {
+        const double c = ldc(coef + (size_t)i * m + j);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][e] += c * (sj * (double)u[e]);
+      }
+  };
+  if (r + 4u <= D) {
+    int j = 0;
+    for (; j + kRitzAhead <= m; j += kRitzAhead) {
+      v4 u[kRitzAhead];
+#pragma unroll
+      for (int c = 0; c < kRitzAhead; ++c) u[c] = *reinterpret_cast<const v4*>(vec + (uint64_t)(j + c) * stride + r);
+      issue_barrier();
+#pragma unroll
+      for (int c = 0; c < kRitzAhead; ++c) add(j + c, u[c]);
+    }
+    for (; j < m; ++j) add(j, *reinterpret_cast<const v4*>(vec + (uint64_t)j * stride + r));
+  } else if (r < D) {
+    for (int j = 0; j < m; ++j) {
+      v4 u = {(V)0, (V)0, (V)0, (V)0};
+      for (uint32_t e = 0; e < 3u; ++e)
+        if (r + e < D) u[e] = vec[(uint64_t)j * stride + r + e];
+      add(j, u);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    acc2[i] = 0.0;
+    if (i < nv && r < D) {
+      double* o = out + (uint64_t)i * D + r;
+      if (r + 4u <= D) *reinterpret_cast<o4*>(o) = o4{acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
+#pragma unroll
+      for (uint32_t e = 0; e < 4u; ++e)
+        if (r + e < D) {
+          if (r + 4u > D) o[e] = acc[i][e];
+          acc2[i] += acc[i][e] * acc[i][e];
+        }
+    }
+  }
+}
+
+// Bound by the read of the kept basis; with a handful of problems in a launch
+// by the rounds of dependent waits per row, of which four rows per thread and
+// eight vectors at a time leave one in 32: 130 -> 38 us for a tenth of 64
+// chains of 12 to 20 sites.
 template <class V>
 __global__ __launch_bounds__(kBlock) void batch_ritz_kernel(const RitzJob* __restrict__ jobs,
                                                             const BatchItem* __restrict__ items) {
   const BatchItem it = ldc_struct(items + blockIdx.x);
   const RitzJob* J = jobs + it.job;
-  const V* vec = static_cast<const V*>(ldc(&J->vec));
-  const uint64_t stride = ldc(&J->stride);
-  const uint32_t D = ldc(&J->D);
-  const int m = ldc(&J->m);
   const int nv = ldc(&J->nv);
-  const double* scale = ldc(&J->scale);
-  const double* coef = ldc(&J->coef);
-  const uint32_t r0 = it.idx * kBatchChunk;
-  const uint32_t r1 = min(D, r0 + kBatchChunk);
   double acc2[kMaxRitz];
 #pragma unroll
   for (int i = 0; i < kMaxRitz; ++i) acc2[i] = 0.0;
-  for (uint32_t r = r0 + threadIdx.x; r < r1; r += kBlock) {
-    double acc[kMaxRitz];
-#pragma unroll
-    for (int i = 0; i < kMaxRitz; ++i) acc[i] = 0.0;
-    for (int j = 0; j < m; ++j) {
-      const double u = ldc(scale + j) * (double)vec[(uint64_t)j * stride + r];
-#pragma unroll
-      for (int i = 0; i < kMaxRitz; ++i)
-        if (i < nv) acc[i] += ldc(coef + (size_t)i * m + j) * u;
-    }
-    double* out = ldc(&J->out);
-#pragma unroll
-    for (int i = 0; i < kMaxRitz; ++i)
-      if (i < nv) {
-        out[(uint64_t)i * D + r] = acc[i];
-        acc2[i] += acc[i] * acc[i];
-      }
+  if (nv == 1) {  // uniform
+    double one[1];
+    ritz_rows<V, 1>(J, it.idx * kBatchChunk, nv, one);
+    acc2[0] = one[0];
+  } else {
+    ritz_rows<V, kMaxRitz>(J, it.idx * kBatchChunk, nv, acc2);
   }
   double* part = ldc(&J->part);
   const uint32_t nc = ldc(&J->n_chunks);

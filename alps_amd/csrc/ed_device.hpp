@@ -206,6 +206,28 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Two sums over a workgroup of NT threads, to every thread, through LDS
+// barriers only: the vector elements read before stay in flight.  Once per
+// kernel.
+template <int NT>
+__device__ __forceinline__ void update_sums(double& a, double& b) {
+  __shared__ double red[2][NT / 64];
+  a = wave_sum(a);
+  b = wave_sum(b);
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = a;
+    red[1][threadIdx.x >> 6] = b;
+  }
+  lds_barrier();
+  a = 0.0;
+  b = 0.0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) {
+    a += red[0][w];
+    b += red[1][w];
+  }
+}
+
 // The workgroup's (NT threads) part of clearing the page of B low bits.
 template <int NT>
 __device__ __forceinline__ void clear_page(int B) {

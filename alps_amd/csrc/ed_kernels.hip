@@ -385,27 +385,6 @@ __global__ __launch_bounds__(kBlock) void reorth_update_kernel(uint64_t n, int j
   store_partial(norm_out, acc);
 }
 
-// Two sums over a workgroup of kUpdBlock threads, to every thread, through
-// LDS barriers only: the vector elements read before stay in flight.  Once
-// per kernel.
-__device__ __forceinline__ void update_sums(double& a, double& b) {
-  __shared__ double red[2][kUpdBlock / 64];
-  a = wave_sum(a);
-  b = wave_sum(b);
-  if ((threadIdx.x & 63) == 0) {
-    red[0][threadIdx.x >> 6] = a;
-    red[1][threadIdx.x >> 6] = b;
-  }
-  lds_barrier();
-  a = 0.0;
-  b = 0.0;
-#pragma unroll
-  for (int w = 0; w < kUpdBlock / 64; ++w) {
-    a += red[0][w];
-    b += red[1][w];
-  }
-}
-
 // A thread's share of two sums of partials in index order: the first ones are
 // read by the constructor, used by add().
 struct PartialPair {
@@ -479,7 +458,7 @@ __global__ __launch_bounds__(kUpdBlock) void update_fused_kernel(uint64_t n, con
   const double s_prev = !STEP && has_prev ? *S.scale_jm1 : 0.0;
   double nsum, hsum;
   pp.add(hv_part, norm_prev, hsum, nsum);
-  update_sums(nsum, hsum);
+  update_sums<kUpdBlock>(nsum, hsum);
   const double nrm = STEP ? 1.0 : sqrt(nsum);
   const double sc = STEP ? 1.0 : 1.0 / nrm;
   const double a = sc * sc * hsum;
@@ -582,7 +561,7 @@ __global__ __launch_bounds__(kUpdBlock) void normalize_kernel(uint64_t n, V* v, 
   issue_barrier();
   double ss, none;
   pp.add(norm_in, Partials{nullptr, 0}, ss, none);
-  update_sums(ss, none);
+  update_sums<kUpdBlock>(ss, none);
   const double inv = 1.0 / sqrt(ss);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     if (b_out) *b_out = sqrt(ss);
