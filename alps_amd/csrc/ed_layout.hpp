@@ -41,7 +41,6 @@ namespace alps_ed {
 
 constexpr int kMaxSites = 32;
 constexpr int kXcds = 8;  // accelerator complex dies of an MI355X
-constexpr int kClassSlices = 4;  // contiguous slices of a class swept in turn (uneven segment order)
 
 // Binomial coefficients C(n, k) for 0 <= n <= 64 (Pascal's triangle, built
 // once); 0 outside 0 <= k <= n.
@@ -512,36 +511,23 @@ inline SectorLayout build_layout(const ModelSpec& m, int B_override = -1, bool c
     if (!cls.empty()) L.max_seg = (uint32_t)binom(B, cls[0]);
   }
   // Workgroups are dealt to the 8 XCDs round-robin (block b runs on XCD
-  // b % 8), each XCD with its own L2.  When the segments split evenly by the
-  // top three bits of the high word, block b takes its segment from group
-  // b % 8: most high-high neighbours (hi ^ mask with the top bits unchanged)
-  // of a segment are then read on the XCD that owns them, from its L2.
-  bool grouped = false;
-  if (L.NH >= 3) {
-    std::vector<std::vector<uint32_t>> grp(kXcds);
-    for (uint32_t h : L.proc_hi) grp[h >> (L.NH - 3)].push_back(h);
-    bool even = true;
-    for (const auto& g : grp) even = even && g.size() == grp[0].size();
-    if (even && !grp[0].empty()) {
-      L.proc_hi.clear();
-      for (size_t i = 0; i < grp[0].size(); ++i)
-        for (int g = 0; g < kXcds; ++g) L.proc_hi.push_back(grp[g][i]);
-      grouped = true;
-    }
-  }
-  // Otherwise (popcount(hi) limited to a range narrower than 0..NH, so the
-  // top bits split the segments unevenly) a large sector is dealt class by
-  // class: each class, in address order, is cut into kXcds contiguous runs
-  // of equal count, and the position p of the order takes from run p % 8,
-  // i.e. XCD g sweeps run g of every class.  The high-high and cross
-  // neighbours of a segment (hi ^ mask, near hi in address when the flipped
-  // bits are low ones) are then read mostly on the XCD that reads hi.  Equal
-  // counts of one class are equal work, so the XCDs stay balanced.  A class
-  // is swept in kClassSlices contiguous slices one after the other, each
-  // dealt as eight runs, which keeps the x of the segments in flight (and of
-  // their neighbours) within a quarter of the class (J1-J2 6x5: 4.64 ->
-  // 4.51 ms; 2 slices 4.58, 8 slices 4.50).
-  if (!grouped && L.seg_hi.size() >= 64u * kXcds) {
+  // b % 8), each XCD with its own L2.  A large layout is dealt class by class,
+  // longest first: each class is cut into kXcds runs of equal count, ordered
+  // by the set bits among the high word's low five bits and then by address,
+  // and position p of the order takes from run p % 8, in ascending address.
+  // A bond inside the low five bits, or inside the others, leaves the run's
+  // key as it is and mostly leads to a segment that the same XCD reads at
+  // about the same time; equal counts of one class are equal work, so the
+  // XCDs stay balanced.  Against groups by the top three bits (24 sites) and
+  // four slices per class of runs in address order (the others): ring of 24
+  // sites FP32 14.6 -> 13.6 us, FP64 23.5 -> 21.1, 25 sites XXZ FP64 36.0 ->
+  // 34.5, 26 sites FP32 47.4 -> 45.6, 28-site J1-J2 672 -> 661 us (keys of
+  // four and eight bits within 4 % of that).  A class of more than kSliceClass
+  // segments keeps four slices in address order one after the other, so that
+  // the x of the segments in flight stays within a quarter of it: 30-site
+  // J1-J2 (48620 segments) 3.31 ms, 3.37 with the key; 28 sites (12870) 664
+  // and 661 us.
+  if (L.seg_hi.size() >= 64u * kXcds) {
     std::vector<int> cls_order;
     std::vector<std::vector<uint32_t>> by_pc(L.NH + 1);
     for (uint32_t h : L.proc_hi) {
@@ -550,18 +536,36 @@ inline SectorLayout build_layout(const ModelSpec& m, int B_override = -1, bool c
       by_pc[c].push_back(h);
     }
     L.proc_hi.clear();
+    constexpr size_t kSliceClass = 16384;
     for (int c : cls_order) {
       std::vector<uint32_t>& v = by_pc[c];
-      if (!std::is_sorted(v.begin(), v.end())) std::sort(v.begin(), v.end());  // address order: hi_base ascends with hi
-      // kClassSlices contiguous slices in turn, each dealt as eight runs
-      const size_t slice = (v.size() + kClassSlices - 1) / kClassSlices;
-      for (size_t s0 = 0; s0 < v.size(); s0 += slice) {
-        const size_t n = std::min(slice, v.size() - s0);
-        const size_t base = n / kXcds, s = L.proc_hi.size();
-        for (size_t i = 0; i < base; ++i)
-          for (int j = 0; j < kXcds; ++j) L.proc_hi.push_back(v[s0 + ((s + j) % kXcds) * base + i]);
-        for (size_t r = base * kXcds; r < n; ++r) L.proc_hi.push_back(v[s0 + r]);
+      size_t slice = (v.size() + 3) / 4;
+      if (v.size() <= kSliceClass) {
+        slice = v.size();
+        std::vector<uint32_t> w[6];
+        for (uint32_t h : v) w[__builtin_popcount(h & 31u)].push_back(h);
+        v.clear();
+        for (auto& k : w) v.insert(v.end(), k.begin(), k.end());
       }
+      for (size_t s0 = 0; s0 < v.size(); s0 += slice) {
+        const auto q = v.begin() + s0;
+        const size_t n = std::min(slice, v.size() - s0), run = n / kXcds, s = L.proc_hi.size();
+        for (int g = 0; g < kXcds; ++g) std::sort(q + g * run, q + (g + 1) * run);
+        for (size_t i = 0; i < run; ++i)
+          for (int j = 0; j < kXcds; ++j) L.proc_hi.push_back(q[((s + j) % kXcds) * run + i]);
+        L.proc_hi.insert(L.proc_hi.end(), q + kXcds * run, q + n);
+      }
+    }
+  } else if (L.NH >= 3) {
+    // few segments: groups by the top three bits where these split them evenly
+    std::vector<std::vector<uint32_t>> grp(kXcds);
+    for (uint32_t h : L.proc_hi) grp[h >> (L.NH - 3)].push_back(h);
+    bool even = true;
+    for (const auto& g : grp) even = even && g.size() == grp[0].size();
+    if (even && !grp[0].empty()) {
+      L.proc_hi.clear();
+      for (size_t i = 0; i < grp[0].size(); ++i)
+        for (int g = 0; g < kXcds; ++g) L.proc_hi.push_back(grp[g][i]);
     }
   }
   // terms in bit coordinates
