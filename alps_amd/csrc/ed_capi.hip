@@ -304,6 +304,11 @@ void operator_upload(alps_ed_operator op) {
   ALPS_ED_UP(diag_lo_cls)
   ALPS_ED_UP(diag_hi)
   ALPS_ED_UP(ll_c)
+  if (L.ranked && !L.nbp16.empty()) {
+    ALPS_ED_UP(nbp16)
+    ALPS_ED_UP(nbp_off)
+    d.n_ll_p = L.n_ll_p;
+  }
   pk.add(L.flip->xn16, &d.xn16);
   ALPS_ED_UP(xn_off)
   ALPS_ED_UP(xb_c)

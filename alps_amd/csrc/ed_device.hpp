@@ -596,6 +596,225 @@ __device__ __forceinline__ void hv_segment_at(const DevLayout& L, const SegRec& 
   }
 }
 
+// H.v over a segment with the low-low targets from tables (nbp16, one LDS
+// byte offset per row and bond, the zero slot where the bits are parallel) and
+// the slice of x in LDS by rank: nothing to clear and one barrier, at one more
+// load per four low-low bonds.  It is the faster one where segments are short
+// on average (ranked_rows, ed_layout.hpp), where the fixed part of a segment
+// in hv_rows outweighs its rows.
+template <class V, bool DOT, int NQ, int CLL, int CHH, int CX>
+__device__ __forceinline__ double hv_ranked_rows(const DevLayout& L, const SegRec& S, const V* __restrict__ x,
+                                                 V* __restrict__ y) {
+  const uint32_t h = S.h, len = S.len, base = S.base, e0 = S.e0, e1 = S.e1;
+  const double dh = S.dh;
+  const uint16_t* nbp = L.nbp16 + S.nbp;
+  const uint16_t* xnp = L.xn16 + S.xnp;
+  const double* dlp = L.diag_lo_cls + S.cls0;
+  constexpr uint32_t VS = (uint32_t)sizeof(V);
+  constexpr int QL = NQ - 1;  // the last slot
+  const uint32_t tid = threadIdx.x;
+  const V* xb = x + base;
+  static_assert(CLL % kLLChunk == 0 && CX % kXChunk == 0, "schedule chunks are multiples of the table chunks");
+  typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  const uint32_t rl = tid + QL * kBlock;
+  const bool okl = rl < len;
+  const uint32_t vo0 = lane_off(VS * tid);               // slot 0 (and every full slot)
+  const uint32_t vol = lane_off(okl ? VS * rl : 0u);     // the last slot, clamped
+  // flip-table records (flip_index, ed_layout.hpp): bond chunk k of row r
+  // starts at rec(r) + k * 64 * chunk
+  const uint32_t lo_ll = lane_off(2u * ((tid >> 6) * 64u * (uint32_t)L.n_ll_p + (tid & 63u) * kLLChunk));
+  const uint32_t lo_x = lane_off(2u * ((tid >> 6) * 64u * (uint32_t)L.n_xb_p + (tid & 63u) * kXChunk));
+  const uint32_t ll_slot = (uint32_t)kBlock * (uint32_t)L.n_ll_p;  // u16 entries per slot
+  const uint32_t x_slot = (uint32_t)kBlock * (uint32_t)L.n_xb_p;
+  // element of slot q of the segment starting at p
+  auto seg_ld = [&](const V* p, int q) -> V {
+    return q < QL ? ld_at<V>(p + q * kBlock, vo0) : ld_at<V>(p, vol);
+  };
+  V xo[NQ];
+  double d[NQ], off[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    xo[q] = seg_ld(xb, q);
+    d[q] = dh + (q < QL ? ld_at<double>(dlp + q * kBlock, vo0 * (8u / VS)) : ld_at<double>(dlp, vol * (8u / VS)));
+    off[q] = 0.0;
+  }
+  // The cross-bond table entries of the first chunk are loaded now, so that
+  // they arrive while the other bonds are processed.
+  const int n_xb = (L.n_xb + CX - 1) / CX * CX;
+  constexpr int KX = CX / kXChunk;
+  u16x2 xr[NQ][KX];
+  if (n_xb > 0) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int k = 0; k < KX; ++k) xr[q][k] = ld_at<u16x2>(xnp + q * x_slot + k * kXChunk * 64u, lo_x);
+  }
+  // low-low flips: target rows from the class table, values from LDS.  The
+  // table entries of chunk b + CLL are loaded while chunk b is processed,
+  // into the other of two register sets (ta, tb).
+  const int n_ll = (L.n_ll + CLL - 1) / CLL * CLL;
+  constexpr int KL = CLL / kLLChunk;
+  u16x4 ta[NQ][KL], tb[NQ][KL];
+  auto ll_load = [&](u16x4(&t)[NQ][KL], int b) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int k = 0; k < KL; ++k)
+        t[q][k] = ld_at<u16x4>(nbp + q * ll_slot + (uint32_t)(b + k * kLLChunk) * 64u, lo_ll);
+  };
+  auto ll_apply = [&](const u16x4(&t)[NQ][KL], int b) {
+    double tc[CLL];
+#pragma unroll
+    for (int c = 0; c < CLL; ++c) tc[c] = ldc(&L.ll_c[b + c].t);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int c = 0; c < CLL; ++c) {
+        const uint32_t j = t[q][c / kLLChunk][c % kLLChunk];
+        off[q] = fma(tc[c], lds_ld<double>(j), off[q]);
+      }
+  };
+  if (n_ll > 0) ll_load(ta, 0);
+  // The segment's slice of x into LDS: each thread stores its own rows (the
+  // rows of the segment are exactly the rows of the threads' slots), with
+  // the table loads above already in flight; then the barrier that every
+  // wave of the workgroup passes once (hv_ranked_at).
+#pragma unroll
+  for (int q = 0; q < QL; ++q) lds_st<double>(8u * (tid + q * kBlock), (double)xo[q]);
+  if (okl) lds_st<double>(8u * rl, (double)xo[QL]);
+  if (tid == 0) lds_st<double>(8u * len, 0.0);
+  lds_barrier();
+  for (int b0 = 0; b0 < n_ll; b0 += 2 * CLL) {
+    if (b0 + CLL < n_ll) ll_load(tb, b0 + CLL);
+    ll_apply(ta, b0);
+    if (b0 + CLL >= n_ll) break;
+    if (b0 + 2 * CLL < n_ll) ll_load(ta, b0 + 2 * CLL);
+    ll_apply(tb, b0 + CLL);
+  }
+  // high-high flips: a bond flips every row of the segment or none (its two
+  // bits lie in h), with a contiguous target run.  The bonds that flip h are
+  // listed per high word in bond order (hh_off / hh_ent), padded with
+  // weight-0 reads of this segment; slots of a chunk past the list do the
+  // same.  Bonds that do not flip would add exact zeros, so the sums are
+  // those over all bonds.
+  {
+    for (uint32_t e = e0; e < e1; e += CHH) {
+      // neighbour segment starts as element offsets (a select between
+      // pointers would make the loads generic-address ones)
+      uint32_t xt[CHH];
+      double tt[CHH];
+#pragma unroll
+      for (int c = 0; c < CHH; ++c) {
+        if (c < kHHList || e + c < e1) {
+          const HHEntry en = ldc_struct(L.hh_ent + e + c);
+          xt[c] = en.nb;
+          tt[c] = en.t;
+        } else {
+          xt[c] = base;
+          tt[c] = 0.0;
+        }
+      }
+      V v[NQ][CHH];
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+#pragma unroll
+        for (int c = 0; c < CHH; ++c) v[q][c] = seg_ld(x + xt[c], q);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+#pragma unroll
+        for (int c = 0; c < CHH; ++c) off[q] = fma(tt[c], (double)v[q][c], off[q]);
+    }
+  }
+  // cross bonds: diagonal always, flip when the high and low bits differ
+  // (bit 15 of the table entry is the row's low bit).  Where the
+  // neighbouring high word has no segment no row can flip (its low word
+  // would need a set bit more or fewer than it has), and xb_nb points to this
+  // segment.  The diagonal already holds every cross bond's parallel value
+  // (diag_hi); each antiparallel bond adds its anti - par difference.
+  const uint32_t* xnb = L.xb_nb + h * (uint32_t)L.n_xb_p;
+  for (int b0 = 0; b0 < n_xb; b0 += CX) {
+    uint32_t xt[CX], hx[CX];
+    double de[CX], tx[CX];
+#pragma unroll
+    for (int c = 0; c < CX; ++c) {
+      const XBondConst k = ldc_struct(L.xb_c + b0 + c);
+      hx[c] = (h & k.hbit) != 0u ? 0x8000u : 0u;
+      xt[c] = ldc(xnb + b0 + c);
+      de[c] = k.de;
+      tx[c] = k.t;
+    }
+    uint32_t e[NQ][CX];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int k = 0; k < KX; ++k)
+#pragma unroll
+        for (int c = 0; c < kXChunk; ++c) e[q][k * kXChunk + c] = xr[q][k][c];
+    if (b0 + CX < n_xb) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+#pragma unroll
+        for (int k = 0; k < KX; ++k)
+          xr[q][k] = ld_at<u16x2>(xnp + q * x_slot + (uint32_t)(b0 + CX + k * kXChunk) * 64u, lo_x);
+    }
+    V v[NQ][CX];
+    bool f[NQ][CX];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int c = 0; c < CX; ++c) {
+        f[q][c] = ((e[q][c] ^ hx[c]) & 0x8000u) != 0u;
+        v[q][c] = ld_lane<V>(x + xt[c], f[q][c] ? (e[q][c] & 0x7fffu) * (VS / 4u) : 0u);
+      }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int c = 0; c < CX; ++c) {
+        // the flag as 1.0 / 0.0 and the value selected in the storage type
+        // (one 32-bit select each; the asm keeps the select before the
+        // conversion, where selecting the FP64 value takes two)
+        V w = f[q][c] ? v[q][c] : (V)0;
+        asm volatile("" : "+v"(w));
+        d[q] = fma(f[q][c] ? 1.0 : 0.0, de[c], d[q]);
+        off[q] = fma(tx[c], (double)w, off[q]);
+      }
+  }
+  double dotp = 0.0;
+  V* yb = y + base;
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    if (q < QL || okl) {
+      const double xi = (double)xo[q];
+      const double yv = fma(d[q], xi, off[q]);
+      if (q < QL) st_at<V>(yb + q * kBlock, vo0, (V)yv);
+      else st_at<V>(yb, vol, (V)yv);
+      if (DOT) dotp = fma(xi, yv, dotp);  // FP64 value before the storage rounding
+    }
+  }
+  return dotp;
+}
+
+// The same workgroup and slots as hv_segment_at; dynamic LDS of max_seg + 1
+// doubles.
+template <class V, bool DOT, int CLL = 4, int CHH = 4, int CX = 2>
+__device__ __forceinline__ void hv_ranked_at(const DevLayout& L, const SegRec& S, const V* __restrict__ x,
+                                             V* __restrict__ y, double* __restrict__ dot_slot) {
+  const uint32_t w0 = threadIdx.x & ~63u;
+  const uint32_t nq = __builtin_amdgcn_readfirstlane(S.len > w0 ? (S.len - w0 + kBlock - 1) / kBlock : 0u);
+  static_assert(kMaxSegRows == 4 * kBlock, "one to four row slots");
+  double dotp = 0.0;
+  if (nq == 0) lds_barrier();
+  else if (nq == 1) dotp = hv_ranked_rows<V, DOT, 1, CLL, CHH, CX>(L, S, x, y);
+  else if (nq == 2) dotp = hv_ranked_rows<V, DOT, 2, CLL, CHH, CX>(L, S, x, y);
+  else if (nq == 3) dotp = hv_ranked_rows<V, DOT, 3, CLL, CHH, CX>(L, S, x, y);
+  else dotp = hv_ranked_rows<V, DOT, 4, CLL, CHH, CX>(L, S, x, y);
+  if (DOT) {
+    lds_barrier();  // every wave is done with the slice
+    store_block_sum_lds<kBlock>(dot_slot, dotp);
+  }
+}
+
 // The record of the segment of high word h, looked up in the tables.
 __device__ __forceinline__ SegRec seg_record(const DevLayout& L, uint32_t h) {
   const int kl = L.k - __builtin_popcount(h);
@@ -611,7 +830,7 @@ __device__ __forceinline__ SegRec seg_record(const DevLayout& L, uint32_t h) {
   S.e0 = ldc(L.hh_off + h);
   S.e1 = ldc(L.hh_off + h + 1);
   S.xnp = ldc(L.xn_off + kl);
-  S.pad = 0u;
+  S.nbp = L.nbp16 ? ldc(L.nbp_off + kl) : 0u;
   S.dh = ldc(L.diag_hi + h);
   S.pad2 = 0.0;
   return S;

@@ -23,6 +23,8 @@
 // consumers add the partials in index order.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "ed_device.hpp"
 #include "ed_kernels.hpp"
 
@@ -40,6 +42,13 @@ __global__ __launch_bounds__(NT, W) void hv_kernel(DevLayout L, const V* __restr
                                                    double* __restrict__ dot_out) {
   hv_segment_at<V, DOT, STAGE, NT, CLL, CHH>(L, ldc_struct(L.seg_rec + blockIdx.x), x, y,
                                              DOT ? dot_out + blockIdx.x : nullptr);
+}
+
+template <class V, bool DOT>
+__global__ __launch_bounds__(kBlock, HvWaves<V>::value) void hv_ranked_kernel(DevLayout L, const V* __restrict__ x,
+                                                                             V* __restrict__ y,
+                                                                             double* __restrict__ dot_out) {
+  hv_ranked_at<V, DOT>(L, ldc_struct(L.seg_rec + blockIdx.x), x, y, DOT ? dot_out + blockIdx.x : nullptr);
 }
 
 // seg_rec[i] for processing index i (the record hv_segment would look up).
@@ -79,6 +88,11 @@ void launch_hv_schedule(const DevLayout& L, const V* x, V* y, double* dot_out, h
 
 template <class V, bool DOT>
 void launch_hv_stage(const DevLayout& L, const V* x, V* y, double* dot_out, hipStream_t st, int schedule) {
+  if (L.nbp16 != nullptr) {  // one schedule
+    const size_t lds = std::max<size_t>(kHvMinLds, (L.max_seg + 1) * sizeof(double));
+    hipLaunchKernelGGL((hv_ranked_kernel<V, DOT>), dim3(hv_blocks(L)), dim3(kBlock), lds, st, L, x, y, dot_out);
+    return;
+  }
   if (L.n_xs > 0) launch_hv_schedule<V, DOT, true>(L, x, y, dot_out, st, schedule);
   else launch_hv_schedule<V, DOT, false>(L, x, y, dot_out, st, schedule);
 }

@@ -31,6 +31,10 @@ struct DevLayout {
   const PageBond* ll_c;       // [n_ll] low-low bonds
   const uint32_t* hh_off;     // [2^NH + 1] per high word: its flipping high-high bonds
   const HHEntry* hh_ent;      //   (neighbour segment, coefficient), padded with 0-coefficient entries
+  // low-low target tables (null: hv_segment_at)
+  const uint16_t* nbp16;
+  const uint32_t* nbp_off;
+  int n_ll_p;
   // gathered cross bonds
   const uint16_t* xn16;
   const uint32_t* xn_off;

@@ -157,7 +157,7 @@ struct PageBond {
 // table reads.
 struct SegRec {
   uint32_t h, base, cls0, len;
-  uint32_t e0, e1, xnp, pad;
+  uint32_t e0, e1, xnp, nbp;
   uint32_t cls_up, len_up, cls_dn, len_dn;
   double dh, pad2;
 };
@@ -204,6 +204,7 @@ struct SectorLayout {
   int n_ll_p = 0, n_hh_p = 0, n_xb_p = 0;
   std::vector<uint16_t> nbp16, xn16;
   std::vector<uint32_t> nbp_off, xn_off;  // [B+2]
+  bool ranked = false;                    // ranked_rows
   std::vector<PageBond> ll_c;
   bool stage = false;                     // cross bonds staged, not gathered
   // The high-high bonds that flip the rows of high word h (the two bits of
@@ -370,6 +371,19 @@ inline std::shared_ptr<const FlipTables> flip_tables(int B, const std::vector<ui
 // and 4.38 us, 21 sites 5.82 and 5.36, 20-site J1-J2 13.4 and 10.4; above the
 // line 22 sites 8.23 and 8.28, 23 sites 13.4 and 15.3).
 constexpr size_t kFewSegments = 512;
+
+// Whether single operators take the kernel with low-low target tables
+// (hv_ranked_at, ed_device.hpp): where the segments are short on average, away
+// from half filling.  Xor page and tables, us: rows a segment 168 (27 sites, 9
+// up, FP32) 49.7 and 44.8, 193 (24-site J1-J2, 8 up) 24.3 and 20.5, FP64 37.3
+// and 30.1, 247 (23 sites, 8 up) 5.4 and 5.2, 325 (24-site J1-J2, 15 up) 31.6
+// and 30.1; 333 (26 sites, 10 up) 35.0 and 35.6, 405 (27-site J1-J2, 11 up)
+// 245 and 252.  Up to 1024 segments (half of the workgroups that are resident)
+// the fixed part weighs more: 486 rows (22 sites, 9 up) 5.25 and 5.05, and 631
+// 5.5 and 5.6; up to kFewSegments the larger workgroups hide it.
+inline bool ranked_rows(int B, uint64_t D, size_t n_seg) {
+  return B == 12 && n_seg > kFewSegments && D < (n_seg <= 1024 ? 500u : 330u) * (uint64_t)n_seg;
+}
 
 // Whether the cross bonds are staged in LDS (hv_rows, ed_device.hpp): where a
 // high bit has two or more of them on average, so that a staged segment
@@ -654,21 +668,23 @@ inline SectorLayout build_layout(const ModelSpec& m, int B_override = -1, bool c
     L.xn_off = L.flip->xn_off;
     if (copy_shared) L.xn16 = L.flip->xn16;
   }
-  if (copy_shared) {
+  L.ranked = ranked_rows(B, L.D, L.seg_hi.size());
+  if (copy_shared || (L.ranked && !host_lists)) {
     L.nbp_off = flip_offsets(B, L.n_ll_p);
     L.nbp16.assign(L.nbp_off[B + 1], 0);
     for (int c = 0; c <= B; ++c) {
       const uint32_t len = (uint32_t)binom(B, c);
       for (int b = 0; b < L.n_ll_p; ++b)
         for (uint32_t r = 0; r < len; ++r) {
-          const uint32_t lo = L.lo_state[L.lo_class_off[c] + r];
+          const uint32_t lo = L.low->lo_state[L.lo_class_off[c] + r];
           const uint32_t m = b < (int)L.ll.size() ? L.ll[b].mask : 0u, bits = lo & m;
           L.nbp16[L.nbp_off[c] + flip_index(r, b, L.n_ll_p, kLLChunk)] =
-              (uint16_t)(8u * ((bits != 0u && bits != m) ? L.lo_rank[lo ^ m] : len));
+              (uint16_t)(8u * ((bits != 0u && bits != m) ? L.low->lo_rank[lo ^ m] : len));
         }
     }
   }
   for (const FlipBond& f : L.ll) L.ll_c.push_back(PageBond{f.t, 8u * page_pos(f.mask), 0u});
+  L.ll_c.resize(L.n_ll_p, PageBond{0.0, 0u, 0u});
   L.hh_mask.assign(L.hh.size(), 0u);
   L.hh_t.assign(L.hh.size(), 0.0);
   for (size_t q = 0; q < L.hh.size(); ++q) {
@@ -736,7 +752,7 @@ inline SectorLayout build_layout(const ModelSpec& m, int B_override = -1, bool c
     w[__builtin_ctz(x.lbit)] += x.e_anti - x.e_par;
     w[B] += x.e_anti - x.e_par;
   }
-  L.stage = stage_cross(B, L.xb.size(), L.xb_grp.size());
+  L.stage = !L.ranked && stage_cross(B, L.xb.size(), L.xb_grp.size());
   if (host_lists && L.stage) {
     const XSource X{L.xb_grp.data(), L.xb_w.data(), (int)L.xb_grp.size(), B};
     L.xs.assign((size_t)nhi * L.xb_grp.size(), XStage{0u, 0u});

@@ -1,8 +1,9 @@
 """H.v at the edges of its kernel paths, against the CPU oracle: staged and
 gathered cross bonds on both sides of the rule that picks one (stage_cross,
 ed_layout.hpp), the 512-thread workgroups of layouts with few segments and the
-256-thread ones above them, segments from one row to the longest class, low
-words shorter than 12 bits.
+256-thread ones above them, segments from one row to the longest class (at
+most 64 rows: one wave), sectors on both sides of ranked_rows (the rows per
+segment from which on the xor page is used), low words shorter than 12 bits.
 
 Tolerances: a row adds at most 64 terms |t x| <= 1 (and its diagonal, at most
 64 terms) in FP64: at most 64 u * 64 = 4.5e-13 against entries whose norm is
@@ -51,6 +52,8 @@ CASES = {
     "one_high_bit": (lambda: random_bonds(13, 12, 1, 5), [6, 0, 1, 12, 13]),
     "ring20": (lambda: O.lattice_model("chain lattice", 20), [10, 2, 18]),
     "ring21": (lambda: O.lattice_model("chain lattice", 21), [10]),
+    "short_segments_25": (lambda: random_bonds(25, 9, 9, 10), [4, 5, 22]),
+    "short_staged_25": (lambda: random_bonds(25, 24, 8, 11), [4, 21]),
     "ring22": (lambda: O.lattice_model("chain lattice", 22), [11, 3]),
     "lattice_4x3": (lambda: lattice(4, 3, 6), [6, 3]),
     "lattice_7x3": (lambda: lattice(7, 3, 7), [10, 20]),
@@ -63,9 +66,9 @@ def test_hv_paths_vs_oracle(name, k):
     say("case", name, k)
     m = CASES[name][0]()
     op = A.Operator(to_product(m, k))
-    x = np.random.default_rng(k).uniform(-1, 1, op.dim)
+    # values that FP32 holds, so that one product of the oracle serves both
+    x = np.random.default_rng(k).uniform(-1, 1, op.dim).astype(np.float32).astype(np.float64)
+    want = O.spmv(m, k, x)
     for dtype, tol in (("f64", 1e-13), ("f32", 2e-6)):
-        v = A.Vector.from_numpy(x, dtype)
-        want = O.spmv(m, k, v.numpy())
-        got = op.matvec(v, A.Vector(op.dim, dtype)).numpy()
+        got = op.matvec(A.Vector.from_numpy(x, dtype), A.Vector(op.dim, dtype)).numpy()
         assert np.linalg.norm(got - want) <= tol * max(np.linalg.norm(want), 1e-300)
