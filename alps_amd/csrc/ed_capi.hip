@@ -307,6 +307,7 @@ void operator_upload(alps_ed_operator op) {
   if (L.ranked && !L.nbp16.empty()) {
     ALPS_ED_UP(nbp16)
     ALPS_ED_UP(nbp_off)
+    ALPS_ED_UP(ll_t)
     d.n_ll_p = L.n_ll_p;
   }
   pk.add(L.flip->xn16, &d.xn16);

@@ -601,9 +601,16 @@ __device__ __forceinline__ void hv_segment_at(const DevLayout& L, const SegRec& 
 // the slice of x in LDS by rank: nothing to clear and one barrier, at one more
 // load per four low-low bonds.  It is the faster one where segments are short
 // on average (ranked_rows, ed_layout.hpp), where the fixed part of a segment
-// in hv_rows outweighs its rows.
+// in hv_rows outweighs its rows.  Bound by the chain of dependent loads of a
+// segment, so by the waves in flight and by scalar loads: a row's own element
+// is read from LDS again at the end rather than kept (FP64: 64 registers, 8
+// waves per SIMD instead of 7), the coefficients are contiguous and only the
+// first 40 bytes of the record are read: 24 sites 8 up 7.84 -> 7.52 us (FP32)
+// and 10.68 -> 10.46 (FP64), 22 sites 7 up 4.23 -> 4.14 and 4.68 -> 4.55, 23
+// sites 7 up 4.69 -> 4.54 and 5.44 -> 5.30, 27-site J1-J2 9 up 132.5 -> 130.6
+// and 181.3 -> 180.2.
 template <class V, bool DOT, int NQ, int CLL, int CHH, int CX>
-__device__ __forceinline__ double hv_ranked_rows(const DevLayout& L, const SegRec& S, const V* __restrict__ x,
+__device__ __forceinline__ double hv_ranked_rows(const DevLayout& L, const SegHead& S, const V* __restrict__ x,
                                                  V* __restrict__ y) {
   const uint32_t h = S.h, len = S.len, base = S.base, e0 = S.e0, e1 = S.e1;
   const double dh = S.dh;
@@ -666,7 +673,7 @@ __device__ __forceinline__ double hv_ranked_rows(const DevLayout& L, const SegRe
   auto ll_apply = [&](const u16x4(&t)[NQ][KL], int b) {
     double tc[CLL];
 #pragma unroll
-    for (int c = 0; c < CLL; ++c) tc[c] = ldc(&L.ll_c[b + c].t);
+    for (int c = 0; c < CLL; ++c) tc[c] = ldc(L.ll_t + b + c);
 #pragma unroll
     for (int q = 0; q < NQ; ++q)
 #pragma unroll
@@ -785,7 +792,7 @@ __device__ __forceinline__ double hv_ranked_rows(const DevLayout& L, const SegRe
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
     if (q < QL || okl) {
-      const double xi = (double)xo[q];
+      const double xi = lds_ld<double>(8u * (q < QL ? tid + q * kBlock : rl));
       const double yv = fma(d[q], xi, off[q]);
       if (q < QL) st_at<V>(yb + q * kBlock, vo0, (V)yv);
       else st_at<V>(yb, vol, (V)yv);
@@ -798,7 +805,7 @@ __device__ __forceinline__ double hv_ranked_rows(const DevLayout& L, const SegRe
 // The same workgroup and slots as hv_segment_at; dynamic LDS of max_seg + 1
 // doubles.
 template <class V, bool DOT, int CLL = 4, int CHH = 4, int CX = 2>
-__device__ __forceinline__ void hv_ranked_at(const DevLayout& L, const SegRec& S, const V* __restrict__ x,
+__device__ __forceinline__ void hv_ranked_at(const DevLayout& L, const SegHead& S, const V* __restrict__ x,
                                              V* __restrict__ y, double* __restrict__ dot_slot) {
   const uint32_t w0 = threadIdx.x & ~63u;
   const uint32_t nq = __builtin_amdgcn_readfirstlane(S.len > w0 ? (S.len - w0 + kBlock - 1) / kBlock : 0u);
@@ -832,7 +839,7 @@ __device__ __forceinline__ SegRec seg_record(const DevLayout& L, uint32_t h) {
   S.xnp = ldc(L.xn_off + kl);
   S.nbp = L.nbp16 ? ldc(L.nbp_off + kl) : 0u;
   S.dh = ldc(L.diag_hi + h);
-  S.pad2 = 0.0;
+  S.pad = 0.0;
   return S;
 }
 

@@ -48,7 +48,7 @@ template <class V, bool DOT>
 __global__ __launch_bounds__(kBlock, HvWaves<V>::value) void hv_ranked_kernel(DevLayout L, const V* __restrict__ x,
                                                                              V* __restrict__ y,
                                                                              double* __restrict__ dot_out) {
-  hv_ranked_at<V, DOT>(L, ldc_struct(L.seg_rec + blockIdx.x), x, y, DOT ? dot_out + blockIdx.x : nullptr);
+  hv_ranked_at<V, DOT>(L, ldc_struct<SegHead>(L.seg_rec + blockIdx.x), x, y, DOT ? dot_out + blockIdx.x : nullptr);
 }
 
 // seg_rec[i] for processing index i (the record hv_segment would look up).

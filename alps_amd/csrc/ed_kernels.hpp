@@ -15,7 +15,8 @@ struct DevLayout {
   uint32_t D;
   uint32_t n_seg, max_seg;
   int n_bonds;
-  int n_ll, n_xb, n_xb_p;     // low-low and cross flip bonds; the cross tables' stride
+  int n_ll, n_xb;             // low-low and cross flip bonds
+  int n_ll_p, n_xb_p;         // entries per row of their tables
   int n_xs;                   // high bits with staged cross bonds; 0: gathered
   const uint32_t* lo_rank;
   const uint32_t* lo_state;
@@ -31,10 +32,10 @@ struct DevLayout {
   const PageBond* ll_c;       // [n_ll] low-low bonds
   const uint32_t* hh_off;     // [2^NH + 1] per high word: its flipping high-high bonds
   const HHEntry* hh_ent;      //   (neighbour segment, coefficient), padded with 0-coefficient entries
-  // low-low target tables (null: hv_segment_at)
+  // low-low target tables (null: hv_segment_at) and coefficients [n_ll_p]
   const uint16_t* nbp16;
   const uint32_t* nbp_off;
-  int n_ll_p;
+  const double* ll_t;
   // gathered cross bonds
   const uint16_t* xn16;
   const uint32_t* xn_off;

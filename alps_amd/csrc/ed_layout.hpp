@@ -150,18 +150,21 @@ struct PageBond {
 
 // What the H.v kernel needs of the segment it processes, one record per
 // processing index (built on the device for a single operator): its high
-// word, first row, class offset and length, the flip-table offset, those of the
-// classes with one low bit more and one fewer (the segments across a cross
-// bond), the range of its listed high-high flips and the high word's
-// diagonal.  Read with one scalar load instead of two dependent rounds of
-// table reads.
-struct SegRec {
+// word, first row, class offset and length, the range of its listed high-high
+// flips, the flip-table offsets, the high word's diagonal, and the offset and
+// length of the classes with one low bit more and one fewer (the segments
+// across a cross bond; only the staged bonds need them).  Read with scalar
+// loads instead of two dependent rounds of table reads.
+struct SegHead {
   uint32_t h, base, cls0, len;
   uint32_t e0, e1, xnp, nbp;
-  uint32_t cls_up, len_up, cls_dn, len_dn;
-  double dh, pad2;
+  double dh;
 };
-static_assert(sizeof(SegRec) == 64, "one 64-byte scalar load");
+struct SegRec : SegHead {
+  uint32_t cls_up, len_up, cls_dn, len_dn;
+  double pad;
+};
+static_assert(sizeof(SegRec) == 64, "one scalar load of 16 registers");
 
 struct SectorLayout {
   int N = 0, k = 0, B = 0, NH = 0;
@@ -206,6 +209,7 @@ struct SectorLayout {
   std::vector<uint32_t> nbp_off, xn_off;  // [B+2]
   bool ranked = false;                    // ranked_rows
   std::vector<PageBond> ll_c;
+  std::vector<double> ll_t;               // [n_ll_p]
   bool stage = false;                     // cross bonds staged, not gathered
   // The high-high bonds that flip the rows of high word h (the two bits of
   // h & mask differ), in bond order: entries [hh_off[h], hh_off[h+1]) of
@@ -685,6 +689,7 @@ inline SectorLayout build_layout(const ModelSpec& m, int B_override = -1, bool c
   }
   for (const FlipBond& f : L.ll) L.ll_c.push_back(PageBond{f.t, 8u * page_pos(f.mask), 0u});
   L.ll_c.resize(L.n_ll_p, PageBond{0.0, 0u, 0u});
+  for (const PageBond& c : L.ll_c) L.ll_t.push_back(c.t);
   L.hh_mask.assign(L.hh.size(), 0u);
   L.hh_t.assign(L.hh.size(), 0.0);
   for (size_t q = 0; q < L.hh.size(); ++q) {

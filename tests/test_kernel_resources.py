@@ -1,0 +1,53 @@
+"""What the compiled kernels take of a compute unit, read from the metadata of
+the gfx950 code objects in the engine library (no device)."""
+import os
+import re
+import struct
+
+import msgpack
+
+import alps_amd as A
+
+MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
+
+
+def kernels():
+    """Metadata of every gfx950 kernel: name -> dict."""
+    with open(A.LIB_PATH, "rb") as f:
+        d = f.read()
+    out = {}
+    at = d.find(MAGIC)
+    while at >= 0:
+        (n,) = struct.unpack_from("<Q", d, at + 24)
+        p = at + 32
+        for _ in range(n):
+            off, size, tl = struct.unpack_from("<QQQ", d, p)
+            triple = d[p + 24:p + 24 + tl].decode()
+            p += 24 + tl
+            if "gfx950" in triple and size:
+                out.update(metadata(d[at + off:at + off + size]))
+        at = d.find(MAGIC, at + 1)
+    return out
+
+
+def metadata(elf):
+    (shoff,) = struct.unpack_from("<Q", elf, 40)
+    shsize, shnum = struct.unpack_from("<HH", elf, 58)
+    for s in range(shnum):
+        sh = shoff + s * shsize
+        if struct.unpack_from("<I", elf, sh + 4)[0] == 7:  # SHT_NOTE
+            (o,) = struct.unpack_from("<Q", elf, sh + 24)
+            name, desc, _ = struct.unpack_from("<III", elf, o)
+            md = msgpack.unpackb(elf[o + 12 + (name + 3) // 4 * 4:][:desc])
+            return {k[".name"]: k for k in md["amdhsa.kernels"]}
+    return {}
+
+
+def test_table_kernel_keeps_eight_waves():
+    # short segments: the kernel with low-low target tables lives on waves in
+    # flight (512 registers per lane and SIMD, eight waves of 64)
+    ks = {n: k for n, k in kernels().items() if "hv_ranked_kernel" in n}
+    assert any(re.search("hv_ranked_kernelId", n) for n in ks)
+    for n, k in ks.items():
+        if re.search("hv_ranked_kernelId", n):
+            assert k[".vgpr_count"] + k[".agpr_count"] <= 64 and k[".vgpr_spill_count"] == 0, n
