@@ -175,7 +175,8 @@ hipError_t op_hv(const alps_ed_operator_s* op, const V* x, V* y, double* dot_out
 }
 
 // The H.v autotuner: an operator of a fixed-Sz sector with at least
-// kTuneMinDim states times every FP32 schedule on its own sector (two
+// kTuneMinDim states and more than kFewSegments segments (the others have one
+// schedule) times every FP32 schedule on its own sector (two
 // round-robin passes of one warm-up and three timed launches each, HIP
 // events on the engine's stream) and keeps the fastest.  Choices are cached per sector shape (sites, up
 // spins, low-word size and the bonds), so later operators of the same shape
@@ -191,7 +192,7 @@ std::vector<uint64_t> schedule_key(const SectorLayout& L) {
 }
 
 void tune_schedule(alps_ed_operator op) {
-  if (op->bloch || op->layout.D < kTuneMinDim) return;
+  if (op->bloch || op->layout.D < kTuneMinDim || op->dev.n_seg <= kFewSegments) return;
   static std::mutex mu;
   static std::map<std::vector<uint64_t>, std::pair<int, std::vector<double>>> cache;
   const std::vector<uint64_t> key = schedule_key(op->layout);

@@ -44,11 +44,11 @@ __global__ __launch_bounds__(NT, W) void hv_kernel(DevLayout L, const V* __restr
                                              DOT ? dot_out + blockIdx.x : nullptr);
 }
 
-template <class V, bool DOT>
-__global__ __launch_bounds__(kBlock, HvWaves<V>::value) void hv_ranked_kernel(DevLayout L, const V* __restrict__ x,
-                                                                             V* __restrict__ y,
-                                                                             double* __restrict__ dot_out) {
-  hv_ranked_at<V, DOT>(L, ldc_struct<SegHead>(L.seg_rec + blockIdx.x), x, y, DOT ? dot_out + blockIdx.x : nullptr);
+template <class V, bool DOT, int W, int CLL, int CHH, int CX>
+__global__ __launch_bounds__(kBlock, W) void hv_ranked_kernel(DevLayout L, const V* __restrict__ x,
+                                                              V* __restrict__ y, double* __restrict__ dot_out) {
+  hv_ranked_at<V, DOT, CLL, CHH, CX>(L, ldc_struct<SegHead>(L.seg_rec + blockIdx.x), x, y,
+                                     DOT ? dot_out + blockIdx.x : nullptr);
 }
 
 // seg_rec[i] for processing index i (the record hv_segment would look up).
@@ -86,11 +86,34 @@ void launch_hv_schedule(const DevLayout& L, const V* x, V* y, double* dot_out, h
   }
 }
 
+template <class V, bool DOT, int S>
+void launch_hv_ranked_with(const DevLayout& L, const V* x, V* y, double* dot_out, hipStream_t st) {
+  constexpr HvRankedSchedule c = kHvRankedSchedule[S];
+  const size_t lds = std::max<size_t>(kHvMinLds, (L.max_seg + 1) * sizeof(double));
+  hipLaunchKernelGGL((hv_ranked_kernel<V, DOT, sizeof(V) == 4 ? c.waves : 1, c.cll, c.chh, c.cx>), dim3(hv_blocks(L)),
+                     dim3(kBlock), lds, st, L, x, y, dot_out);
+}
+
+template <class V, bool DOT>
+void launch_hv_ranked(const DevLayout& L, const V* x, V* y, double* dot_out, hipStream_t st, int schedule) {
+  if constexpr (sizeof(V) == 4) {
+    static_assert(kHvSchedules == 6, "one case per schedule");
+    switch (schedule) {
+      case 1: launch_hv_ranked_with<V, DOT, 1>(L, x, y, dot_out, st); return;
+      case 2: launch_hv_ranked_with<V, DOT, 2>(L, x, y, dot_out, st); return;
+      case 3: launch_hv_ranked_with<V, DOT, 3>(L, x, y, dot_out, st); return;
+      case 4: launch_hv_ranked_with<V, DOT, 4>(L, x, y, dot_out, st); return;
+      case 5: launch_hv_ranked_with<V, DOT, 5>(L, x, y, dot_out, st); return;
+      default: break;
+    }
+  }
+  launch_hv_ranked_with<V, DOT, 0>(L, x, y, dot_out, st);
+}
+
 template <class V, bool DOT>
 void launch_hv_stage(const DevLayout& L, const V* x, V* y, double* dot_out, hipStream_t st, int schedule) {
-  if (L.nbp16 != nullptr) {  // one schedule
-    const size_t lds = std::max<size_t>(kHvMinLds, (L.max_seg + 1) * sizeof(double));
-    hipLaunchKernelGGL((hv_ranked_kernel<V, DOT>), dim3(hv_blocks(L)), dim3(kBlock), lds, st, L, x, y, dot_out);
+  if (L.nbp16 != nullptr) {
+    launch_hv_ranked<V, DOT>(L, x, y, dot_out, st, schedule);
     return;
   }
   if (L.n_xs > 0) launch_hv_schedule<V, DOT, true>(L, x, y, dot_out, st, schedule);

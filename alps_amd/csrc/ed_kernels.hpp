@@ -155,7 +155,16 @@ struct HvSchedule {
 constexpr int kHvSchedules = 6;
 constexpr HvSchedule kHvSchedule[kHvSchedules] = {{8, 2, 4}, {8, 1, 4}, {8, 4, 4}, {7, 2, 4}, {6, 2, 4}, {6, 4, 4}};
 // Layouts of at most kFewSegments segments take 512 threads a workgroup
-// instead of kBlock, whatever the schedule.
+// instead of kBlock, whatever the schedule.  Layouts with low-low target
+// tables (DevLayout::nbp16) have six of their own, with the cross bonds per
+// chunk: the best of them over the first, us: 24-site J1-J2 (width 3) 8 up
+// 19.9 and 20.5 (schedule 4), 27 sites 9 up 126.1 and 130.5 (4), 23-site ring
+// 8 up 5.13 and 5.19 (3).
+struct HvRankedSchedule {
+  int waves, cll, chh, cx;
+};
+constexpr HvRankedSchedule kHvRankedSchedule[kHvSchedules] = {{8, 4, 4, 2}, {8, 4, 8, 2}, {6, 4, 8, 2},
+                                                              {6, 4, 4, 2}, {8, 8, 4, 2}, {6, 8, 8, 4}};
 
 // y = H x; with dot_out set, per-block partials of sum_i x_i (H x)_i (FP64,
 // before y is rounded to the storage type).

@@ -107,11 +107,12 @@ int alps_ed_operator_create_momentum(const alps_ed_model* model, int n_translati
 int alps_ed_operator_destroy(alps_ed_operator op);
 /* No counterpart in the reference: the H.v schedule (waves per SIMD and
  * flip-loop chunk sizes) an operator uses with FP32 vectors.  Operators of
- * fixed-Sz sectors with at least 200000 states pick theirs at creation by
- * timing all ALPS_ED_HV_SCHEDULES of them; seconds[s] receives each one's
- * time per H.v (-1 when the operator was not timed; seconds may be null).
- * Schedules differ only in speed: every one gives the same y.
- * set_schedule forces one (for inspection and tests). */
+ * fixed-Sz sectors with at least 200000 states and more than 512 high words
+ * (the bits above the lowest 12) pick theirs at creation by timing all
+ * ALPS_ED_HV_SCHEDULES of them; seconds[s] receives each one's time per H.v
+ * (-1 when the operator was not timed; seconds may be null).  Sectors of fewer
+ * high words have one schedule.  Schedules differ only in speed: every one
+ * gives the same y.  set_schedule forces one (for inspection and tests). */
 #define ALPS_ED_HV_SCHEDULES 6
 int alps_ed_operator_schedule(alps_ed_operator op, int* schedule, double* seconds);
 int alps_ed_operator_set_schedule(alps_ed_operator op, int schedule);

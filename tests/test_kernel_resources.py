@@ -51,3 +51,12 @@ def test_table_kernel_keeps_eight_waves():
     for n, k in ks.items():
         if re.search("hv_ranked_kernelId", n):
             assert k[".vgpr_count"] + k[".agpr_count"] <= 64 and k[".vgpr_spill_count"] == 0, n
+
+
+def test_every_schedule_is_a_kernel():
+    # six FP32 schedules (ALPS_ED_HV_SCHEDULES) with and without the dot, of
+    # the page kernel (gathered and staged; and its 512-thread form) and of the
+    # table kernel
+    ks = [n for n in kernels() if "9hv_kernelIf" in n or "hv_ranked_kernelIf" in n]
+    assert sum("hv_ranked_kernelIf" in n for n in ks) == 2 * A.Operator.HV_SCHEDULES
+    assert sum("9hv_kernelIf" in n for n in ks) == 4 * (A.Operator.HV_SCHEDULES + 1)
