@@ -275,7 +275,9 @@ class PackedUpload {
 // where they are, the per-high-word lists are built on the device).
 SectorLayout operator_layout(const alps_ed_model* model) { return build_layout(model_spec(model), -1, false); }
 
-void operator_upload(alps_ed_operator op) {
+// momentum: the operator becomes a momentum sector (bloch_upload), whose
+// product reads none of the H.v tables.
+void operator_upload(alps_ed_operator op, bool momentum = false) {
   SectorLayout& L = op->layout;
   DevLayout& d = op->dev;
   d = DevLayout{};
@@ -305,8 +307,10 @@ void operator_upload(alps_ed_operator op) {
   ALPS_ED_UP(diag_lo_cls)
   ALPS_ED_UP(diag_hi)
   ALPS_ED_UP(ll_c)
-  if (L.ranked && !L.nbp16.empty()) {
-    ALPS_ED_UP(nbp16)
+  std::shared_ptr<const std::vector<uint16_t>> ll_table;
+  if (L.ranked && L.n_ll_p > 0 && !momentum) {
+    ll_table = low_flip_table(L);
+    pk.add(*ll_table, &d.nbp16);
     ALPS_ED_UP(nbp_off)
     ALPS_ED_UP(ll_t)
     d.n_ll_p = L.n_ll_p;
@@ -536,7 +540,7 @@ int alps_ed_operator_create_momentum(const alps_ed_model* model, int n_translati
     std::unique_ptr<alps_ed_operator_s> op(new alps_ed_operator_s);
     op->layout = operator_layout(model);
     require(op->layout.D >= 1, "empty sector");
-    operator_upload(op.get());
+    operator_upload(op.get(), true);
     bloch_upload(op.get(), bloch_sector(bloch_orbits(op->layout, t), t, op->layout.N));
     *out = op.release();
   });
@@ -1539,7 +1543,7 @@ SectorSolve solve_sector(const alps_ed_model* model, const alps_ed_solve_params*
   out.op.reset(new alps_ed_operator_s);
   alps_ed_operator_s* op = out.op.get();
   op->layout = mom ? *mom->layout : operator_layout(model);
-  if (op->layout.D > 0) operator_upload(op);
+  if (op->layout.D > 0) operator_upload(op, mom != nullptr);
   if (mom && op->layout.D > 0) bloch_upload(op, bloch_sector(*mom->orbits, *mom->trans, op->layout.N));
   const uint64_t D = mom ? op->n / 2 : op->layout.D;  // the sector's dimension
   result->dim = D;

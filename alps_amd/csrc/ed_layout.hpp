@@ -200,7 +200,8 @@ struct SectorLayout {
   //     bits across which there is no segment have none (info 0, at the end);
   //   xw[h * kXwStride + p]: what low bit p set adds to the diagonal of the
   //     rows of h through the cross bonds, and [B]: what every row gets.
-  // A host-side description of the low-low flips (only with copy_shared):
+  // Low-low flips of the kernel that reads their targets (low_flip_table;
+  // here only with copy_shared):
   //   nbp16[nbp_off[c] + flip_index(r, b, n_ll_p, kLLChunk)]: 8 * the row
   //     reached from row r of a class-c segment by low-low bond b, or
   //     8 * C(B,c) if the bond does not flip it.
@@ -368,6 +369,38 @@ inline std::shared_ptr<const FlipTables> flip_tables(int B, const std::vector<ui
   return F;
 }
 
+// The low-low target table of a layout (SectorLayout::nbp16), cached by its
+// bonds: a program's operators mostly share the lattice.
+inline std::shared_ptr<const std::vector<uint16_t>> low_flip_table(const SectorLayout& L) {
+  std::vector<uint32_t> key{(uint32_t)L.B, (uint32_t)L.n_ll_p};
+  for (const FlipBond& f : L.ll) key.push_back(f.mask);
+  static std::mutex mu;
+  static std::map<std::vector<uint32_t>, std::shared_ptr<const std::vector<uint16_t>>> cache;
+  {
+    std::lock_guard<std::mutex> g(mu);
+    auto it = cache.find(key);
+    if (it != cache.end()) return it->second;
+  }
+  const LowTables& T = low_tables(L.B);
+  const std::vector<uint32_t> off = flip_offsets(L.B, L.n_ll_p);
+  std::shared_ptr<std::vector<uint16_t>> F(new std::vector<uint16_t>(off[L.B + 1], 0));
+  for (int c = 0; c <= L.B; ++c) {
+    const uint32_t len = (uint32_t)binom(L.B, c);
+    for (int b = 0; b < L.n_ll_p; ++b) {
+      const uint32_t m = b < (int)L.ll.size() ? L.ll[b].mask : 0u;
+      for (uint32_t r = 0; r < len; ++r) {
+        const uint32_t lo = T.lo_state[T.lo_class_off[c] + r], bits = lo & m;
+        (*F)[off[c] + flip_index(r, b, L.n_ll_p, kLLChunk)] =
+            (uint16_t)(8u * ((bits != 0u && bits != m) ? T.lo_rank[lo ^ m] : len));
+      }
+    }
+  }
+  std::lock_guard<std::mutex> g(mu);
+  if (cache.size() > 256) cache.clear();  // bounded, as flip_tables
+  cache[key] = F;
+  return F;
+}
+
 // Layouts of at most this many segments are launched with a workgroup of 512
 // threads per segment instead of 256: with two segments or fewer per compute
 // unit the launch lasts as long as one segment's chain of memory rounds, and
@@ -442,6 +475,26 @@ inline double cross_weight(uint32_t h, int p, const XSource& X) {
   return w;
 }
 
+// Appends the n ascending high words at v to the processing order as kXcds
+// runs of equal count: ordered by the set bits of their low five bits, then
+// by address (keyed) or by address alone, cut into runs, and dealt so that
+// position p takes from run p % kXcds, each run in ascending address; what is
+// left over (fewer than kXcds) comes last, in run order.  One pass, no sort.
+inline void deal_runs(const uint32_t* v, uint32_t n, bool keyed, std::vector<uint32_t>& out) {
+  const uint32_t run = n / kXcds, s = (uint32_t)out.size();
+  out.resize((size_t)s + n);
+  uint32_t next[7] = {}, filled[kXcds] = {};  // the next place of a key, and of a run
+  if (keyed) {
+    for (uint32_t i = 0; i < n; ++i) ++next[__builtin_popcount(v[i] & 31u) + 1];
+    for (int k = 1; k < 7; ++k) next[k] += next[k - 1];
+  }
+  for (uint32_t i = 0; i < n; ++i) {
+    const uint32_t at = next[keyed ? __builtin_popcount(v[i] & 31u) : 0]++;
+    const uint32_t g = at < run * kXcds ? at / run : (uint32_t)kXcds;
+    out[s + (g < (uint32_t)kXcds ? kXcds * filled[g]++ + (g - s) % kXcds : at)] = v[i];
+  }
+}
+
 // copy_shared = false leaves lo_rank, lo_state, nbp16 and xn16 empty: the
 // engine reads the shared tables (L.low, L.flip; the batch uploads them once
 // per shape) and needs no nbp16.  host_lists = false leaves the per-high-word lists
@@ -505,85 +558,67 @@ inline SectorLayout build_layout(const ModelSpec& m, int B_override = -1, bool c
   {
     std::vector<std::vector<uint32_t>> by_len(B + 1);  // by class kl, in ascending hi
     for (uint32_t h : L.seg_hi) by_len[L.k - __builtin_popcount(h)].push_back(h);
+    // (more low bits first among classes of equal length: their first high
+    // word is the smaller one)
     std::vector<int> cls;
-    for (int c = 0; c <= B; ++c)
+    for (int c = B; c >= 0; --c)
       if (!by_len[c].empty()) cls.push_back(c);
     std::stable_sort(cls.begin(), cls.end(), [&](int a, int b) { return binom(B, a) > binom(B, b); });
-    // classes of equal length interleave in ascending hi, as a stable sort
-    // of the whole list by length leaves them
+    if (!cls.empty()) L.max_seg = (uint32_t)binom(B, cls[0]);
     L.proc_hi.clear();
     L.proc_hi.reserve(L.seg_hi.size());
-    for (size_t i = 0; i < cls.size();) {
-      size_t j = i;
-      while (j < cls.size() && binom(B, cls[j]) == binom(B, cls[i])) ++j;
-      // each class's list is ascending: merge them (at most two classes,
-      // c and B - c, share a length)
-      const size_t start = L.proc_hi.size();
-      for (size_t q = i; q < j; ++q) {
-        const size_t mid = L.proc_hi.size();
-        L.proc_hi.insert(L.proc_hi.end(), by_len[cls[q]].begin(), by_len[cls[q]].end());
-        std::inplace_merge(L.proc_hi.begin() + start, L.proc_hi.begin() + mid, L.proc_hi.end());
+    // Workgroups are dealt to the 8 XCDs round-robin (block b runs on XCD
+    // b % 8), each XCD with its own L2.  A large layout is dealt class by class,
+    // longest first: each class is cut into kXcds runs of equal count, ordered
+    // by the set bits among the high word's low five bits and then by address,
+    // and position p of the order takes from run p % 8, in ascending address.
+    // A bond inside the low five bits, or inside the others, leaves the run's
+    // key as it is and mostly leads to a segment that the same XCD reads at
+    // about the same time; equal counts of one class are equal work, so the
+    // XCDs stay balanced.  Against groups by the top three bits (24 sites) and
+    // four slices per class of runs in address order (the others): ring of 24
+    // sites FP32 14.6 -> 13.6 us, FP64 23.5 -> 21.1, 25 sites XXZ FP64 36.0 ->
+    // 34.5, 26 sites FP32 47.4 -> 45.6, 28-site J1-J2 672 -> 661 us (keys of
+    // four and eight bits within 4 % of that).  A class of more than kSliceClass
+    // segments keeps four slices in address order one after the other, so that
+    // the x of the segments in flight stays within a quarter of it: 30-site
+    // J1-J2 (48620 segments) 3.31 ms, 3.37 with the key; 28 sites (12870) 664
+    // and 661 us.
+    if (L.seg_hi.size() >= 64u * kXcds) {
+      constexpr size_t kSliceClass = 16384;
+      for (int c : cls) {
+        const std::vector<uint32_t>& v = by_len[c];
+        const bool keyed = v.size() <= kSliceClass;
+        const size_t slice = keyed ? v.size() : (v.size() + 3) / 4;
+        for (size_t s0 = 0; s0 < v.size(); s0 += slice)
+          deal_runs(v.data() + s0, (uint32_t)std::min(slice, v.size() - s0), keyed, L.proc_hi);
       }
-      i = j;
-    }
-    if (!cls.empty()) L.max_seg = (uint32_t)binom(B, cls[0]);
-  }
-  // Workgroups are dealt to the 8 XCDs round-robin (block b runs on XCD
-  // b % 8), each XCD with its own L2.  A large layout is dealt class by class,
-  // longest first: each class is cut into kXcds runs of equal count, ordered
-  // by the set bits among the high word's low five bits and then by address,
-  // and position p of the order takes from run p % 8, in ascending address.
-  // A bond inside the low five bits, or inside the others, leaves the run's
-  // key as it is and mostly leads to a segment that the same XCD reads at
-  // about the same time; equal counts of one class are equal work, so the
-  // XCDs stay balanced.  Against groups by the top three bits (24 sites) and
-  // four slices per class of runs in address order (the others): ring of 24
-  // sites FP32 14.6 -> 13.6 us, FP64 23.5 -> 21.1, 25 sites XXZ FP64 36.0 ->
-  // 34.5, 26 sites FP32 47.4 -> 45.6, 28-site J1-J2 672 -> 661 us (keys of
-  // four and eight bits within 4 % of that).  A class of more than kSliceClass
-  // segments keeps four slices in address order one after the other, so that
-  // the x of the segments in flight stays within a quarter of it: 30-site
-  // J1-J2 (48620 segments) 3.31 ms, 3.37 with the key; 28 sites (12870) 664
-  // and 661 us.
-  if (L.seg_hi.size() >= 64u * kXcds) {
-    std::vector<int> cls_order;
-    std::vector<std::vector<uint32_t>> by_pc(L.NH + 1);
-    for (uint32_t h : L.proc_hi) {
-      const int c = __builtin_popcount(h);
-      if (by_pc[c].empty()) cls_order.push_back(c);
-      by_pc[c].push_back(h);
-    }
-    L.proc_hi.clear();
-    constexpr size_t kSliceClass = 16384;
-    for (int c : cls_order) {
-      std::vector<uint32_t>& v = by_pc[c];
-      size_t slice = (v.size() + 3) / 4;
-      if (v.size() <= kSliceClass) {
-        slice = v.size();
-        std::vector<uint32_t> w[6];
-        for (uint32_t h : v) w[__builtin_popcount(h & 31u)].push_back(h);
-        v.clear();
-        for (auto& k : w) v.insert(v.end(), k.begin(), k.end());
+    } else {
+      for (size_t i = 0; i < cls.size();) {
+        size_t j = i;
+        while (j < cls.size() && binom(B, cls[j]) == binom(B, cls[i])) ++j;
+        // each class's list is ascending: merge them (at most two classes,
+        // c and B - c, share a length)
+        const size_t start = L.proc_hi.size();
+        for (size_t q = i; q < j; ++q) {
+          const size_t mid = L.proc_hi.size();
+          L.proc_hi.insert(L.proc_hi.end(), by_len[cls[q]].begin(), by_len[cls[q]].end());
+          std::inplace_merge(L.proc_hi.begin() + start, L.proc_hi.begin() + mid, L.proc_hi.end());
+        }
+        i = j;
       }
-      for (size_t s0 = 0; s0 < v.size(); s0 += slice) {
-        const auto q = v.begin() + s0;
-        const size_t n = std::min(slice, v.size() - s0), run = n / kXcds, s = L.proc_hi.size();
-        for (int g = 0; g < kXcds; ++g) std::sort(q + g * run, q + (g + 1) * run);
-        for (size_t i = 0; i < run; ++i)
-          for (int j = 0; j < kXcds; ++j) L.proc_hi.push_back(q[((s + j) % kXcds) * run + i]);
-        L.proc_hi.insert(L.proc_hi.end(), q + kXcds * run, q + n);
+      if (L.NH >= 3) {
+        // groups by the top three bits where these split the segments evenly
+        std::vector<std::vector<uint32_t>> grp(kXcds);
+        for (uint32_t h : L.proc_hi) grp[h >> (L.NH - 3)].push_back(h);
+        bool even = true;
+        for (const auto& g : grp) even = even && g.size() == grp[0].size();
+        if (even && !grp[0].empty()) {
+          L.proc_hi.clear();
+          for (size_t i = 0; i < grp[0].size(); ++i)
+            for (int g = 0; g < kXcds; ++g) L.proc_hi.push_back(grp[g][i]);
+        }
       }
-    }
-  } else if (L.NH >= 3) {
-    // few segments: groups by the top three bits where these split them evenly
-    std::vector<std::vector<uint32_t>> grp(kXcds);
-    for (uint32_t h : L.proc_hi) grp[h >> (L.NH - 3)].push_back(h);
-    bool even = true;
-    for (const auto& g : grp) even = even && g.size() == grp[0].size();
-    if (even && !grp[0].empty()) {
-      L.proc_hi.clear();
-      for (size_t i = 0; i < grp[0].size(); ++i)
-        for (int g = 0; g < kXcds; ++g) L.proc_hi.push_back(grp[g][i]);
     }
   }
   // terms in bit coordinates
@@ -673,20 +708,8 @@ inline SectorLayout build_layout(const ModelSpec& m, int B_override = -1, bool c
     if (copy_shared) L.xn16 = L.flip->xn16;
   }
   L.ranked = ranked_rows(B, L.D, L.seg_hi.size());
-  if (copy_shared || (L.ranked && !host_lists)) {
-    L.nbp_off = flip_offsets(B, L.n_ll_p);
-    L.nbp16.assign(L.nbp_off[B + 1], 0);
-    for (int c = 0; c <= B; ++c) {
-      const uint32_t len = (uint32_t)binom(B, c);
-      for (int b = 0; b < L.n_ll_p; ++b)
-        for (uint32_t r = 0; r < len; ++r) {
-          const uint32_t lo = L.low->lo_state[L.lo_class_off[c] + r];
-          const uint32_t m = b < (int)L.ll.size() ? L.ll[b].mask : 0u, bits = lo & m;
-          L.nbp16[L.nbp_off[c] + flip_index(r, b, L.n_ll_p, kLLChunk)] =
-              (uint16_t)(8u * ((bits != 0u && bits != m) ? L.low->lo_rank[lo ^ m] : len));
-        }
-    }
-  }
+  L.nbp_off = flip_offsets(B, L.n_ll_p);
+  if (copy_shared) L.nbp16 = *low_flip_table(L);
   for (const FlipBond& f : L.ll) L.ll_c.push_back(PageBond{f.t, 8u * page_pos(f.mask), 0u});
   L.ll_c.resize(L.n_ll_p, PageBond{0.0, 0u, 0u});
   for (const PageBond& c : L.ll_c) L.ll_t.push_back(c.t);
