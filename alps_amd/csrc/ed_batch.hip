@@ -304,6 +304,7 @@ size_t table_bytes(const SectorLayout& L) {
   add(L.xb_c.size(), sizeof(XBondConst));
   add(L.xb_nb.size(), 4);
   add(L.xb_p.size(), sizeof(PageBond));
+  add(L.proc_index.size(), 4);
   add(L.xs.size(), sizeof(XStage));
   add(L.xw.size(), 8);
   add(L.site_dn.size(), 8);
@@ -370,6 +371,7 @@ DevLayout place_tables(const SectorLayout& L, char* base, char* stage, const Sha
   d.xb_c = put(L.xb_c);
   d.xb_nb = put(L.xb_nb);
   d.xb_p = put(L.xb_p);
+  d.proc_index = put(L.proc_index);
   d.xs = put(L.xs);
   d.xw = put(L.xw);
   d.site_dn = put(L.site_dn);

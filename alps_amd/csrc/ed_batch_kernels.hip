@@ -62,8 +62,7 @@ __global__ __launch_bounds__(kBlock, HvWaves<V>::value) void batch_hv_kernel(con
     store_block_sum_lds<kBlock>(part + it.idx, p);
     return;
   }
-  const uint32_t h = ldc(L.proc_hi + it.idx);
-  hv_segment_at<V, true, STAGE>(L, seg_record(L, h), x, y, part + it.idx);
+  hv_segment_at<V, true, STAGE>(L, seg_record(L, it.idx), x, y, part + it.idx);
 }
 
 // Where stage j (the start for j = 0, the update of step j - 1 otherwise)
@@ -303,11 +302,10 @@ __global__ __launch_bounds__(kBlock) void batch_plain_hv_kernel(const PlainHvJob
     store_block_sum_lds<kBlock>(ldc(&J->part) + it.idx, p);
     return;
   }
-  const uint32_t h = ldc(L.proc_hi + it.idx);
   if (L.n_xs > 0)
-    hv_segment_at<double, true, true>(L, seg_record(L, h), ldc(&J->x), ldc(&J->y), ldc(&J->part) + it.idx);
+    hv_segment_at<double, true, true>(L, seg_record(L, it.idx), ldc(&J->x), ldc(&J->y), ldc(&J->part) + it.idx);
   else
-    hv_segment_at<double, true, false>(L, seg_record(L, h), ldc(&J->x), ldc(&J->y), ldc(&J->part) + it.idx);
+    hv_segment_at<double, true, false>(L, seg_record(L, it.idx), ldc(&J->x), ldc(&J->y), ldc(&J->part) + it.idx);
 }
 
 }  // namespace

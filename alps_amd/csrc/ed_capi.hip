@@ -319,6 +319,7 @@ void operator_upload(alps_ed_operator op, bool momentum = false) {
   ALPS_ED_UP(xn_off)
   ALPS_ED_UP(xb_c)
   ALPS_ED_UP(xb_p)
+  ALPS_ED_UP(proc_index)
   const bool dev_lists = L.hh_off.empty();  // host_lists = false: built below
   const uint32_t *hh_mask = nullptr, *xb_hbit = nullptr;
   const double* hh_t = nullptr;
@@ -354,16 +355,16 @@ void operator_upload(alps_ed_operator op, bool momentum = false) {
     const uint32_t nhi = 1u << L.NH;
     auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
     const size_t nb_at = up((size_t)(nhi + 1) * 4), xs_at = nb_at + (L.stage ? 0 : up((size_t)nhi * L.n_xb_p * 4)),
-                 xw_at = xs_at + up((size_t)nhi * d.n_xs * sizeof(XStage)),
-                 end = xw_at + (L.stage ? (size_t)nhi * kXwStride * sizeof(double) : 0);
+                 xw_at = xs_at + up((size_t)d.n_seg * d.n_xs * sizeof(XStage)),
+                 end = xw_at + (L.stage ? (size_t)d.n_seg * kXwStride * sizeof(double) : 0);
     op->lists.alloc(end);
     char* lists = op->lists.as<char>();
     uint32_t* off = reinterpret_cast<uint32_t*>(lists);
     uint32_t* xnb = reinterpret_cast<uint32_t*>(lists + nb_at);
     XStage* xs = reinterpret_cast<XStage*>(lists + xs_at);
     double* xw = reinterpret_cast<double*>(lists + xw_at);
-    hip_check(launch_hh_count(nhi, d.hi_base, hh_mask, (int)L.hh_mask.size(), off, xb_hbit, L.n_xb_p, xnb, X, xs, xw,
-                              nullptr),
+    hip_check(launch_hh_count(nhi, d.hi_base, hh_mask, (int)L.hh_mask.size(), off, xb_hbit, L.n_xb_p, xnb, d.n_seg,
+                              d.seg_hi, X, xs, xw, nullptr),
               "high-high lists");
     uint32_t total = 0;
     hip_check(hipMemcpy(&total, off + nhi, sizeof(uint32_t), hipMemcpyDeviceToHost), "high-high lists");

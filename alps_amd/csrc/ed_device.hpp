@@ -408,7 +408,7 @@ __device__ __forceinline__ double hv_rows(const DevLayout& L, const SegRec& S, c
     };
     V sv[AHEAD][MQ];
     uint32_t sp[MQ];
-    const XStage* xs = L.xs + (size_t)S.h * L.n_xs;
+    const XStage* xs = L.xs + (size_t)S.h_or_index * L.n_xs;
     auto stage_of = [&](int i) { return i < L.n_xs ? ldc_struct(xs + i) : XStage{0u, 0u}; };
     auto rows_of = [&](uint32_t info) { return (int)info < 0 ? S.len_up : S.len_dn; };
     auto stage_load = [&](V(&v)[MQ], XStage st) {
@@ -472,7 +472,7 @@ __device__ __forceinline__ double hv_rows(const DevLayout& L, const SegRec& S, c
     lds_barrier();
     if (tid < 128u) {
       const uint32_t hf = __builtin_amdgcn_readfirstlane(tid >> 6);
-      const double* w = L.xw + (size_t)S.h * kXwStride;
+      const double* w = L.xw + (size_t)S.h_or_index * kXwStride;
       double s = hf ? S.dh : ldc(w + L.B);
 #pragma unroll
       for (uint32_t p = 0; p < 6u; ++p) s = fma((tid >> p & 1u) ? 1.0 : 0.0, ldc(w + 6u * hf + p), s);
@@ -501,14 +501,15 @@ __device__ __forceinline__ double hv_rows(const DevLayout& L, const SegRec& S, c
     const uint32_t x_slot = (uint32_t)NT * (uint32_t)L.n_xb_p;  // u16 entries per slot
 #pragma unroll
     for (int q = 0; q < NQ; ++q) d[q] = S.dh;
-    const uint32_t* xnb = L.xb_nb + S.h * (uint32_t)L.n_xb_p;
+    const uint32_t h = S.h_or_index;  // not staged: the high word
+    const uint32_t* xnb = L.xb_nb + h * (uint32_t)L.n_xb_p;
     for (int b0 = 0; NQ > 0 && b0 < L.n_xb; b0 += kXChunk) {
       // the two bonds' entries, bits 15 and 31 set where the row flips
       uint32_t e[NA];
 #pragma unroll
       for (int q = 0; q < NQ; ++q) e[q] = ld_at<uint32_t>(xnp + q * x_slot + (uint32_t)b0 * 64u, lo_x);
       const XBondConst k0 = ldc_struct(L.xb_c + b0), k1 = ldc_struct(L.xb_c + b0 + 1);
-      const uint32_t hx = ((S.h & k0.hbit) != 0u ? 0x8000u : 0u) | ((S.h & k1.hbit) != 0u ? 0x80000000u : 0u);
+      const uint32_t hx = ((h & k0.hbit) != 0u ? 0x8000u : 0u) | ((h & k1.hbit) != 0u ? 0x80000000u : 0u);
       const V *x0 = x + ldc(xnb + b0), *x1 = x + ldc(xnb + b0 + 1);
       // all ones where the row flips: it masks the gathered offset (to the
       // segment's first row), the value and the 1.0 of the diagonal
@@ -547,8 +548,8 @@ __device__ __forceinline__ double hv_rows(const DevLayout& L, const SegRec& S, c
   return dotp;
 }
 
-// H.v over the row segment of record S (high word S.h; one workgroup of
-// NT threads; dynamic LDS of at least page_bytes(L.B)):
+// H.v over the row segment of record S (one workgroup of NT threads; dynamic
+// LDS of at least page_bytes(L.B)):
 //   y[r] = sum_c H[r][c] x[c] for the segment's rows r;
 // with DOT, *dot_slot receives the segment's sum of x_r (H x)_r (FP64, before
 // y is rounded to the storage type).  STAGE: L.n_xs > 0.
@@ -604,16 +605,15 @@ __device__ __forceinline__ void hv_segment_at(const DevLayout& L, const SegRec& 
 // in hv_rows outweighs its rows.  Bound by the chain of dependent loads of a
 // segment, so by the waves in flight and by scalar loads: a row's own element
 // is read from LDS again at the end rather than kept (FP64: 64 registers, 8
-// waves per SIMD instead of 7), the coefficients are contiguous and only the
-// first 40 bytes of the record are read: 24 sites 8 up 7.84 -> 7.52 us (FP32)
+// waves per SIMD instead of 7), the coefficients are contiguous and only
+// what it needs of the record is read: 24 sites 8 up 7.84 -> 7.52 us (FP32)
 // and 10.68 -> 10.46 (FP64), 22 sites 7 up 4.23 -> 4.14 and 4.68 -> 4.55, 23
 // sites 7 up 4.69 -> 4.54 and 5.44 -> 5.30, 27-site J1-J2 9 up 132.5 -> 130.6
 // and 181.3 -> 180.2.
 template <class V, bool DOT, int NQ, int CLL, int CHH, int CX>
-__device__ __forceinline__ double hv_ranked_rows(const DevLayout& L, const SegHead& S, const V* __restrict__ x,
-                                                 V* __restrict__ y) {
-  const uint32_t h = S.h, len = S.len, base = S.base, e0 = S.e0, e1 = S.e1;
-  const double dh = S.dh;
+__device__ __forceinline__ double hv_ranked_rows(const DevLayout& L, const SegHead& S, double dh,
+                                                 const V* __restrict__ x, V* __restrict__ y) {
+  const uint32_t h = S.h_or_index, len = S.len, base = S.base, e0 = S.e0, e1 = S.e1;
   const uint16_t* nbp = L.nbp16 + S.nbp;
   const uint16_t* xnp = L.xn16 + S.xnp;
   const double* dlp = L.diag_lo_cls + S.cls0;
@@ -805,28 +805,30 @@ __device__ __forceinline__ double hv_ranked_rows(const DevLayout& L, const SegHe
 // The same workgroup and slots as hv_segment_at; dynamic LDS of max_seg + 1
 // doubles.
 template <class V, bool DOT, int CLL = 4, int CHH = 4, int CX = 2>
-__device__ __forceinline__ void hv_ranked_at(const DevLayout& L, const SegHead& S, const V* __restrict__ x,
-                                             V* __restrict__ y, double* __restrict__ dot_slot) {
+__device__ __forceinline__ void hv_ranked_at(const DevLayout& L, const SegHead& S, double dh,
+                                             const V* __restrict__ x, V* __restrict__ y,
+                                             double* __restrict__ dot_slot) {
   const uint32_t w0 = threadIdx.x & ~63u;
   const uint32_t nq = __builtin_amdgcn_readfirstlane(S.len > w0 ? (S.len - w0 + kBlock - 1) / kBlock : 0u);
   static_assert(kMaxSegRows == 4 * kBlock, "one to four row slots");
   double dotp = 0.0;
   if (nq == 0) lds_barrier();
-  else if (nq == 1) dotp = hv_ranked_rows<V, DOT, 1, CLL, CHH, CX>(L, S, x, y);
-  else if (nq == 2) dotp = hv_ranked_rows<V, DOT, 2, CLL, CHH, CX>(L, S, x, y);
-  else if (nq == 3) dotp = hv_ranked_rows<V, DOT, 3, CLL, CHH, CX>(L, S, x, y);
-  else dotp = hv_ranked_rows<V, DOT, 4, CLL, CHH, CX>(L, S, x, y);
+  else if (nq == 1) dotp = hv_ranked_rows<V, DOT, 1, CLL, CHH, CX>(L, S, dh, x, y);
+  else if (nq == 2) dotp = hv_ranked_rows<V, DOT, 2, CLL, CHH, CX>(L, S, dh, x, y);
+  else if (nq == 3) dotp = hv_ranked_rows<V, DOT, 3, CLL, CHH, CX>(L, S, dh, x, y);
+  else dotp = hv_ranked_rows<V, DOT, 4, CLL, CHH, CX>(L, S, dh, x, y);
   if (DOT) {
     lds_barrier();  // every wave is done with the slice
     store_block_sum_lds<kBlock>(dot_slot, dotp);
   }
 }
 
-// The record of the segment of high word h, looked up in the tables.
-__device__ __forceinline__ SegRec seg_record(const DevLayout& L, uint32_t h) {
+// The record of segment seg of the processing order, looked up in the tables.
+__device__ __forceinline__ SegRec seg_record(const DevLayout& L, uint32_t seg) {
+  const uint32_t h = ldc(L.proc_hi + seg);
   const int kl = L.k - __builtin_popcount(h);
   SegRec S;
-  S.h = h;
+  S.h_or_index = L.n_xs > 0 ? ldc(L.proc_index + seg) : h;
   S.base = ldc(L.hi_base + h);
   S.cls0 = ldc(L.lo_class_off + kl);
   S.cls_up = ldc(L.lo_class_off + kl + 1);

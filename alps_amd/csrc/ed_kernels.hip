@@ -47,7 +47,8 @@ __global__ __launch_bounds__(NT, W) void hv_kernel(DevLayout L, const V* __restr
 template <class V, bool DOT, int W, int CLL, int CHH, int CX>
 __global__ __launch_bounds__(kBlock, W) void hv_ranked_kernel(DevLayout L, const V* __restrict__ x,
                                                               V* __restrict__ y, double* __restrict__ dot_out) {
-  hv_ranked_at<V, DOT, CLL, CHH, CX>(L, ldc_struct<SegHead>(L.seg_rec + blockIdx.x), x, y,
+  const SegRec* rec = L.seg_rec + blockIdx.x;
+  hv_ranked_at<V, DOT, CLL, CHH, CX>(L, ldc_struct<SegHead>(rec), ldc(&rec->dh), x, y,
                                      DOT ? dot_out + blockIdx.x : nullptr);
 }
 
@@ -55,7 +56,7 @@ __global__ __launch_bounds__(kBlock, W) void hv_ranked_kernel(DevLayout L, const
 __global__ __launch_bounds__(kBlock) void seg_rec_kernel(DevLayout L, SegRec* __restrict__ out) {
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= L.n_seg) return;
-  out[i] = seg_record(L, L.proc_hi[i]);
+  out[i] = seg_record(L, i);
 }
 
 template <class V, bool DOT, bool STAGE, int NT, int W, int CLL, int CHH>
@@ -202,14 +203,15 @@ __global__ __launch_bounds__(kBlock) void xb_nb_kernel(uint32_t nhi, int n_xb_p,
   out[i] = v;
 }
 
-// kXwStride threads per high word: its entries of xw, the last one its stages.
-__global__ __launch_bounds__(kBlock) void cross_stages_kernel(uint32_t nhi, const uint32_t* __restrict__ hi_base,
-                                                              XSource X, XStage* __restrict__ xs,
-                                                              double* __restrict__ xw) {
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x, h = i / kXwStride, p = i % kXwStride;
-  if (h >= nhi || hi_base[h] == 0xffffffffu) return;
+// kXwStride threads per segment: its entries of xw, the last one its stages.
+__global__ __launch_bounds__(kBlock) void cross_stages_kernel(uint32_t n_seg, const uint32_t* __restrict__ seg_hi,
+                                                              const uint32_t* __restrict__ hi_base, XSource X,
+                                                              XStage* __restrict__ xs, double* __restrict__ xw) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x, q = i / kXwStride, p = i % kXwStride;
+  if (q >= n_seg) return;
+  const uint32_t h = seg_hi[q];
   if (p <= (uint32_t)X.B) xw[i] = cross_weight(h, (int)p, X);
-  if (p == kXwStride - 1) cross_stages(h, hi_base, X, xs + (size_t)h * X.ng);
+  if (p == kXwStride - 1) cross_stages(h, hi_base, X, xs + (size_t)q * X.ng);
 }
 
 // One workgroup per item; 16-byte moves where source and destination allow.
@@ -853,15 +855,15 @@ hipError_t launch_normalize(uint64_t n, V* v, Partials norm_in, double* b_out, d
 }
 
 hipError_t launch_hh_count(uint32_t nhi, const uint32_t* hi_base, const uint32_t* mask, int nb, uint32_t* off,
-                           const uint32_t* hbit, int n_xb_p, uint32_t* xb_nb, const XSource& X, XStage* xs,
-                           double* xw, hipStream_t st) {
+                           const uint32_t* hbit, int n_xb_p, uint32_t* xb_nb, uint32_t n_seg,
+                           const uint32_t* seg_hi, const XSource& X, XStage* xs, double* xw, hipStream_t st) {
   const unsigned g = (unsigned)((nhi + kBlock - 1) / kBlock);
   hipLaunchKernelGGL(hh_count_kernel, dim3(g), dim3(kBlock), 0, st, nhi, hi_base, mask, nb, off);
   hipLaunchKernelGGL(scan_inclusive_kernel, dim3(1), dim3(kScanBlock), 0, st, off + 1, nhi);
   const uint64_t nx = (uint64_t)nhi * n_xb_p;
   if (X.ng > 0)
-    hipLaunchKernelGGL(cross_stages_kernel, dim3((nhi * kXwStride + kBlock - 1) / kBlock), dim3(kBlock), 0, st, nhi,
-                       hi_base, X, xs, xw);
+    hipLaunchKernelGGL(cross_stages_kernel, dim3((n_seg * kXwStride + kBlock - 1) / kBlock), dim3(kBlock), 0, st, n_seg,
+                       seg_hi, hi_base, X, xs, xw);
   else if (nx > 0)
     hipLaunchKernelGGL(xb_nb_kernel, dim3((unsigned)((nx + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, nhi, n_xb_p,
                        hi_base, hbit, xb_nb);

@@ -15,8 +15,7 @@ struct DevLayout {
   uint32_t D;
   uint32_t n_seg, max_seg;
   int n_bonds;
-  int n_ll, n_xb;             // low-low and cross flip bonds
-  int n_ll_p, n_xb_p;         // entries per row of their tables
+  int n_ll, n_xb, n_xb_p;     // low-low and cross flip bonds; the cross tables' stride
   int n_xs;                   // high bits with staged cross bonds; 0: gathered
   const uint32_t* lo_rank;
   const uint32_t* lo_state;
@@ -43,8 +42,8 @@ struct DevLayout {
   const uint32_t* xb_nb;      // [2^NH * n_xb_p] first row of the neighbour segment
   // staged cross bonds
   const PageBond* xb_p;
-  const XStage* xs;           // [2^NH * n_xs] per high word: the segments staged for them
-  const double* xw;           // [2^NH * kXwStride] and their share of the diagonal
+  const XStage* xs;           // [n_seg * n_xs] per segment of seg_hi: the segments staged for them
+  const double* xw;           // [n_seg * kXwStride] and their share of the diagonal
   const SegRec* seg_rec;      // [n_seg] per processing index (single operators; the batch looks them up)
   // reference-order description for the element enumeration
   const double* site_dn;
@@ -54,6 +53,11 @@ struct DevLayout {
   const double* bond_par;
   const double* bond_anti;
   const double* bond_t;
+  // Behind what the page kernel reads, whose wide argument loads are sensitive
+  // to what lies between (24-site J1-J2 in FP32: 44.5 us, 44.9 with these two
+  // among the others).
+  const uint32_t* proc_index;  // [n_seg] per processing index: the segment's position in seg_hi (staged)
+  int n_ll_p;                  // entries per row of nbp16
 };
 
 // A momentum sector (Bloch basis, ed_bloch.hpp) on the device.  Vectors of
@@ -216,11 +220,11 @@ hipError_t launch_reorth(uint64_t n, int j, V* r, const double* scale, const Reo
 // off[0..nhi] (the prefix sums of each high word's flipping high-high bond
 // count, rounded up to kHHList; 0xffffffff once they reach 2^32 - 1) and, for
 // gathered cross bonds, xb_nb[nhi * n_xb_p], for staged ones (X.ng > 0)
-// xs[nhi * ng] and xw; launch_hh_fill then writes the off[nhi] entries.  The
+// xs[n_seg * ng] and xw; launch_hh_fill then writes the off[nhi] entries.  The
 // same lists build_layout makes on the host with host_lists.
 hipError_t launch_hh_count(uint32_t nhi, const uint32_t* hi_base, const uint32_t* mask, int nb, uint32_t* off,
-                           const uint32_t* hbit, int n_xb_p, uint32_t* xb_nb, const XSource& X, XStage* xs,
-                           double* xw, hipStream_t st);
+                           const uint32_t* hbit, int n_xb_p, uint32_t* xb_nb, uint32_t n_seg,
+                           const uint32_t* seg_hi, const XSource& X, XStage* xs, double* xw, hipStream_t st);
 hipError_t launch_hh_fill(uint32_t nhi, const uint32_t* hi_base, const uint32_t* mask, const double* t, int nb,
                           const uint32_t* off, HHEntry* ent, hipStream_t st);
 

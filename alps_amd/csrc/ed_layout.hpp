@@ -150,19 +150,21 @@ struct PageBond {
 
 // What the H.v kernel needs of the segment it processes, one record per
 // processing index (built on the device for a single operator): its high
-// word, first row, class offset and length, the range of its listed high-high
-// flips, the flip-table offsets, the high word's diagonal, and the offset and
-// length of the classes with one low bit more and one fewer (the segments
-// across a cross bond; only the staged bonds need them).  Read with scalar
-// loads instead of two dependent rounds of table reads.
+// word or, with staged cross bonds, whose tables go by it, its position in
+// seg_hi; its first row, class offset and length, the range of its listed
+// high-high flips, the flip-table offsets, the offset and length of the
+// classes with one low bit more and one fewer (the segments across a cross
+// bond; only staged bonds need them), and the high word's diagonal.  Read with
+// scalar loads instead of two dependent rounds of table reads; the first field
+// is one that every kernel uses, so that the load stays whole (20-site J1-J2:
+// 10.2 us, 10.4 with the position in the place of nbp).
 struct SegHead {
-  uint32_t h, base, cls0, len;
+  uint32_t h_or_index, base, cls0, len;
   uint32_t e0, e1, xnp, nbp;
-  double dh;
 };
 struct SegRec : SegHead {
   uint32_t cls_up, len_up, cls_dn, len_dn;
-  double pad;
+  double dh, pad;
 };
 static_assert(sizeof(SegRec) == 64, "one scalar load of 16 registers");
 
@@ -195,11 +197,15 @@ struct SectorLayout {
   // Where several share one (stage true): staged in an LDS page,
   //   xb_p[xb.size()]: the bonds, those of one high bit adjacent;
   //   xb_grp[n_xs]: per high bit that has any, its bit and their range;
-  //   xs[h * n_xs + i]: the segments that high word h stages for them, the
-  //     bits set in h first (their segments' words have one low bit more);
-  //     bits across which there is no segment have none (info 0, at the end);
-  //   xw[h * kXwStride + p]: what low bit p set adds to the diagonal of the
+  //   proc_index[i]: the position in seg_hi of proc_hi[i];
+  //   xs[q * n_xs + i]: the segments that high word h = seg_hi[q] stages for
+  //     them, the bits set in h first (their segments' words have one low bit
+  //     more); bits across which there is no segment have none (info 0, at
+  //     the end);
+  //   xw[q * kXwStride + p]: what low bit p set adds to the diagonal of the
   //     rows of h through the cross bonds, and [B]: what every row gets.
+  // (By segment, not by high word: a sector of few up spins has few segments
+  // among its high words.  In address order: neighbours run on the same XCD.)
   // Low-low flips of the kernel that reads their targets (low_flip_table;
   // here only with copy_shared):
   //   nbp16[nbp_off[c] + flip_index(r, b, n_ll_p, kLLChunk)]: 8 * the row
@@ -229,8 +235,9 @@ struct SectorLayout {
   std::vector<PageBond> xb_p;
   std::vector<XGroup> xb_grp;
   std::vector<double> xb_w;               // XSource::w
-  std::vector<XStage> xs;                 // [2^NH * n_xs] (empty when built on the device)
-  std::vector<double> xw;                 // [2^NH * kXwStride] (empty when built on the device)
+  std::vector<uint32_t> proc_index;       // [n_seg], with staged cross bonds
+  std::vector<XStage> xs;                 // [n_seg * n_xs] (empty when built on the device)
+  std::vector<double> xw;                 // [n_seg * kXwStride] (empty when built on the device)
   std::vector<double> diag_lo;         // [2^B] site + low-low bond diagonal
   std::vector<double> diag_hi;         // [2^NH] site + high-high bond diagonal + every cross bond's par value
   std::vector<FlipBond> ll, hh;        // low-low and high-high flip bonds
@@ -460,7 +467,7 @@ inline void cross_stages(uint32_t h, const uint32_t* hi_base, const XSource& X, 
   for (; n < X.ng; ++n) out[n] = XStage{0u, 0u};
 }
 
-// Entry p of xw[h]: a cross bond is antiparallel where the low bit differs
+// Entry p of the xw of high word h: a cross bond is antiparallel where the low bit differs
 // from the high one.
 #ifdef __HIPCC__
 __host__ __device__
@@ -781,15 +788,19 @@ inline SectorLayout build_layout(const ModelSpec& m, int B_override = -1, bool c
     w[B] += x.e_anti - x.e_par;
   }
   L.stage = !L.ranked && stage_cross(B, L.xb.size(), L.xb_grp.size());
+  if (L.stage) {
+    std::vector<uint32_t> at(nhi);
+    for (size_t q = 0; q < L.seg_hi.size(); ++q) at[L.seg_hi[q]] = (uint32_t)q;
+    for (uint32_t h : L.proc_hi) L.proc_index.push_back(at[h]);
+  }
   if (host_lists && L.stage) {
     const XSource X{L.xb_grp.data(), L.xb_w.data(), (int)L.xb_grp.size(), B};
-    L.xs.assign((size_t)nhi * L.xb_grp.size(), XStage{0u, 0u});
-    L.xw.assign((size_t)nhi * kXwStride, 0.0);
-    for (uint32_t h = 0; h < nhi; ++h)
-      if (L.hi_base[h] != 0xffffffffu) {
-        cross_stages(h, L.hi_base.data(), X, L.xs.data() + (size_t)h * X.ng);
-        for (int p = 0; p <= B; ++p) L.xw[(size_t)h * kXwStride + p] = cross_weight(h, p, X);
-      }
+    L.xs.assign(L.seg_hi.size() * X.ng, XStage{0u, 0u});
+    L.xw.assign(L.seg_hi.size() * kXwStride, 0.0);
+    for (size_t q = 0; q < L.seg_hi.size(); ++q) {
+      cross_stages(L.seg_hi[q], L.hi_base.data(), X, L.xs.data() + q * X.ng);
+      for (int p = 0; p <= B; ++p) L.xw[q * kXwStride + p] = cross_weight(L.seg_hi[q], p, X);
+    }
   }
   const bool host_nb = host_lists && (copy_shared || !L.stage);
   if (host_nb) L.xb_nb.assign((size_t)nhi * L.n_xb_p, 0u);

@@ -1,5 +1,6 @@
 // Host checks of what the H.v kernels read of a layout (no device).  Each
 // check prints "<name> <mismatches> <checked>".
+#include <cmath>
 #include <cstdio>
 #include <random>
 
@@ -74,8 +75,94 @@ static void segment_order() {
   report("segment_order", bad, n);
 }
 
+// The first row of the segment of a high word: the rank of its smallest state.
+static uint32_t first_row(const SectorLayout& L, uint32_t h) {
+  const int kl = L.k - __builtin_popcount(h);
+  if (kl < 0 || kl > L.B) return 0xffffffffu;
+  const uint32_t st = (h << L.B) | ((1u << kl) - 1u);
+  uint64_t r = 0;
+  int m = 0;
+  for (int p = 0; p < L.N; ++p)
+    if (st >> p & 1u) r += binom(p, ++m);
+  return (uint32_t)r;
+}
+
+// Page positions are linear over xor and distinct for words of one parity.
+static void page_positions() {
+  long bad = 0, n = 0;
+  for (int B = 1; B <= 12; ++B) {
+    const uint32_t nlo = 1u << B, np = std::max(1u, nlo / 2);
+    std::vector<int> seen(2 * np, 0);
+    for (uint32_t a = 0; a < nlo; ++a, ++n) {
+      const uint32_t at = page_pos(a);
+      bad += at >= np || seen[(__builtin_popcount(a) & 1) * np + at]++ != 0;
+      for (int p = 0; p < B; ++p) bad += page_pos(a ^ (1u << p)) != (at ^ page_pos(1u << p));
+    }
+    const LowTables& T = low_tables(B);
+    for (uint32_t i = 0; i < nlo; ++i) bad += T.lo_word[i] != T.lo_state[i] || T.lo_page[i] != 8 * page_pos(T.lo_state[i]);
+  }
+  report("page_positions", bad, n);
+}
+
+// What a segment stages for the cross bonds, and their share of its rows'
+// diagonal, against the bonds: one entry per segment, so that sectors of few
+// up spins among many high words stay small.
+static void cross_stages_of_segments() {
+  long bad = 0, n = 0;
+  std::mt19937 rng(3);
+  std::uniform_real_distribution<double> U(-1, 1);
+  const int cases[][2] = {{14, 7}, {16, 8}, {17, 3}, {20, 10}, {20, 2}, {20, 18}, {22, 11}, {24, 2}};
+  for (const auto& c : cases) {
+    ModelSpec s = ring(c[0], c[1]);
+    const int high = c[0] - 12;
+    for (int b = 0; b < 8 * high; ++b)
+      s.bonds.push_back(make_bond((int)(rng() % high), high + (int)(rng() % 12), U(rng), U(rng), U(rng)));
+    const SectorLayout L = build_layout(s, -1, false, true);
+    const size_t ng = L.xb_grp.size(), ns = L.seg_hi.size();
+    bad += !L.stage || L.xs.size() != ns * ng || L.xw.size() != ns * kXwStride || !L.xb_nb.empty();
+    if (bad) break;
+    for (size_t q = 0; q < ns; ++q) {
+      const uint32_t h = L.seg_hi[q];
+      bad += L.seg_hi[L.proc_index[q]] != L.proc_hi[q];
+      size_t i = 0;
+      for (int set = 1; set >= 0; --set)
+        for (uint32_t bit = 1; bit < (1u << L.NH); bit <<= 1) {
+          size_t b0 = 0, b1 = 0;
+          for (size_t b = 0; b < L.xb.size(); ++b)
+            if (L.xb[b].hbit == bit) {
+              if (b1 == 0) b0 = b;
+              b1 = b + 1;
+            }
+          const uint32_t nb = first_row(L, h ^ bit);
+          if (b1 == 0 || ((h & bit) != 0u) != (set == 1) || nb == 0xffffffffu) continue;
+          const XStage st = L.xs[q * ng + i++];
+          bad += st.nb != nb || (int)(st.info >> 31) != set || (st.info & 0xffffu) != b0 ||
+                 (st.info >> 16 & 0x7fffu) != b1 - b0;
+          ++n;
+        }
+      for (; i < ng; ++i) bad += L.xs[q * ng + i].info != 0u;
+      const int kl = L.k - __builtin_popcount(h);
+      for (uint32_t r = L.lo_class_off[kl]; r < L.lo_class_off[kl + 1]; r += 1 + rng() % 64) {
+        const uint32_t lo = L.low->lo_state[r];
+        double want = 0, got = L.xw[q * kXwStride + L.B];
+        for (const CrossBond& x : L.xb)
+          if (((lo & x.lbit) != 0u) != ((h & x.hbit) != 0u)) want += x.e_anti - x.e_par;
+        for (int p = 0; p < L.B; ++p)
+          if (lo >> p & 1u) got += L.xw[q * kXwStride + p];
+        bad += !(std::abs(got - want) < 1e-11);  // at most 112 terms below 2, added twice
+        ++n;
+      }
+    }
+    for (size_t b = 0; b < L.xb.size(); ++b)
+      bad += L.xb_p[b].t != L.xb[b].t || L.xb_p[b].m != 8 * page_pos(L.xb[b].lbit);
+  }
+  report("cross_stages", bad, n);
+}
+
 int main() {
   shared_low_table();
   segment_order();
+  page_positions();
+  cross_stages_of_segments();
   return 0;
 }
