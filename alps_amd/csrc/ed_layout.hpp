@@ -772,7 +772,6 @@ inline SectorLayout build_layout(const ModelSpec& m, int B_override = -1, bool c
   }
   L.xb_hbit.assign(L.n_xb_p, 0u);
   for (size_t b = 0; b < L.xb.size(); ++b) L.xb_hbit[b] = L.xb[b].hbit;
-  if (L.xb.size() >= 0x7fffu) throw std::invalid_argument("too many cross bonds");
   L.xb_c.assign(L.n_xb_p, XBondConst{0.0, 0.0, 0u, 0u});
   for (size_t b = 0; b < L.xb.size(); ++b) {
     const CrossBond& x = L.xb[b];
@@ -787,7 +786,8 @@ inline SectorLayout build_layout(const ModelSpec& m, int B_override = -1, bool c
     w[__builtin_ctz(x.lbit)] += x.e_anti - x.e_par;
     w[B] += x.e_anti - x.e_par;
   }
-  L.stage = !L.ranked && stage_cross(B, L.xb.size(), L.xb_grp.size());
+  // (XStage packs the bonds of a stage into 16 + 15 bits)
+  L.stage = !L.ranked && L.xb.size() <= 0x7fffu && stage_cross(B, L.xb.size(), L.xb_grp.size());
   if (L.stage) {
     std::vector<uint32_t> at(nhi);
     for (size_t q = 0; q < L.seg_hi.size(); ++q) at[L.seg_hi[q]] = (uint32_t)q;

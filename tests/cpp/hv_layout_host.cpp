@@ -159,7 +159,29 @@ static void cross_stages_of_segments() {
   report("cross_stages", bad, n);
 }
 
+// Any number of cross bonds has a layout; more than a stage can name are
+// gathered.
+static void many_cross_bonds() {
+  long bad = 0, n = 0;
+  for (int count : {0x7fff, 0x8000}) {
+    ModelSpec s;
+    s.n_sites = 14;
+    s.n_up = 7;
+    for (int i = 0; i < 14; ++i) s.sites.push_back(make_site(0.0, 0.0));
+    for (int b = 0; b < count; ++b) s.bonds.push_back(make_bond(b & 1, 2 + b % 12, 1.0, 1.0, 0.0));
+    try {
+      const SectorLayout L = build_layout(s, -1, false);
+      bad += L.stage != (count <= 0x7fff) || L.xb.size() != (size_t)count;
+    } catch (const std::exception&) {
+      ++bad;
+    }
+    ++n;
+  }
+  report("many_cross_bonds", bad, n);
+}
+
 int main() {
+  many_cross_bonds();
   shared_low_table();
   segment_order();
   page_positions();

@@ -6,7 +6,7 @@ import subprocess
 import pytest
 
 BIN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "_build", "hv_layout_host")
-CHECKS = ["shared_low_table", "segment_order", "page_positions", "cross_stages"]
+CHECKS = ["shared_low_table", "segment_order", "page_positions", "cross_stages", "many_cross_bonds"]
 
 
 @pytest.fixture(scope="module")
