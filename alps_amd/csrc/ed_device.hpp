@@ -228,6 +228,22 @@ __device__ __forceinline__ void update_sums(double& a, double& b) {
   }
 }
 
+// The sum of v over a workgroup of NT threads, in wave order, to
+// out[blockIdx.x].  Once per kernel.
+template <int NT>
+__device__ __forceinline__ void store_update_partial(double* out, double v) {
+  __shared__ double red_out[NT / 64];
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red_out[threadIdx.x >> 6] = v;
+  lds_barrier();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+#pragma unroll
+    for (int q = 0; q < NT / 64; ++q) s += red_out[q];
+    out[blockIdx.x] = s;
+  }
+}
+
 // The workgroup's (NT threads) part of clearing the page of B low bits.
 template <int NT>
 __device__ __forceinline__ void clear_page(int B) {

@@ -60,3 +60,11 @@ def test_every_schedule_is_a_kernel():
     ks = [n for n in kernels() if "9hv_kernelIf" in n or "hv_ranked_kernelIf" in n]
     assert sum("hv_ranked_kernelIf" in n for n in ks) == 2 * A.Operator.HV_SCHEDULES
     assert sum("9hv_kernelIf" in n for n in ks) == 4 * (A.Operator.HV_SCHEDULES + 1)
+
+
+def test_reorthogonalization_launches_the_updates_threads():
+    # its grid is the update's (one norm partial per block): so are its blocks
+    ks = kernels()
+    sizes = {kind: {k[".max_flat_workgroup_size"] for n, k in ks.items() if kind in n}
+             for kind in ("update_fused_kernel", "reorth_update_kernel")}
+    assert sizes["update_fused_kernel"] == sizes["reorth_update_kernel"] != set()
