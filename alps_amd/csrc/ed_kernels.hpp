@@ -161,14 +161,19 @@ constexpr HvSchedule kHvSchedule[kHvSchedules] = {{8, 2, 4}, {8, 1, 4}, {8, 4, 4
 // Layouts of at most kFewSegments segments take 512 threads a workgroup
 // instead of kBlock, whatever the schedule.  Layouts with low-low target
 // tables (DevLayout::nbp16) have six of their own, with the cross bonds per
-// chunk: the best of them over the first, us: 24-site J1-J2 (width 3) 8 up
-// 19.9 and 20.5 (schedule 4), 27 sites 9 up 126.1 and 130.5 (4), 23-site ring
-// 8 up 5.13 and 5.19 (3).
+// chunk, all of 8 waves: the form with the dot partials, which the recurrences
+// launch and the tuner does not time, is much slower compiled for 6 or 7 (27-
+// site J1-J2 9 up: product 130 us with 8 waves, 137 with 6, a step of the
+// recurrence 183 and 197 us; 23-site ring 8 up 5.28 and 5.25, 13.4 and 14.3).
+// The best over the first, product and step, us: that J1-J2 sector 130 and
+// 125, 184 and 182.5 (8, 8, 4, 4); 24 sites (width 4) 8 up 22.7 and 21.7, 34.7
+// and 33.6, 25 sites 8 up 41.2 and 38.4, 58.8 and 55.7 (8, 4, 4, 4); on rings
+// the first.
 struct HvRankedSchedule {
   int waves, cll, chh, cx;
 };
-constexpr HvRankedSchedule kHvRankedSchedule[kHvSchedules] = {{8, 4, 4, 2}, {8, 4, 8, 2}, {6, 4, 8, 2},
-                                                              {6, 4, 4, 2}, {8, 8, 4, 2}, {6, 8, 8, 4}};
+constexpr HvRankedSchedule kHvRankedSchedule[kHvSchedules] = {{8, 4, 4, 2}, {8, 4, 8, 2}, {8, 4, 4, 4},
+                                                              {8, 4, 8, 4}, {8, 8, 4, 2}, {8, 8, 4, 4}};
 
 // y = H x; with dot_out set, per-block partials of sum_i x_i (H x)_i (FP64,
 // before y is rounded to the storage type).
