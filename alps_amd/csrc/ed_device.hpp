@@ -489,7 +489,7 @@ __device__ __forceinline__ double hv_rows(const DevLayout& L, const SegRec& S, c
     if (tid < 128u) {
       const uint32_t hf = __builtin_amdgcn_readfirstlane(tid >> 6);
       const double* w = L.xw + (size_t)S.h_or_index * kXwStride;
-      double s = hf ? S.dh : ldc(w + L.B);
+      double s = hf ? S.dh_page : ldc(w + L.B);
 #pragma unroll
       for (uint32_t p = 0; p < 6u; ++p) s = fma((tid >> p & 1u) ? 1.0 : 0.0, ldc(w + 6u * hf + p), s);
       lds_st<double>(8u * tid, s);
@@ -516,7 +516,7 @@ __device__ __forceinline__ double hv_rows(const DevLayout& L, const SegRec& S, c
     const uint32_t lo_x = lane_off(2u * ((tid >> 6) * 64u * (uint32_t)L.n_xb_p + (tid & 63u) * kXChunk));
     const uint32_t x_slot = (uint32_t)NT * (uint32_t)L.n_xb_p;  // u16 entries per slot
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) d[q] = S.dh;
+    for (int q = 0; q < NQ; ++q) d[q] = S.dh_page;
     const uint32_t h = S.h_or_index;  // not staged: the high word
     const uint32_t* xnb = L.xb_nb + h * (uint32_t)L.n_xb_p;
     for (int b0 = 0; NQ > 0 && b0 < L.n_xb; b0 += kXChunk) {
@@ -627,9 +627,10 @@ __device__ __forceinline__ void hv_segment_at(const DevLayout& L, const SegRec& 
 // sites 7 up 4.69 -> 4.54 and 5.44 -> 5.30, 27-site J1-J2 9 up 132.5 -> 130.6
 // and 181.3 -> 180.2.
 template <class V, bool DOT, int NQ, int CLL, int CHH, int CX>
-__device__ __forceinline__ double hv_ranked_rows(const DevLayout& L, const SegHead& S, double dh,
-                                                 const V* __restrict__ x, V* __restrict__ y) {
+__device__ __forceinline__ double hv_ranked_rows(const DevLayout& L, const SegHead& S, const V* __restrict__ x,
+                                                 V* __restrict__ y) {
   const uint32_t h = S.h_or_index, len = S.len, base = S.base, e0 = S.e0, e1 = S.e1;
+  const double dh = S.dh;
   const uint16_t* nbp = L.nbp16 + S.nbp;
   const uint16_t* xnp = L.xn16 + S.xnp;
   const double* dlp = L.diag_lo_cls + S.cls0;
@@ -821,18 +822,17 @@ __device__ __forceinline__ double hv_ranked_rows(const DevLayout& L, const SegHe
 // The same workgroup and slots as hv_segment_at; dynamic LDS of max_seg + 1
 // doubles.
 template <class V, bool DOT, int CLL = 4, int CHH = 4, int CX = 2>
-__device__ __forceinline__ void hv_ranked_at(const DevLayout& L, const SegHead& S, double dh,
-                                             const V* __restrict__ x, V* __restrict__ y,
-                                             double* __restrict__ dot_slot) {
+__device__ __forceinline__ void hv_ranked_at(const DevLayout& L, const SegHead& S, const V* __restrict__ x,
+                                             V* __restrict__ y, double* __restrict__ dot_slot) {
   const uint32_t w0 = threadIdx.x & ~63u;
   const uint32_t nq = __builtin_amdgcn_readfirstlane(S.len > w0 ? (S.len - w0 + kBlock - 1) / kBlock : 0u);
   static_assert(kMaxSegRows == 4 * kBlock, "one to four row slots");
   double dotp = 0.0;
   if (nq == 0) lds_barrier();
-  else if (nq == 1) dotp = hv_ranked_rows<V, DOT, 1, CLL, CHH, CX>(L, S, dh, x, y);
-  else if (nq == 2) dotp = hv_ranked_rows<V, DOT, 2, CLL, CHH, CX>(L, S, dh, x, y);
-  else if (nq == 3) dotp = hv_ranked_rows<V, DOT, 3, CLL, CHH, CX>(L, S, dh, x, y);
-  else dotp = hv_ranked_rows<V, DOT, 4, CLL, CHH, CX>(L, S, dh, x, y);
+  else if (nq == 1) dotp = hv_ranked_rows<V, DOT, 1, CLL, CHH, CX>(L, S, x, y);
+  else if (nq == 2) dotp = hv_ranked_rows<V, DOT, 2, CLL, CHH, CX>(L, S, x, y);
+  else if (nq == 3) dotp = hv_ranked_rows<V, DOT, 3, CLL, CHH, CX>(L, S, x, y);
+  else dotp = hv_ranked_rows<V, DOT, 4, CLL, CHH, CX>(L, S, x, y);
   if (DOT) {
     lds_barrier();  // every wave is done with the slice
     store_block_sum_lds<kBlock>(dot_slot, dotp);
@@ -857,7 +857,7 @@ __device__ __forceinline__ SegRec seg_record(const DevLayout& L, uint32_t seg) {
   S.xnp = ldc(L.xn_off + kl);
   S.nbp = L.nbp16 ? ldc(L.nbp_off + kl) : 0u;
   S.dh = ldc(L.diag_hi + h);
-  S.pad = 0.0;
+  S.dh_page = S.dh;
   return S;
 }
 

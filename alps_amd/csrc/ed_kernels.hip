@@ -47,8 +47,7 @@ __global__ __launch_bounds__(NT, W) void hv_kernel(DevLayout L, const V* __restr
 template <class V, bool DOT, int W, int CLL, int CHH, int CX>
 __global__ __launch_bounds__(kBlock, W) void hv_ranked_kernel(DevLayout L, const V* __restrict__ x,
                                                               V* __restrict__ y, double* __restrict__ dot_out) {
-  const SegRec* rec = L.seg_rec + blockIdx.x;
-  hv_ranked_at<V, DOT, CLL, CHH, CX>(L, ldc_struct<SegHead>(rec), ldc(&rec->dh), x, y,
+  hv_ranked_at<V, DOT, CLL, CHH, CX>(L, ldc_struct<SegHead>(L.seg_rec + blockIdx.x), x, y,
                                      DOT ? dot_out + blockIdx.x : nullptr);
 }
 

@@ -14,7 +14,7 @@ struct DevLayout {
   int N, k, B, NH;
   uint32_t D;
   uint32_t n_seg, max_seg;
-  int n_bonds;
+  int n_ll_p;                 // entries per row of nbp16
   int n_ll, n_xb, n_xb_p;     // low-low and cross flip bonds; the cross tables' stride
   int n_xs;                   // high bits with staged cross bonds; 0: gathered
   const uint32_t* lo_rank;
@@ -53,11 +53,12 @@ struct DevLayout {
   const double* bond_par;
   const double* bond_anti;
   const double* bond_t;
+  int n_bonds;
+  // [n_seg] per processing index: the segment's position in seg_hi (staged).
   // Behind what the page kernel reads, whose wide argument loads are sensitive
-  // to what lies between (24-site J1-J2 in FP32: 44.5 us, 44.9 with these two
+  // to what lies between (24-site J1-J2 in FP32: 44.5 us, 44.9 with this one
   // among the others).
-  const uint32_t* proc_index;  // [n_seg] per processing index: the segment's position in seg_hi (staged)
-  int n_ll_p;                  // entries per row of nbp16
+  const uint32_t* proc_index;
 };
 
 // A momentum sector (Bloch basis, ed_bloch.hpp) on the device.  Vectors of

@@ -152,19 +152,24 @@ struct PageBond {
 // processing index (built on the device for a single operator): its high
 // word or, with staged cross bonds, whose tables go by it, its position in
 // seg_hi; its first row, class offset and length, the range of its listed
-// high-high flips, the flip-table offsets, the offset and length of the
-// classes with one low bit more and one fewer (the segments across a cross
-// bond; only staged bonds need them), and the high word's diagonal.  Read with
-// scalar loads instead of two dependent rounds of table reads; the first field
-// is one that every kernel uses, so that the load stays whole (20-site J1-J2:
-// 10.2 us, 10.4 with the position in the place of nbp).
+// high-high flips, the flip-table offsets, the high word's diagonal, and the
+// offset and length of the classes with one low bit more and one fewer (the
+// segments across a cross bond; only staged bonds need them).  Read with
+// scalar loads instead of two dependent rounds of table reads.
+// The order follows the loads: the first field is one that every kernel uses,
+// so that the page kernel's one load stays whole (20-site J1-J2: 10.2 us, 10.4
+// with the position in the place of nbp); the table kernel reads the head
+// alone (22-site ring 8 up, FP32: 4.40 us, 4.45 with the diagonal behind the
+// classes), and the page kernel the copy of the diagonal at the end (24-site
+// J1-J2, FP32: 44.5 us, 45.0 with the one in the head).
 struct SegHead {
   uint32_t h_or_index, base, cls0, len;
   uint32_t e0, e1, xnp, nbp;
+  double dh;
 };
 struct SegRec : SegHead {
   uint32_t cls_up, len_up, cls_dn, len_dn;
-  double dh, pad;
+  double dh_page;
 };
 static_assert(sizeof(SegRec) == 64, "one scalar load of 16 registers");
 
