@@ -179,6 +179,12 @@ struct SharedTables {
   const uint16_t *lo_page = nullptr, *lo_word = nullptr, *xn16 = nullptr;
 };
 
+// Device copy of a low-low target table (low_flip_table).
+struct LowTable {
+  DevBuf buf;
+  std::shared_ptr<const std::vector<uint16_t>> keep;  // keeps the key alive
+};
+
 enum State { kPending, kRunning, kRefining, kDone };
 
 struct Problem {
@@ -223,8 +229,12 @@ struct Problem {
   double t_submit = 0, t_admit = 0, t_done = 0;
   bool sized = false;  // layout built
   alps_ed_solve_result result{};
-  // Which of the H.v launches its items belong to (launch_batch_hv).
-  bool staged() const { return !trans && layout.stage; }
+  // Which of the H.v launches its items belong to.
+  BatchHv form() const {
+    if (trans) return kHvGathered;
+    const bool tables = layout.ranked && layout.n_ll_p > 0 && layout.D < kBatchTableRows * layout.seg_hi.size();
+    return layout.stage ? kHvStaged : tables ? kHvTables : kHvGathered;
+  }
   // Whether its updates form the scalars of a step.
   bool fused() const { return n_hv + n_chunks <= kBatchFuse; }
 };
@@ -270,6 +280,7 @@ struct alps_ed_batch_s {
   size_t rdev_cap = 0;
   // shared low-word and flip tables, one device copy per lattice topology
   std::map<std::pair<const void*, const void*>, std::unique_ptr<SharedTables>> shared;
+  std::map<const void*, std::unique_ptr<LowTable>> low_tables;
 
   ~alps_ed_batch_s() {
     if (stream64) (void)hipStreamSynchronize(stream64);
@@ -299,6 +310,8 @@ size_t table_bytes(const SectorLayout& L) {
   add(L.diag_lo_cls.size(), 8);
   add(L.diag_hi.size(), 8);
   add(L.ll_c.size(), sizeof(PageBond));
+  add(L.nbp_off.size(), 4);
+  add(L.ll_t.size(), 8);
   add(L.hh_off.size(), 4);
   add(L.hh_ent.size(), sizeof(HHEntry));
   add(L.xb_c.size(), sizeof(XBondConst));
@@ -330,7 +343,8 @@ size_t problem_table_bytes(const Problem& p) { return table_bytes(p.layout) + bl
 // Lays the tables out at [base, base + table_bytes) of the device, writing
 // their bytes to the same offsets of the host staging area `stage`, and
 // returns the device layout; one copy of the staging area uploads them.
-DevLayout place_tables(const SectorLayout& L, char* base, char* stage, const SharedTables& sh) {
+DevLayout place_tables(const SectorLayout& L, char* base, char* stage, const SharedTables& sh,
+                       const uint16_t* nbp16) {
   DevLayout d{};
   d.N = L.N;
   d.k = L.k;
@@ -344,6 +358,8 @@ DevLayout place_tables(const SectorLayout& L, char* base, char* stage, const Sha
   d.n_xb_p = L.n_xb_p;
   d.n_xs = L.stage ? (int)L.xb_grp.size() : 0;
   d.n_bonds = (int)L.bond_p1.size();
+  d.n_ll_p = L.n_ll_p;
+  d.nbp16 = nbp16;
   d.lo_rank = sh.lo_rank;
   d.lo_state = sh.lo_state;
   d.lo_class_off = sh.lo_class_off;
@@ -366,6 +382,8 @@ DevLayout place_tables(const SectorLayout& L, char* base, char* stage, const Sha
   d.diag_lo_cls = put(L.diag_lo_cls);
   d.diag_hi = put(L.diag_hi);
   d.ll_c = put(L.ll_c);
+  d.nbp_off = put(L.nbp_off);
+  d.ll_t = put(L.ll_t);
   d.hh_off = put(L.hh_off);
   d.hh_ent = put(L.hh_ent);
   d.xb_c = put(L.xb_c);
@@ -427,11 +445,11 @@ T* dev_ptr(alps_ed_batch b, size_t off) {
 
 // Places an admitted problem in its regions; its tables are staged at
 // `stage` (table_bytes of them) for the caller to upload.
-void place(alps_ed_batch b, Problem& p, char* stage, const SharedTables& sh) {
+void place(alps_ed_batch b, Problem& p, char* stage, const SharedTables& sh, const uint16_t* nbp16) {
   char* base = static_cast<char*>(b->dev_base) + p.dev_off;
   BatchJob& J = p.job;
   J = BatchJob{};
-  J.L = place_tables(p.layout, base, stage, sh);
+  J.L = place_tables(p.layout, base, stage, sh, nbp16);
   if (!p.bloch.rep_state.empty()) {  // the momentum sector's basis after the layout tables
     size_t o = table_bytes(p.layout);
     auto put = [&](const auto& v) {
@@ -627,8 +645,8 @@ void ensure_stage(alps_ed_batch b, size_t bytes) {
 // Copies jobs, work items and the job list of a launch group to the device.
 struct Group {
   BatchJob* jobs = nullptr;
-  BatchItem* hv32[2] = {nullptr, nullptr};  // gathered, staged (Problem::staged)
-  BatchItem* hv64[2] = {nullptr, nullptr};
+  BatchItem* hv32[kBatchHvForms] = {};  // by Problem::form
+  BatchItem* hv64[kBatchHvForms] = {};
   BatchItem* up32 = nullptr;
   BatchItem* up64 = nullptr;
   BatchItem* st32 = nullptr;  // start-vector items of the problems new this round
@@ -636,7 +654,7 @@ struct Group {
   uint32_t* list = nullptr;     // fused jobs
   uint32_t* big_list = nullptr; // the others
   uint32_t* st_list = nullptr;  // and those of them new this round
-  uint32_t n_hv32[2] = {0, 0}, n_hv64[2] = {0, 0};
+  uint32_t n_hv32[kBatchHvForms] = {}, n_hv64[kBatchHvForms] = {};
   uint32_t n_up32 = 0, n_up64 = 0, n_list = 0, n_big_list = 0, n_st32 = 0, n_st64 = 0,
            n_st_list = 0;
   uint32_t lds32 = kHvMinLds, lds64 = kHvMinLds;  // the largest LDS need of an H.v item
@@ -650,10 +668,10 @@ Group upload_group(alps_ed_batch b, const std::vector<Problem*>& run) {
   // new this round, then the job list and the new jobs' list.
   Group g;
   const size_t nj = run.size();
-  size_t n_hv[2][2] = {{0, 0}, {0, 0}}, n_up[2] = {0, 0}, n_st[2] = {0, 0};
+  size_t n_hv[2][kBatchHvForms] = {}, n_up[2] = {0, 0}, n_st[2] = {0, 0};
   for (const Problem* p : run) {
     const int f = p->fp32 ? 1 : 0;
-    n_hv[f][p->staged()] += p->n_hv;
+    n_hv[f][p->form()] += p->n_hv;
     n_up[f] += p->n_chunks;
     if (p->j == 0) {
       n_st[f] += p->n_chunks;
@@ -666,8 +684,9 @@ Group upload_group(alps_ed_batch b, const std::vector<Problem*>& run) {
   auto ib = [](size_t n) { return align_up((n + 1) * sizeof(BatchItem)); };
   const size_t bj = align_up(nj * sizeof(BatchJob));
   const size_t bl = align_up((nj + 1) * sizeof(uint32_t));
-  const size_t total = bj + ib(n_hv[1][0]) + ib(n_hv[1][1]) + ib(n_hv[0][0]) + ib(n_hv[0][1]) + ib(n_up[1]) +
-                       ib(n_up[0]) + ib(n_st[1]) + ib(n_st[0]) + 2 * bl;
+  size_t total = bj + ib(n_up[1]) + ib(n_up[0]) + ib(n_st[1]) + ib(n_st[0]) + 2 * bl;
+  for (const auto& f : n_hv)
+    for (size_t n : f) total += ib(n);
   ensure_buf(b->jobs_d, b->jobs_cap, total);
   ensure_stage(b, total);
   char* s = static_cast<char*>(b->stage);
@@ -682,10 +701,10 @@ Group upload_group(alps_ed_batch b, const std::vector<Problem*>& run) {
     o += ib(n);
     return h;
   };
-  BatchItem* hv32[2];
-  BatchItem* hv64[2];
-  for (int s = 0; s < 2; ++s) hv32[s] = region(n_hv[1][s], g.hv32[s], g.n_hv32[s]);
-  for (int s = 0; s < 2; ++s) hv64[s] = region(n_hv[0][s], g.hv64[s], g.n_hv64[s]);
+  BatchItem* hv32[kBatchHvForms];
+  BatchItem* hv64[kBatchHvForms];
+  for (int s = 0; s < kBatchHvForms; ++s) hv32[s] = region(n_hv[1][s], g.hv32[s], g.n_hv32[s]);
+  for (int s = 0; s < kBatchHvForms; ++s) hv64[s] = region(n_hv[0][s], g.hv64[s], g.n_hv64[s]);
   BatchItem* up32 = region(n_up[1], g.up32, g.n_up32);
   BatchItem* up64 = region(n_up[0], g.up64, g.n_up64);
   BatchItem* st32 = region(n_st[1], g.st32, g.n_st32);
@@ -698,7 +717,7 @@ Group upload_group(alps_ed_batch b, const std::vector<Problem*>& run) {
   g.st_list = reinterpret_cast<uint32_t*>(d + o);
   for (uint32_t i = 0; i < nj; ++i) {
     const Problem& p = *run[i];
-    BatchItem*& hv = (p.fp32 ? hv32 : hv64)[p.staged()];
+    BatchItem*& hv = (p.fp32 ? hv32 : hv64)[p.form()];
     BatchItem*& up = p.fp32 ? up32 : up64;
     for (uint32_t sg = 0; sg < p.n_hv; ++sg) *hv++ = {i, sg};
     for (uint32_t c = 0; c < p.n_chunks; ++c) *up++ = {i, c};
@@ -778,6 +797,21 @@ const SharedTables& shared_tables(alps_ed_batch b, const SectorLayout& L) {
   return t;
 }
 
+// That of a problem's low-low target table, null where its form has none.
+const uint16_t* low_table(alps_ed_batch b, const Problem& p) {
+  if (p.form() != kHvTables) return nullptr;
+  std::shared_ptr<const std::vector<uint16_t>> t = low_flip_table(p.layout);
+  std::unique_ptr<LowTable>& slot = b->low_tables[t.get()];
+  if (!slot) {
+    slot.reset(new LowTable);
+    slot->keep = t;
+    slot->buf.alloc(t->size() * sizeof(uint16_t));
+    hip_check(hipMemcpyAsync(slot->buf.p, t->data(), t->size() * sizeof(uint16_t), hipMemcpyHostToDevice, b->stream),
+              "upload low-low table");
+  }
+  return slot->buf.as<uint16_t>();
+}
+
 void ensure_tstage(alps_ed_batch b, size_t bytes) {
   if (bytes <= b->tstage_cap) return;
   if (b->tstage) hip_check(hipHostFree(b->tstage), "hipHostFree");
@@ -847,8 +881,12 @@ void admit(alps_ed_batch b, std::vector<Problem*>& started) {
   ensure_tstage(b, stage_bytes);
   char* st = static_cast<char*>(b->tstage);
   std::vector<const SharedTables*> sh(placed.size());
-  for (size_t i = 0; i < placed.size(); ++i) sh[i] = &shared_tables(b, placed[i]->layout);
-  b->pool->parallel_for(placed.size(), [&](size_t i) { place(b, *placed[i], st + at[i], *sh[i]); });
+  std::vector<const uint16_t*> lt(placed.size());
+  for (size_t i = 0; i < placed.size(); ++i) {
+    sh[i] = &shared_tables(b, placed[i]->layout);
+    lt[i] = low_table(b, *placed[i]);
+  }
+  b->pool->parallel_for(placed.size(), [&](size_t i) { place(b, *placed[i], st + at[i], *sh[i], lt[i]); });
   ScatterItem* items = reinterpret_cast<ScatterItem*>(st + items_at);
   for (size_t i = 0; i < placed.size(); ++i)
     items[i] = ScatterItem{at[i], problem_table_bytes(*placed[i]), static_cast<char*>(b->dev_base) + placed[i]->dev_off};
@@ -1081,9 +1119,10 @@ void round(alps_ed_batch b) {
         hip_check(hipStreamWaitEvent(st64, b->fork->e, 0), "event");
       }
       for (int t = 0; t < S; ++t) {
-        for (int s = 0; s < 2; ++s) {
-          hip_check(launch_batch_hv<float>(g.jobs, g.hv32[s], g.n_hv32[s], t, s == 1, g.lds32, b->stream), "batch hv");
-          hip_check(launch_batch_hv<double>(g.jobs, g.hv64[s], g.n_hv64[s], t, s == 1, g.lds64, st64), "batch hv");
+        for (int s = 0; s < kBatchHvForms; ++s) {
+          const BatchHv form = static_cast<BatchHv>(s);
+          hip_check(launch_batch_hv<float>(g.jobs, g.hv32[s], g.n_hv32[s], t, form, g.lds32, b->stream), "batch hv");
+          hip_check(launch_batch_hv<double>(g.jobs, g.hv64[s], g.n_hv64[s], t, form, g.lds64, st64), "batch hv");
         }
         hip_check(launch_batch_finish(g.jobs, g.big_list, g.n_big_list, t, kBatchAlpha, b->stream), "batch finish");
         hip_check(launch_batch_update<float>(g.jobs, g.up32, g.n_up32, t, b->stream), "batch update");
@@ -1101,10 +1140,10 @@ void round(alps_ed_batch b) {
     // a round that repeats the previous one replays them from a graph.
     bool replayed = false;
     if (b->cfg.graphs && g.n_st32 + g.n_st64 == 0) {
-      const std::vector<uint64_t> key{(uint64_t)g.jobs, (uint64_t)g.hv32[0], (uint64_t)g.hv32[1], (uint64_t)g.hv64[0],
-                                      (uint64_t)g.hv64[1], (uint64_t)g.up32, (uint64_t)g.up64, (uint64_t)g.list,
-                                      g.n_hv32[0], g.n_hv32[1], g.n_hv64[0], g.n_hv64[1], g.n_up32, g.n_up64,
-                                      g.n_list, g.n_big_list, g.lds32, g.lds64, (uint64_t)S};
+      std::vector<uint64_t> key{(uint64_t)g.jobs, (uint64_t)g.up32, (uint64_t)g.up64, (uint64_t)g.list, g.n_up32,
+                                g.n_up64, g.n_list, g.n_big_list, g.lds32, g.lds64, (uint64_t)S};
+      for (int s = 0; s < kBatchHvForms; ++s)
+        key.insert(key.end(), {(uint64_t)g.hv32[s], (uint64_t)g.hv64[s], g.n_hv32[s], g.n_hv64[s]});
       if (key == b->last_key) {
         if (!b->graph_exec || key != b->graph_key) {
           if (b->graph_exec) hip_check(hipGraphExecDestroy(b->graph_exec), "graph destroy");

@@ -98,9 +98,22 @@ enum { kBatchStart = 0, kBatchAlpha = 1, kBatchBeta = 2, kBatchLast = 3 };
 // launch_fill_random) with partials of |u_0|^2.
 template <class V>
 hipError_t launch_batch_start(const BatchJob* jobs, const BatchItem* items, uint32_t n_items, hipStream_t st);
+// The H.v launches of a step: problems with gathered cross bonds and momentum
+// sectors, with staged ones, and with low-low target tables (short segments:
+// ranked_rows, ed_layout.hpp).
+enum BatchHv { kHvGathered = 0, kHvStaged = 1, kHvTables = 2 };
+// Up to this many rows a segment on average a batched problem takes the tables;
+// beyond, the page with gathered cross bonds is as fast or faster here.  Whole
+// solves with the page and with the tables, FP32 and FP64, ms: 8 27-site J1-J2
+// sectors 6 up (17 rows) 89.0 and 86.6, 139.7 and 126.8; 24 22-site chains 6, 7
+// or 15 up (82 to 176 rows) 7.6 and 7.3, 12.3 and 11.8; 4 24-site J1-J2 8 up
+// (193) 15.6 and 15.6, 29.6 and 28.2; 8 24-site chains 8 up (193) 10.30 and
+// 10.09, 17.3 and 16.7; 4 24-site J1-J2 15 up (325) 15.6 and 16.1, 28.9 and 29.4.
+constexpr uint64_t kBatchTableRows = 250;
+constexpr int kBatchHvForms = 3;
 // Step t of a launch group: w = H u_j into slot j+1, alpha partials.
 template <class V>
-hipError_t launch_batch_hv(const BatchJob* jobs, const BatchItem* items, uint32_t n_items, int t, bool stage,
+hipError_t launch_batch_hv(const BatchJob* jobs, const BatchItem* items, uint32_t n_items, int t, BatchHv form,
                            uint32_t lds, hipStream_t st);
 // r = s_j w - alpha_j s_j u_j - beta_{j-1} s_{j-1} u_{j-1} in place of w; for
 // fused jobs with alpha_j, s_j and beta_{j-1} from the partials.

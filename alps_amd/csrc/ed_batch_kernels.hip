@@ -39,10 +39,9 @@ __global__ __launch_bounds__(kBlock) void batch_start_kernel(const BatchJob* __r
   if (threadIdx.x == 0) part[it.idx] = s;
 }
 
-// STAGE: the items' problems stage their cross bonds (n_xs > 0); the others,
-// and momentum sectors, have a launch of their own, so that neither variant's
-// code costs the other registers.
-template <class V, bool STAGE>
+// Each form has a launch of its own, so that none's code costs the others
+// registers.
+template <class V, BatchHv FORM>
 __global__ __launch_bounds__(kBlock, HvWaves<V>::value) void batch_hv_kernel(const BatchJob* __restrict__ jobs,
                                                           const BatchItem* __restrict__ items, int t) {
   const BatchItem it = ldc_struct(items + blockIdx.x);
@@ -56,13 +55,16 @@ __global__ __launch_bounds__(kBlock, HvWaves<V>::value) void batch_hv_kernel(con
   const V* x = slot_ptr<V>(vec, stride, cap, j);
   V* y = slot_ptr<V>(vec, stride, cap, j + 1);
   double* part = ldc(&J->part_hv);
-  if (!STAGE && ldc(&J->Bl.dk) != 0u) {  // momentum sector: uniform over the workgroup
+  if (FORM == kHvGathered && ldc(&J->Bl.dk) != 0u) {  // momentum sector: uniform over the workgroup
     const DevBloch Bl = ldc_struct(&J->Bl);
     const double p = bloch_row<V, true>(L, Bl, x, y, it.idx * kBlock + threadIdx.x);
     store_block_sum_lds<kBlock>(part + it.idx, p);
     return;
   }
-  hv_segment_at<V, true, STAGE>(L, seg_record(L, it.idx), x, y, part + it.idx);
+  if constexpr (FORM == kHvTables)
+    hv_ranked_at<V, true>(L, seg_record(L, it.idx, false, true), x, y, part + it.idx);
+  else
+    hv_segment_at<V, true, FORM == kHvStaged>(L, seg_record(L, it.idx, FORM == kHvStaged, false), x, y, part + it.idx);
 }
 
 // Where stage j (the start for j = 0, the update of step j - 1 otherwise)
@@ -303,9 +305,9 @@ __global__ __launch_bounds__(kBlock) void batch_plain_hv_kernel(const PlainHvJob
     return;
   }
   if (L.n_xs > 0)
-    hv_segment_at<double, true, true>(L, seg_record(L, it.idx), ldc(&J->x), ldc(&J->y), ldc(&J->part) + it.idx);
+    hv_segment_at<double, true, true>(L, seg_record(L, it.idx, true, false), ldc(&J->x), ldc(&J->y), ldc(&J->part) + it.idx);
   else
-    hv_segment_at<double, true, false>(L, seg_record(L, it.idx), ldc(&J->x), ldc(&J->y), ldc(&J->part) + it.idx);
+    hv_segment_at<double, true, false>(L, seg_record(L, it.idx, false, false), ldc(&J->x), ldc(&J->y), ldc(&J->part) + it.idx);
 }
 
 }  // namespace
@@ -318,13 +320,13 @@ hipError_t launch_batch_start(const BatchJob* jobs, const BatchItem* items, uint
 }
 
 template <class V>
-hipError_t launch_batch_hv(const BatchJob* jobs, const BatchItem* items, uint32_t n_items, int t, bool stage,
+hipError_t launch_batch_hv(const BatchJob* jobs, const BatchItem* items, uint32_t n_items, int t, BatchHv form,
                            uint32_t lds, hipStream_t st) {
   if (n_items == 0) return hipSuccess;
-  if (stage)
-    hipLaunchKernelGGL((batch_hv_kernel<V, true>), dim3(n_items), dim3(kBlock), lds, st, jobs, items, t);
-  else
-    hipLaunchKernelGGL((batch_hv_kernel<V, false>), dim3(n_items), dim3(kBlock), lds, st, jobs, items, t);
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(n_items), dim3(kBlock), lds, st, jobs, items, t); };
+  if (form == kHvTables) launch(batch_hv_kernel<V, kHvTables>);
+  else if (form == kHvStaged) launch(batch_hv_kernel<V, kHvStaged>);
+  else launch(batch_hv_kernel<V, kHvGathered>);
   return hipGetLastError();
 }
 
@@ -359,7 +361,7 @@ hipError_t launch_batch_plain_hv(const PlainHvJob* jobs, const BatchItem* items,
 
 #define ALPS_ED_BATCH_INSTANTIATE(V)                                                                           \
   template hipError_t launch_batch_start<V>(const BatchJob*, const BatchItem*, uint32_t, hipStream_t);       \
-  template hipError_t launch_batch_hv<V>(const BatchJob*, const BatchItem*, uint32_t, int, bool, uint32_t,   \
+  template hipError_t launch_batch_hv<V>(const BatchJob*, const BatchItem*, uint32_t, int, BatchHv, uint32_t, \
                                          hipStream_t);                                                       \
   template hipError_t launch_batch_update<V>(const BatchJob*, const BatchItem*, uint32_t, int, hipStream_t); \
   template hipError_t launch_batch_ritz<V>(const RitzJob*, const BatchItem*, uint32_t, hipStream_t);

@@ -839,12 +839,13 @@ __device__ __forceinline__ void hv_ranked_at(const DevLayout& L, const SegHead& 
   }
 }
 
-// The record of segment seg of the processing order, looked up in the tables.
-__device__ __forceinline__ SegRec seg_record(const DevLayout& L, uint32_t seg) {
+// The record of segment seg of the processing order, looked up in the tables
+// (staged: cross bonds staged; tables: low-low target tables).
+__device__ __forceinline__ SegRec seg_record(const DevLayout& L, uint32_t seg, bool staged, bool tables) {
   const uint32_t h = ldc(L.proc_hi + seg);
   const int kl = L.k - __builtin_popcount(h);
   SegRec S;
-  S.h_or_index = L.n_xs > 0 ? ldc(L.proc_index + seg) : h;
+  S.h_or_index = staged ? ldc(L.proc_index + seg) : h;
   S.base = ldc(L.hi_base + h);
   S.cls0 = ldc(L.lo_class_off + kl);
   S.cls_up = ldc(L.lo_class_off + kl + 1);
@@ -855,7 +856,7 @@ __device__ __forceinline__ SegRec seg_record(const DevLayout& L, uint32_t seg) {
   S.e0 = ldc(L.hh_off + h);
   S.e1 = ldc(L.hh_off + h + 1);
   S.xnp = ldc(L.xn_off + kl);
-  S.nbp = L.nbp16 ? ldc(L.nbp_off + kl) : 0u;
+  S.nbp = tables ? ldc(L.nbp_off + kl) : 0u;
   S.dh = ldc(L.diag_hi + h);
   S.dh_page = S.dh;
   return S;

@@ -55,7 +55,7 @@ __global__ __launch_bounds__(kBlock, W) void hv_ranked_kernel(DevLayout L, const
 __global__ __launch_bounds__(kBlock) void seg_rec_kernel(DevLayout L, SegRec* __restrict__ out) {
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= L.n_seg) return;
-  out[i] = seg_record(L, i);
+  out[i] = seg_record(L, i, L.n_xs > 0, L.nbp16 != nullptr);
 }
 
 template <class V, bool DOT, bool STAGE, int NT, int W, int CLL, int CHH>
