@@ -1108,11 +1108,17 @@ void round(alps_ed_batch b) {
       hip_check(launch_batch_start<double>(g.jobs, g.st64, g.n_st64, b->stream), "batch start");
       hip_check(launch_batch_finish(g.jobs, g.st_list, g.n_st_list, 0, kBatchStart, b->stream), "batch finish");
     }
+    // Without reduction launches the two precisions meet only at the end of
+    // the group, so the FP64 problems (small ones, a few wavefronts) run
+    // beside the FP32 ones on a stream of their own, made when it is first
+    // needed (here, not while the stream is captured).
+    const bool two = g.n_big_list == 0 && g.n_up32 != 0 && g.n_up64 != 0;
+    if (two && !b->stream64) {
+      b->fork.reset(new Event);
+      b->join.reset(new Event);
+      hip_check(hipStreamCreateWithFlags(&b->stream64, hipStreamNonBlocking), "hipStreamCreate");
+    }
     auto steps = [&] {
-      // Without reduction launches the two precisions meet only at the end
-      // of the group, so the FP64 problems (small ones, a few wavefronts)
-      // run beside the FP32 ones on a stream of their own.
-      const bool two = g.n_big_list == 0 && g.n_up32 != 0 && g.n_up64 != 0;
       hipStream_t st64 = two ? b->stream64 : b->stream;
       if (two) {
         hip_check(hipEventRecord(b->fork->e, b->stream), "event");
@@ -1259,9 +1265,6 @@ int alps_ed_batch_create(const alps_ed_batch_config* cfg, alps_ed_batch* out) {
     }
     budget = align_up(budget);
     hip_check(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking), "hipStreamCreate");
-    hip_check(hipStreamCreateWithFlags(&b->stream64, hipStreamNonBlocking), "hipStreamCreate");
-    b->fork.reset(new Event);
-    b->join.reset(new Event);
     hip_check(hipMalloc(&b->dev_base, budget), "hipMalloc arena");
     b->arena.init(budget);
     const size_t hbytes = align_up(cfg->host_bytes ? cfg->host_bytes : ((size_t)256 << 20));
