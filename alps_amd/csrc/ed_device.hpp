@@ -71,7 +71,10 @@ __device__ __forceinline__ double thread_partials(const Partials& P) {
 __device__ __forceinline__ double sum_partials(const Partials& P) { return block_sum_all(thread_partials(P)); }
 
 // LDS by address.  The kernels that use LDS pages hold all their LDS in the
-// dynamic allocation, which then starts at address 0, and xor page addresses.
+// dynamic allocation, which then starts at address 0, and xor page addresses:
+// none of them may have a __shared__ variable, its own or of a function that
+// it calls (tests/test_kernel_resources.py reads their static LDS from the
+// built library and names every kernel that these functions are used in).
 template <class T>
 __device__ __forceinline__ T lds_ld(uint32_t addr) {
   return *reinterpret_cast<const __attribute__((address_space(3))) T*>(addr);

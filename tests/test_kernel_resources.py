@@ -68,3 +68,14 @@ def test_reorthogonalization_launches_the_updates_threads():
     sizes = {kind: {k[".max_flat_workgroup_size"] for n, k in ks.items() if kind in n}
              for kind in ("update_fused_kernel", "reorth_update_kernel")}
     assert sizes["update_fused_kernel"] == sizes["reorth_update_kernel"] != set()
+
+
+def test_kernels_that_address_lds_hold_no_static_lds():
+    # lds_ld / lds_st (ed_device.hpp) take addresses from 0 on, where the
+    # dynamic allocation starts only if the kernel has no __shared__ variable
+    ks = kernels()
+    for kind in ("9hv_kernelI", "hv_ranked_kernelI", "batch_hv_kernelI", "batch_plain_hv_kernel", "flip_gram_kernelI"):
+        found = {n: k[".group_segment_fixed_size"] for n, k in ks.items() if kind in n}
+        assert found and not any(found.values()), (kind, found)
+    # the metadata does tell: kernels that have such variables report them
+    assert any(k[".group_segment_fixed_size"] for n, k in ks.items() if "update_fused_kernel" in n)
