@@ -434,7 +434,7 @@ template <class V>
 double dot_sync(uint64_t n, const V* x, const V* y) {
   Reducer& r = thread_reducer();
   hip_check(launch_dot<V>(n, x, y, r.a(), current_stream()), "dot");
-  hip_check(launch_finish(Partials{r.a(), stream_blocks(n)}, nullptr, r.result(0), nullptr, kSum, current_stream(),
+  hip_check(launch_finish(Partials{r.a(), stream_blocks(n)}, r.result(0), nullptr, kSum, current_stream(),
                           r.mapped_d(0)),
             "finish");
   hip_check(hipStreamSynchronize(current_stream()), "sync");
@@ -477,7 +477,7 @@ void lanczos_step_dev(alps_ed_lanczos lz, int j) {
 
 // beta_{n-1} and scale_n after n steps (the host reads beta).
 void finish_norm(alps_ed_lanczos lz, int n) {
-  hip_check(launch_finish(Partials{norm_buf(lz, n), lz->norm_count[n & 1]}, nullptr, lz->beta.as<double>() + n - 1,
+  hip_check(launch_finish(Partials{norm_buf(lz, n), lz->norm_count[n & 1]}, lz->beta.as<double>() + n - 1,
                           lz->scale.as<double>() + n, kNorm, lz->stream, lz->beta_h(n - 1)),
             "finish");
 }
@@ -958,13 +958,13 @@ int alps_ed_lanczos_step_vectors(alps_ed_operator op, alps_ed_vector v_prev, alp
 }  // extern "C"
 
 // Scratch of the allocation-free step: the H.v dot partials (one per H.v
-// block), the norm partials of the update (one per streaming block) and the
+// block), the norm partials of the update (one per block of it) and the
 // scalar results, 2 MiB + 8 KiB + 128 B.  Each GPU holds its own copy for the
 // life of the process.
 constexpr size_t kStaticHvPartials = size_t(1) << 18;
 constexpr size_t kStaticNormPartials = 1024;
 constexpr size_t kStaticResults = 16;
-static_assert(kStaticNormPartials >= 1024, "stream_blocks() is at most 1024");
+static_assert(kStaticNormPartials >= kUpdBlocks, "one per block of the update");
 static __device__ __align__(256) double scratch[kStaticHvPartials + kStaticNormPartials + kStaticResults];
 
 namespace {
@@ -1138,7 +1138,7 @@ int alps_ed_lanczos_start(alps_ed_lanczos lz, uint64_t seed, alps_ed_vector star
       // scale[0] = 1/|u0|; |u0| goes to a spare slot of beta
       hip_check(launch_dot<V>(n, u0, u0, norm_buf(lz, 0), lz->stream), "norm");
       lz->norm_count[0] = stream_blocks(n);
-      hip_check(launch_finish(Partials{norm_buf(lz, 0), lz->norm_count[0]}, nullptr,
+      hip_check(launch_finish(Partials{norm_buf(lz, 0), lz->norm_count[0]},
                               lz->beta.as<double>() + lz->max_steps + 1, lz->scale.as<double>(), kNorm, lz->stream),
                 "finish");
       lanczos_step_dev<V>(lz, 0);
@@ -1489,10 +1489,10 @@ double rayleigh_quotient(alps_ed_lanczos lz, alps_ed_vector y, alps_ed_vector hy
   const uint64_t n = lz->op->n;
   double* res = lz->red.result(0);
   hip_check(op_hv<double>(lz->op, y->buf.as<double>(), hy->buf.as<double>(), lz->red.a(), lz->stream), "hv");
-  hip_check(launch_finish(Partials{lz->red.a(), op_hv_blocks(lz->op)}, nullptr, res, nullptr, kSum, lz->stream),
+  hip_check(launch_finish(Partials{lz->red.a(), op_hv_blocks(lz->op)}, res, nullptr, kSum, lz->stream),
             "finish");
   hip_check(launch_dot<double>(n, y->buf.as<double>(), y->buf.as<double>(), lz->red.b(), lz->stream), "dot");
-  hip_check(launch_finish(Partials{lz->red.b(), stream_blocks(n)}, nullptr, res + 1, nullptr, kSum, lz->stream),
+  hip_check(launch_finish(Partials{lz->red.b(), stream_blocks(n)}, res + 1, nullptr, kSum, lz->stream),
             "finish");
   double h[2];
   hip_check(hipMemcpyAsync(h, res, 2 * sizeof(double), hipMemcpyDeviceToHost, lz->stream), "copy");

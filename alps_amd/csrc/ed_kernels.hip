@@ -227,9 +227,6 @@ __global__ __launch_bounds__(kBlock) void scatter_copy_kernel(const unsigned cha
 }
 
 // ---------------------------------------------------------------------------
-// Lanczos update, reductions, vector kernels
-// ---------------------------------------------------------------------------
-// ---------------------------------------------------------------------------
 // Partial reorthogonalization (ReorthDev, ed_kernels.hpp)
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double block_max_all(double v) {
@@ -426,6 +423,9 @@ __global__ __launch_bounds__(kUpdBlock) void reorth_update_kernel(uint64_t n, in
   store_update_partial<kUpdBlock>(norm_out, acc);
 }
 
+// ---------------------------------------------------------------------------
+// Lanczos update, reductions, vector kernels
+// ---------------------------------------------------------------------------
 // A thread's share of two sums of partials in index order: the first ones are
 // read by the constructor, used by add().
 struct PartialPair {
@@ -553,20 +553,12 @@ __global__ __launch_bounds__(kBlock) void dot_kernel(uint64_t n, const V* __rest
   store_partial(partials, acc);
 }
 
-__global__ __launch_bounds__(kBlock) void finish_kernel(Partials in, const double* scale, double* out, double* out2,
-                                                        int mode, double* out_h) {
+__global__ __launch_bounds__(kBlock) void finish_kernel(Partials in, double* out, double* out2, int mode,
+                                                        double* out_h) {
   const double s = sum_partials(in);
   if (threadIdx.x == 0) {
-    double v;
-    if (mode == kNorm) {
-      v = sqrt(s);
-      if (out2) out2[0] = 1.0 / sqrt(s);
-    } else if (mode == kAlpha) {
-      const double sc = scale ? *scale : 1.0;
-      v = sc * sc * s;
-    } else {
-      v = s;
-    }
+    const double v = mode == kNorm ? sqrt(s) : s;
+    if (mode == kNorm && out2) out2[0] = 1.0 / v;
     out[0] = v;
     if (out_h) out_h[0] = v;
   }
@@ -835,9 +827,8 @@ hipError_t launch_dot(uint64_t n, const V* x, const V* y, double* partials, hipS
   return hipGetLastError();
 }
 
-hipError_t launch_finish(Partials in, const double* scale, double* out, double* out2, int mode, hipStream_t st,
-                         double* out_h) {
-  hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(kBlock), 0, st, in, scale, out, out2, mode, out_h);
+hipError_t launch_finish(Partials in, double* out, double* out2, int mode, hipStream_t st, double* out_h) {
+  hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(kBlock), 0, st, in, out, out2, mode, out_h);
   return hipGetLastError();
 }
 

@@ -140,9 +140,10 @@ inline unsigned stream_blocks(uint64_t n) {
 // elements that a thread reads ahead (half as many in FP64) and blocks.
 constexpr int kUpdBlock = 512;
 constexpr int kUpdAhead = 2;
+constexpr unsigned kUpdBlocks = 512;  // at most
 inline unsigned fused_blocks(uint64_t n) {
   const uint64_t b = (n + (uint64_t)kUpdBlock * 4 - 1) / ((uint64_t)kUpdBlock * 4);
-  return (unsigned)(b < 1 ? 1 : b > 512 ? 512 : b);
+  return (unsigned)(b < 1 ? 1 : b > kUpdBlocks ? kUpdBlocks : b);
 }
 
 // Blocks of the H.v kernel: one per segment.
@@ -181,13 +182,12 @@ constexpr HvRankedSchedule kHvRankedSchedule[kHvSchedules] = {{8, 4, 4, 2}, {8, 
 template <class V>
 hipError_t launch_hv(const DevLayout& L, const V* x, V* y, double* dot_out, hipStream_t st, int schedule = 0);
 
-// Lanczos scalars between the kernels of one step (one block):
-//   mode kAlpha: alpha = scale^2 * sum(in)            -> out[0]
-//   mode kBeta:  beta = sqrt(sum(in)), scale = 1/beta -> out[0], out2[0]
-enum { kSum = 0, kNorm = 1, kAlpha = 2 };
+// A sum of partials (one block):
+//   mode kSum:  sum(in)                              -> out[0]
+//   mode kNorm: beta = sqrt(sum(in)), scale = 1/beta -> out[0], out2[0]
+enum { kSum = 0, kNorm = 1 };
 // out_h, when set (host-mapped memory), receives a copy of out[0].
-hipError_t launch_finish(Partials in, const double* scale, double* out, double* out2, int mode, hipStream_t st,
-                         double* out_h = nullptr);
+hipError_t launch_finish(Partials in, double* out, double* out2, int mode, hipStream_t st, double* out_h = nullptr);
 
 // Partial reorthogonalization (Simon, "The Lanczos algorithm with partial
 // reorthogonalization", Math. Comp. 42 (1984) 115-142) of a recurrence whose

@@ -216,7 +216,7 @@ struct SectorLayout {
   //   nbp16[nbp_off[c] + flip_index(r, b, n_ll_p, kLLChunk)]: 8 * the row
   //     reached from row r of a class-c segment by low-low bond b, or
   //     8 * C(B,c) if the bond does not flip it.
-  int n_ll_p = 0, n_hh_p = 0, n_xb_p = 0;
+  int n_ll_p = 0, n_xb_p = 0;
   std::vector<uint16_t> nbp16, xn16;
   std::vector<uint32_t> nbp_off, xn_off;  // [B+2]
   bool ranked = false;                    // ranked_rows
@@ -256,7 +256,7 @@ struct SectorLayout {
 // The H.v schedules (ed_kernels.hpp) process the flip bonds of each class in
 // chunks of up to 8; bond lists and flip tables are padded to these
 // multiples, which every schedule's chunk sizes divide.
-constexpr int kPadLL = 8, kPadHH = 8, kPadX = 4;
+constexpr int kPadLL = 8, kPadX = 4;
 // padding of each high word's list of flipping high-high bonds
 constexpr int kHHList = 4;
 
@@ -281,7 +281,7 @@ inline int choose_low_bits(int N) {
   return N < 12 ? N : 12;
 }
 
-// Position of low word lo in an LDS page of 2^(B-1) elements (page_entries):
+// Position of low word lo in an LDS page of 2^(B-1) elements:
 // its Gray code without the lowest bit.  The map is linear over xor, so the
 // flip of the bits m moves every row by the same xor, page_pos(lo ^ m) =
 // page_pos(lo) ^ page_pos(m), and needs no table.  Two words share a position
@@ -710,7 +710,6 @@ inline SectorLayout build_layout(const ModelSpec& m, int B_override = -1, bool c
   for (uint32_t i = 0; i < nlo; ++i) L.diag_lo_cls[i] = L.diag_lo[L.low->lo_state[i]];
   // padded H.v tables
   L.n_ll_p = round_up((int)L.ll.size(), kPadLL);
-  L.n_hh_p = round_up((int)L.hh.size(), kPadHH);
   L.n_xb_p = round_up((int)L.xb.size(), kPadX);
   {
     std::vector<uint32_t> xlb;
