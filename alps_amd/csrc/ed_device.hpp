@@ -581,14 +581,19 @@ __device__ __forceinline__ double hv_rows(const DevLayout& L, const SegRec& S, c
 // their part of the page).  CLL, CHH: chunk sizes of the flip loops (the
 // schedule, ed_kernels.hpp).
 //
-// What bounds it: at 24 sites (2.7 M rows, FP32) the 51 MB of neighbour reads
-// that miss the XCDs' L2 take 7 us at the 7.4 TB/s such misses reach, the rest
-// is the chain of dependent rounds of a segment (record -> x -> page -> list
-// entries -> neighbour rows) with 2 generations of workgroups; on the 30-site
-// J1-J2 lattice (155 M rows) 15.6 GB of misses take 2.1 of 3.3 ms and the load
-// and LDS instructions are next.  Measured against flip tables in memory, a
-// page indexed by rank and __syncthreads: 15.7 -> 14.3 us at 24 sites, 4.22 ->
-// 3.32 ms on J1-J2, FP64 38.9 -> 36.5 us (25 sites), 5.0 -> 4.4 us (20 sites).
+// What bounds it: at 24 sites (2.7 M rows, FP32) 33 MB of neighbour reads that
+// miss the XCDs' L2 and 11 MB of y take 5.9 us at the 7.4 TB/s such misses
+// reach, the rest is the chain of dependent rounds of a segment (record -> x ->
+// page -> list entries -> neighbour rows) with 2 generations of workgroups
+// (waves wait for 47 % of their cycles, the address unit is busy for 57 % of
+// the 14.7 us); at 25 sites (4.5 M rows, FP64) 104 + 36 MB take 18.9 of 34.5
+// us. On the 30-site J1-J2 lattice (155 M rows) 15.3 GB of misses and 0.7 GB of
+// writes take 2.2 of 3.3 ms; the address unit is busy for 62 % of it (98 % with
+// tables and gathers), LDS for 52 %, half of that bank conflicts, the vector
+// ALUs for 46 %.  Measured against flip tables in memory, a page indexed by
+// rank and __syncthreads, the earlier segment order on both sides: 15.7 -> 14.3
+// us at 24 sites, 4.22 -> 3.32 ms on J1-J2, FP64 38.9 -> 36.5 us (25 sites),
+// 5.0 -> 4.4 us (20 sites).
 // Of that, the table loads that the xor positions save are the most (a
 // quarter of the J1-J2 launch's vector loads), then the staged cross bonds
 // (3.93 -> 3.37 ms) and barriers that do not drain the loads in flight.

@@ -30,16 +30,16 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-# HBM bytes per launch of hv_kernel<float,false> on this workload (L=24), per
+# HBM bytes per launch of hv_kernel<float,false,...> on this workload (L=24), per
 # schedule (the order of SCHEDULES below), from rocprofv3 --pmc FETCH_SIZE and
 # WRITE_SIZE scaled by a copy kernel of known size
 # (profiles/hv_kernel_heisenberg_L24.md); valid for that kernel version and L
 # only.
-PMC_TRAFFIC_BYTES = {24: [53.38e6, 53.47e6, 53.35e6, 53.30e6, 58.25e6, 54.01e6]}
+PMC_TRAFFIC_BYTES = {24: [43.93e6, 43.96e6, 62.58e6, 43.91e6, 43.91e6, 43.86e6]}
 # SHA-256 of the row kernel's source (alps_amd/csrc/ed_device.hpp) when those
 # counters were taken: if the source differs, the table no longer describes
 # the kernel that runs, and the bench reports traffic as unknown instead.
-PMC_TRAFFIC_KERNEL_SHA256 = "8dd16111070282a21ca2d360f4733c5027e3ac0292ebee8e726dea2ee30cccc5"
+PMC_TRAFFIC_KERNEL_SHA256 = "ee31d05edbbeb133c810f7c54b9e462acd4cc8c792f03b582846181c4f878247"
 PMC_TRAFFIC_SOURCE = ("profiles/hv_kernel_heisenberg_L24.md, section 'HBM byte counters', column "
                       "'traffic per launch' (FETCH_SIZE + WRITE_SIZE, scaled by the copy kernel), "
                       "row of the chosen schedule")
