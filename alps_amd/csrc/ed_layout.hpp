@@ -424,8 +424,8 @@ constexpr size_t kFewSegments = 512;
 // Whether single operators take the kernel with low-low target tables
 // (hv_ranked_at, ed_device.hpp): where the segments are short on average, away
 // from half filling.  Xor page and tables, us: rows a segment 168 (27 sites, 9
-// up, FP32) 49.7 and 44.8, 193 (24-site J1-J2, 8 up) 24.3 and 20.5, FP64 37.3
-// and 30.1, 247 (23 sites, 8 up) 5.4 and 5.2, 325 (24-site J1-J2, 15 up) 31.6
+// up, FP32) 49.7 and 44.4, 193 (24-site J1-J2, 8 up) 24.3 and 20.1, FP64 37.3
+// and 30.0, 247 (23 sites, 8 up) 5.4 and 5.2, 325 (24-site J1-J2, 15 up) 31.6
 // and 30.1; 333 (26 sites, 10 up) 35.0 and 35.6, 405 (27-site J1-J2, 11 up)
 // 245 and 252.  Up to 1024 segments (half of the workgroups that are resident)
 // the fixed part weighs more: 486 rows (22 sites, 9 up) 5.25 and 5.05, and 631
