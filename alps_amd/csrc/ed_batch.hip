@@ -764,8 +764,8 @@ const SharedTables& shared_tables(alps_ed_batch b, const SectorLayout& L) {
   const auto key = std::make_pair(static_cast<const void*>(L.low), static_cast<const void*>(L.flip.get()));
   std::unique_ptr<SharedTables>& slot = b->shared[key];
   if (slot) return *slot;
-  slot.reset(new SharedTables);
-  SharedTables& t = *slot;
+  std::unique_ptr<SharedTables> made(new SharedTables);  // the slot stays empty if a call below fails
+  SharedTables& t = *made;
   t.keep = L.flip;
   size_t total = 0;
   auto sz = [&](size_t n, size_t es) {
@@ -794,7 +794,8 @@ const SharedTables& shared_tables(alps_ed_batch b, const SectorLayout& L) {
   t.lo_word = up(o5, low.lo_word);
   t.xn16 = up(o6, flip.xn16);
   t.xn_off = up(o7, flip.xn_off);
-  return t;
+  slot = std::move(made);
+  return *slot;
 }
 
 // That of a problem's low-low target table, null where its form has none.
@@ -803,11 +804,12 @@ const uint16_t* low_table(alps_ed_batch b, const Problem& p) {
   std::shared_ptr<const std::vector<uint16_t>> t = low_flip_table(p.layout);
   std::unique_ptr<LowTable>& slot = b->low_tables[t.get()];
   if (!slot) {
-    slot.reset(new LowTable);
-    slot->keep = t;
-    slot->buf.alloc(t->size() * sizeof(uint16_t));
-    hip_check(hipMemcpyAsync(slot->buf.p, t->data(), t->size() * sizeof(uint16_t), hipMemcpyHostToDevice, b->stream),
+    std::unique_ptr<LowTable> made(new LowTable);  // the slot stays empty if a call below fails
+    made->keep = t;
+    made->buf.alloc(t->size() * sizeof(uint16_t));
+    hip_check(hipMemcpyAsync(made->buf.p, t->data(), t->size() * sizeof(uint16_t), hipMemcpyHostToDevice, b->stream),
               "upload low-low table");
+    slot = std::move(made);
   }
   return slot->buf.as<uint16_t>();
 }
@@ -848,6 +850,9 @@ void admit(alps_ed_batch b, std::vector<Problem*>& started) {
       finish_problem(b, *q);
       continue;
     }
+    // allocations and uploads that can fail, while the problem is still queued
+    shared_tables(b, p.layout);
+    low_table(b, p);
     if (!b->arena.alloc(f.dev, &doff)) break;
     if (!b->harena.alloc(f.host, &hoff)) {
       b->arena.release(doff, f.dev);

@@ -293,6 +293,9 @@ __global__ __launch_bounds__(kBlock) void batch_ritz_kernel(const RitzJob* __res
   }
 }
 
+// y = H x of a refinement, once per reported level: all forms in one kernel
+// (the registers that they cost each other matter in the steps, not here), the
+// page also for short segments.
 __global__ __launch_bounds__(kBlock) void batch_plain_hv_kernel(const PlainHvJob* __restrict__ jobs,
                                                                 const BatchItem* __restrict__ items) {
   const BatchItem it = ldc_struct(items + blockIdx.x);
